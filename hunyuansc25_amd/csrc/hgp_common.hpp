@@ -250,55 +250,152 @@ __device__ inline void wave_lds_sync()
     __builtin_amdgcn_wave_barrier();
 }
 
+// Lane exchanges on the VALU (DPP and the permlane swaps) instead of through
+// LDS: a __shfl_xor is a ds_bpermute with an LDS round trip of over 100
+// cycles, and a 64-lane reduction is six of them in a row, which the
+// latency-bound row kernels wait out once per row.  Here a 64-lane reduction
+// is four DPP moves and two swaps, a few cycles each.
+
+// v of the lane that DPP control Ctrl names, for a T of whole words; every
+// source lane must be active.
+template <int Ctrl, class T>
+__device__ inline T dpp_move(T v)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    int32_t a[sizeof(T) / 4];
+    __builtin_memcpy(a, &v, sizeof(T));
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 4); i++) a[i] = __builtin_amdgcn_mov_dpp(a[i], Ctrl, 0xf, 0xf, true);
+    T r;
+    __builtin_memcpy(&r, a, sizeof(T));
+    return r;
+}
+
+// The values of the two halves of each 2H lanes (H = 16 or 32), in every lane
+// of the pair, for a value that is uniform over each H lanes.
+template <int H, class T>
+__device__ inline void half_values(T v, T &lo, T &hi)
+{
+    static_assert(sizeof(T) % 4 == 0 && (H == 16 || H == 32), "whole words");
+    uint32_t a[sizeof(T) / 4], b[sizeof(T) / 4];
+    __builtin_memcpy(a, &v, sizeof(T));
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 4); i++) {
+        if constexpr (H == 16) {
+            auto r = __builtin_amdgcn_permlane16_swap(a[i], a[i], false, false);
+            a[i] = r[0];
+            b[i] = r[1];
+        } else {
+            auto r = __builtin_amdgcn_permlane32_swap(a[i], a[i], false, false);
+            a[i] = r[0];
+            b[i] = r[1];
+        }
+    }
+    __builtin_memcpy(&lo, a, sizeof(T));
+    __builtin_memcpy(&hi, b, sizeof(T));
+}
+
+// op over the G lanes of each group (G a power of two up to 64, aligned),
+// the result in all of them; op commutes and associates.  The groups of a
+// wave may diverge, a group's lanes may not.
+template <int G, class T, class Op>
+__device__ inline T lanes_reduce(T v, Op op)
+{
+    if constexpr (G >= 2) v = op(v, dpp_move<0xB1>(v));    // quad_perm [1,0,3,2]
+    if constexpr (G >= 4) v = op(v, dpp_move<0x4E>(v));    // quad_perm [2,3,0,1]
+    if constexpr (G >= 8) v = op(v, dpp_move<0x141>(v));   // row_half_mirror: the other quad of 8 lanes
+    if constexpr (G >= 16) v = op(v, dpp_move<0x140>(v));  // row_mirror: the other half of 16 lanes
+    if constexpr (G >= 32) {
+        T lo, hi;
+        half_values<16>(v, lo, hi);
+        v = op(lo, hi);
+    }
+    if constexpr (G >= 64) {
+        T lo, hi;
+        half_values<32>(v, lo, hi);
+        v = op(lo, hi);
+    }
+    return v;
+}
+
 template <class T>
 __device__ inline T wave_sum(T v)
 {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
+    return lanes_reduce<kWave>(v, [](T a, T b) { return a + b; });
 }
 
 template <class T>
 __device__ inline T wave_max(T v)
 {
-    for (int o = 32; o > 0; o >>= 1) {
-        T u = __shfl_xor(v, o, kWave);
-        v = u > v ? u : v;
-    }
-    return v;
+    return lanes_reduce<kWave>(v, [](T a, T b) { return b > a ? b : a; });
 }
 
-// Inclusive wave scan (Hillis-Steele over 64 lanes).
+// v plus the value of the lane that Ctrl names; the lanes of rows outside
+// RowMask and those without a source lane keep v.
+template <int Ctrl, int RowMask, class T>
+__device__ inline T dpp_add(T v)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    int32_t a[sizeof(T) / 4];
+    __builtin_memcpy(a, &v, sizeof(T));
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 4); i++)
+        a[i] = __builtin_amdgcn_update_dpp(0, a[i], Ctrl, RowMask, 0xf, false);
+    T t;
+    __builtin_memcpy(&t, a, sizeof(T));
+    return v + t;
+}
+
+// Inclusive wave scan (whole waves): four row shifts inside the rows of 16
+// lanes, then lane 15 of rows 0 and 2 and lane 31 broadcast to the lanes after
+// them.
 template <class T>
 __device__ inline T wave_inclusive_scan(T v)
 {
-    int l = lane_id();
-    for (int o = 1; o < kWave; o <<= 1) {
-        T u = __shfl_up(v, o, kWave);
-        if (l >= o) v += u;
-    }
+    v = dpp_add<0x111, 0xf>(v);   // row_shr:1
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    v = dpp_add<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+    v = dpp_add<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
     return v;
 }
 
+// v of lane l; l must be the same in every lane.
+template <class T>
+__device__ inline T wave_read(T v, int l)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    int32_t a[sizeof(T) / 4];
+    __builtin_memcpy(a, &v, sizeof(T));
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 4); i++) a[i] = __builtin_amdgcn_readlane(a[i], l);
+    T r;
+    __builtin_memcpy(&r, a, sizeof(T));
+    return r;
+}
+
 // Block-wide exclusive scan of one value per thread (blockDim.x <= 1024,
-// multiple of 64).  `sh` needs blockDim.x/64 + 1 elements.  Returns the
-// exclusive prefix; *total receives the block total.
+// multiple of 64).  `sh` needs blockDim.x/64 elements.  Returns the
+// exclusive prefix; *total receives the block total.  Every thread adds the
+// wave totals itself: the LDS reads are broadcasts that do not wait for each
+// other, where one thread's running sum would.
 template <class T>
 __device__ inline T block_exclusive_scan(T v, T *sh, T *total)
 {
-    int w = threadIdx.x / kWave, nw = blockDim.x / kWave;
-    T inc = wave_inclusive_scan(v);
+    const int w = threadIdx.x / kWave, nw = blockDim.x / kWave;
+    const T inc = wave_inclusive_scan(v);
     if (lane_id() == kWave - 1) sh[w] = inc;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        T acc = 0;
-        for (int i = 0; i < nw; i++) { T t = sh[i]; sh[i] = acc; acc += t; }
-        sh[nw] = acc;
+    T pre = 0, all = 0;
+    for (int i = 0; i < nw; i++) {
+        const T x = sh[i];
+        pre += i < w ? x : (T)0;
+        all += x;
     }
+    if (total) *total = all;
     __syncthreads();
-    T r = sh[w] + inc - v;
-    if (total) *total = sh[nw];
-    __syncthreads();
-    return r;
+    return pre + inc - v;
 }
 
 // Kernel-timer byte counters come in groups of kKbLanes, spread over by block

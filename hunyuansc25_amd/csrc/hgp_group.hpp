@@ -2,9 +2,9 @@
 //
 // Row-parallel kernels take their vertices from degree classes (RowBins):
 // rows of <= 8 entries get 8-lane groups, rows of <= 512 entries one wave,
-// longer rows one block per segment.  Group reductions are xor-shuffles
-// inside a wave for G <= 64 and go through LDS across the block's waves for
-// a whole block (G > 64).  Every reduction here uses a strict total order (or an integer
+// longer rows one block per segment.  Group reductions are DPP moves and lane
+// swaps inside a wave for G <= 64 and go through LDS across the block's waves
+// for a whole block (G > 64).  Every reduction here uses a strict total order (or an integer
 // sum), so results do not depend on which lane saw which entry.
 #pragma once
 
@@ -71,37 +71,17 @@ __device__ inline int glane() { return (int)(threadIdx.x % G); }
 template <int G>
 __device__ inline int64_t gindex() { return ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / G; }
 
-template <class T>
-__device__ inline T shfl_xor_pod(T v, int o, int width)
-{
-    static_assert(sizeof(T) % 4 == 0, "pod shuffle needs 4-byte multiples");
-    T r;
-    const int32_t *p = reinterpret_cast<const int32_t *>(&v);
-    int32_t *q = reinterpret_cast<int32_t *>(&r);
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(T) / 4); i++) q[i] = __shfl_xor(p[i], o, width);
-    return r;
-}
-
 // All lanes of the group receive the best value under `better` (a strict
 // total order on distinct values).
 template <int G, class T, class Better>
 __device__ inline T group_best(T v, Better better)
 {
+    auto pick = [&](const T &a, const T &b) { return better(b, a) ? b : a; };
     if constexpr (G <= kWave) {
-#pragma unroll
-        for (int o = G / 2; o > 0; o >>= 1) {
-            T u = shfl_xor_pod(v, o, G);
-            if (better(u, v)) v = u;
-        }
-        return v;
+        return lanes_reduce<G>(v, pick);
     } else {
         __shared__ T sh[G / kWave];
-#pragma unroll
-        for (int o = kWave / 2; o > 0; o >>= 1) {
-            T u = shfl_xor_pod(v, o, kWave);
-            if (better(u, v)) v = u;
-        }
+        v = lanes_reduce<kWave>(v, pick);
         if (lane_id() == 0) sh[threadIdx.x / kWave] = v;
         __syncthreads();
         T r = sh[0];
@@ -117,9 +97,7 @@ template <int G, class T>
 __device__ inline T group_sum(T v)
 {
     if constexpr (G <= kWave) {
-#pragma unroll
-        for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, G);
-        return v;
+        return lanes_reduce<G>(v, [](T a, T b) { return a + b; });
     } else {
         __shared__ T sh[G / kWave];
         v = wave_sum(v);

@@ -34,34 +34,55 @@ __global__ void __launch_bounds__(kScanBS) k_tile_reduce(const T *__restrict__ i
     }
 }
 
-// Inclusive scan of each tile plus the inclusive prefix of the previous
-// tiles (incl_sums[tile-1]).
+// Inclusive scan of each tile plus the prefix of the tiles before it: the
+// inclusive scan of the tile totals (sums[tile - 1]), or, raw, the block's own
+// sum of the totals before its tile (few tiles, so this costs less than a
+// launch).  Bound by latency on the levels that use it most (a few tiles), so
+// a wave issues the loads of its 8 rows of 64 items at once, scans each row on
+// the VALU and carries the row totals; the block meets at one barrier.  (Eight
+// rounds of a block scan each, three barriers a round, took 8.8 us a launch.)
 template <class T>
 __global__ void __launch_bounds__(kScanBS) k_tile_scan(const T *in, T *out, int64_t n, const T *__restrict__ sums,
                                                       int raw)
 {
-    __shared__ T sh[kScanBS / kWave + 1];
-    int64_t base = (int64_t)blockIdx.x * (kScanBS * kScanR);
-    T carry = 0;
+    constexpr int NW = kScanBS / kWave;
+    __shared__ T sh[NW], shp[NW];
+    const int w = threadIdx.x / kWave, lane = lane_id();
+    const int64_t base = (int64_t)blockIdx.x * (kScanBS * kScanR) + w * (kWave * kScanR) + lane;
+    T x[kScanR];
+#pragma unroll
+    for (int r = 0; r < kScanR; r++) {
+        const int64_t i = base + r * kWave;
+        x[r] = i < n ? in[i] : (T)0;
+    }
+    T part = 0;
     if (sums && blockIdx.x > 0) {
         if (raw) {
-            // sums[t] = total of tile t (not scanned): the block adds those of
-            // the tiles before its own (few tiles, so this costs less than a launch)
-            T part = 0;
+#pragma unroll 8
             for (int i = threadIdx.x; i < (int)blockIdx.x; i += kScanBS) part += sums[i];
-            block_exclusive_scan(part, sh, &carry);
-        } else {
-            carry = sums[blockIdx.x - 1];   // inclusive scan of the tile totals
+        } else if (threadIdx.x == 0) {
+            part = sums[blockIdx.x - 1];
         }
     }
+    T run = 0;
+#pragma unroll
     for (int r = 0; r < kScanR; r++) {
-        int64_t i = base + r * kScanBS + threadIdx.x;
-        T v = i < n ? in[i] : (T)0;
-        T tot;
-        T ex = block_exclusive_scan(v, sh, &tot);
-        if (i < n) out[i] = carry + ex + v;
-        carry += tot;
-        if (base + (r + 1) * kScanBS >= n) break;   // uniform across the block
+        x[r] = wave_inclusive_scan(x[r]) + run;
+        run = wave_read(x[r], kWave - 1);
+    }
+    part = wave_sum(part);
+    if (lane == 0) {
+        sh[w] = run;
+        shp[w] = part;
+    }
+    __syncthreads();
+    T carry = 0;
+#pragma unroll
+    for (int i = 0; i < NW; i++) carry += shp[i] + (i < w ? sh[i] : (T)0);
+#pragma unroll
+    for (int r = 0; r < kScanR; r++) {
+        const int64_t i = base + r * kWave;
+        if (i < n) out[i] = carry + x[r];
     }
 }
 
@@ -343,43 +364,67 @@ __global__ void k_compact(const uint8_t *__restrict__ f, const int32_t *__restri
 
 // Flag compaction in two launches (up to kRawTiles tiles): per-tile flag
 // counts, then each block adds the counts of the tiles before its own, ranks
-// its tile's flags with block scans and writes their indices in order.
+// its tile's flags with one block scan and writes their indices in order.  A
+// thread takes 8 consecutive flags as one 8-byte load (f is 8-byte aligned;
+// the last bytes of the array one by one), so a tile is one scan, not eight.
+__device__ inline uint32_t load_flags8(const uint8_t *__restrict__ f, int64_t i0, int64_t n)
+{
+    uint32_t m = 0;   // bit j: flag i0 + j set
+    if (i0 + 8 <= n) {
+        const uint64_t x = *(const uint64_t *)(f + i0);
+#pragma unroll
+        for (int j = 0; j < 8; j++) m |= ((x >> (8 * j)) & 255u) != 0 ? 1u << j : 0u;
+    } else {
+        for (int j = 0; i0 + j < n; j++) m |= f[i0 + j] != 0 ? 1u << j : 0u;
+    }
+    return m;
+}
+
 __global__ void __launch_bounds__(kScanBS) k_flag_tile_count(const uint8_t *__restrict__ f, int64_t n,
                                                              int32_t *__restrict__ tsum)
 {
-    __shared__ int32_t sh[kScanBS / kWave + 1];
-    const int64_t base = (int64_t)blockIdx.x * (kScanBS * kScanR);
-    int32_t cnt = 0;
-#pragma unroll
-    for (int r = 0; r < kScanR; r++) {
-        const int64_t i = base + r * kScanBS + threadIdx.x;
-        cnt += (i < n && f[i]) ? 1 : 0;
+    static_assert(kScanR == 8, "one 8-byte load per thread");
+    __shared__ int32_t sh[kScanBS / kWave];
+    const int64_t i0 = (int64_t)blockIdx.x * (kScanBS * kScanR) + threadIdx.x * 8;
+    const int32_t cnt = wave_sum((int32_t)__popc(load_flags8(f, i0, n)));
+    if (lane_id() == 0) sh[threadIdx.x / kWave] = cnt;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int32_t t = 0;
+        for (int w = 0; w < kScanBS / kWave; w++) t += sh[w];
+        tsum[blockIdx.x] = t;
     }
-    int32_t tot;
-    block_exclusive_scan(cnt, sh, &tot);
-    if (threadIdx.x == 0) tsum[blockIdx.x] = tot;
 }
 
 __global__ void __launch_bounds__(kScanBS) k_flag_compact(const uint8_t *__restrict__ f, int64_t n,
                                                           const int32_t *__restrict__ tsum,
                                                           int32_t *__restrict__ idx, int64_t *count)
 {
-    __shared__ int32_t sh[kScanBS / kWave + 1];
-    const int64_t base = (int64_t)blockIdx.x * (kScanBS * kScanR);
+    __shared__ int32_t sh[kScanBS / kWave], shp[kScanBS / kWave];
+    const int w = threadIdx.x / kWave;
+    const int64_t i0 = (int64_t)blockIdx.x * (kScanBS * kScanR) + threadIdx.x * 8;
+    uint32_t m = load_flags8(f, i0, n);
     int32_t part = 0;
+#pragma unroll 8
     for (int i = threadIdx.x; i < (int)blockIdx.x; i += kScanBS) part += tsum[i];
-    int32_t carry;
-    block_exclusive_scan(part, sh, &carry);
-    for (int r = 0; r < kScanR; r++) {
-        const int64_t i = base + r * kScanBS + threadIdx.x;
-        const int32_t v = (i < n && f[i]) ? 1 : 0;
-        int32_t tot;
-        const int32_t ex = block_exclusive_scan(v, sh, &tot);
-        if (v) idx[carry + ex] = (int32_t)i;
-        carry += tot;
-        if (base + (r + 1) * kScanBS >= n) break;   // uniform across the block
+    part = wave_sum(part);
+    const int32_t own = __popc(m), incl = wave_inclusive_scan(own);
+    if (lane_id() == kWave - 1) {
+        sh[w] = incl;
+        shp[w] = part;
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *count = carry;
+    __syncthreads();
+    int32_t at = incl - own, all = 0;
+#pragma unroll
+    for (int i = 0; i < kScanBS / kWave; i++) {
+        at += shp[i] + (i < w ? sh[i] : 0);
+        all += shp[i] + sh[i];
+    }
+    while (m) {
+        idx[at++] = (int32_t)(i0 + (__ffs(m) - 1));
+        m &= m - 1;
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *count = all;
 }
 
 // ------------------------------------------------------------ degree classes
