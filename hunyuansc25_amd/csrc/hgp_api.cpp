@@ -1228,6 +1228,10 @@ int hgp_initpart(int32_t n, const int64_t *xadj, const int32_t *adjncy, const in
         with_arena(c, estimate_arena(n, xadj[n], k, true) + extra, [&] {
             DevGraph g = upload(c, n, xadj, adjncy, vwgt, adjwgt);
             int32_t *dw = c.arena.lalloc<int32_t>((size_t)n);
+            g.ascending = true;
+            for (int32_t v = 0; v < n && g.ascending; v++)
+                for (int64_t j = xadj[v] + 1; j < xadj[v + 1]; j++)
+                    if (adjncy[j] <= adjncy[j - 1]) g.ascending = false;
             initial_partition(c, g, k, p, dw);
             to_host(c, where, dw, (size_t)n);
         });

@@ -1626,6 +1626,7 @@ DevGraph contract(Ctx &c, const DevGraph &g, const int32_t *match, const int32_t
 {
     DevGraph cg;
     cg.n = cn;
+    cg.ascending = true;
     cg.xadj = c.arena.lalloc<eid_t>((size_t)cn + 1);
     cg.vwgt = c.arena.lalloc<wgt_t>((size_t)cn);
     int64_t m = g.m;

@@ -18,6 +18,7 @@ struct DevGraph {
     vid_t *adjncy = nullptr;
     wgt_t *adjwgt = nullptr;
     wgt_t *vwgt = nullptr;
+    bool ascending = false;   // every row's neighbours strictly ascend (true of contracted graphs)
     RowBins bins;             // degree classes of the rows (set by attach_bins)
     RowSegs segs;             // segments of the class-2 rows (set by attach_bins)
 };

@@ -12,26 +12,32 @@
 #include "hgp_graph.hpp"
 #include "hgp_prims.hpp"
 
+#include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace hgp {
 
 namespace {
 
-constexpr int kTrialBytesPerVertex = 14;   // where, moved (u8) + ed, id, queue (i32)
-// heap FM: + position index and two heaps of (key, vertex), n + 1 slots each (i32)
-constexpr int kHeapBytesPerVertex = 20;
-constexpr int kLdsBudget = 60 * 1024;
+// LDS of a trial.  Scan FM: (ed, wd) pairs, row offsets (i32), queue (u16)
+// and a state byte, 15 bytes a vertex; node graphs of up to kScanLdsN
+// vertices run in LDS (two trials per CU at that size), larger ones in global
+// scratch with a 32-bit queue.  Heap FM: where, moved (u8), ed, id, queue,
+// position index (i32) and two heaps of (key, vertex), n + 1 slots each.
+constexpr int32_t kScanLdsN = 4864;
+constexpr int kHeapBytesPerVertex = 34;
+constexpr int kHeapLdsBudget = 60 * 1024;
 // fm_kind -1 keeps the scan: on the dense coarsest graphs this pipeline
 // produces (R-MAT 2^22: 995 vertices, average degree ~300) the queues took
 // 188 ms against 7 ms, a move's row being ~300 serial queue updates
 constexpr int32_t kAutoHeapMinVertices = INT32_MAX;
 
-__host__ __device__ inline int64_t trial_bytes(int64_t n, bool heap)
+__host__ __device__ inline int64_t trial_bytes(int64_t n, bool heap, bool in_lds)
 {
-    int64_t b = ((2 * n + 3) & ~3ll) + 12 * n;
-    if (heap) b += 4 * n + 16 * (n + 1);
-    return b;
+    if (heap) return ((2 * n + 3) & ~3ll) + 12 * n + 4 * n + 16 * (n + 1);
+    const int64_t n4 = (n + 3) & ~3ll;   // the arg-max reads four vertices at a time
+    return (8 + 4 + (in_lds ? 2 : 4) + 1) * n4 + 16;
 }
 
 struct Node {
@@ -40,17 +46,28 @@ struct Node {
     int32_t T, trial_off, best, cnt0;
     int64_t woff;       // offset of the node's trial-where block (bytes)
     int64_t soff;       // offset of the node's global scratch block (bytes)
+    int64_t doff, boff; // offsets of the node's dense weight and bit matrices (words)
 };
 
-__global__ void k_ip_init(int32_t n, const wgt_t *__restrict__ vwgt, int32_t *__restrict__ node_of,
-                          int32_t *__restrict__ label, wgt_t *__restrict__ fvw, Node *nodes)
+// The root node: a wave per vertex sums its row's weight.
+__global__ void __launch_bounds__(kRowBS) k_ip_init(int32_t n, const wgt_t *__restrict__ vwgt,
+                                                    const eid_t *__restrict__ xadj,
+                                                    const wgt_t *__restrict__ adjwgt, int32_t *__restrict__ node_of,
+                                                    int32_t *__restrict__ label, wgt_t *__restrict__ fvw,
+                                                    int32_t *__restrict__ fwd, Node *nodes)
 {
-    int32_t v = (int32_t)((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (v < n) {
-        node_of[v] = 1;
-        label[v] = v;
-        fvw[v] = vwgt[v];
-    }
+    const int32_t v = (int32_t)gindex<kWave>();
+    if (v >= n) return;   // whole waves
+    int32_t s = 0;
+    const eid_t e = xadj[v + 1];
+#pragma unroll 4
+    for (eid_t j = xadj[v] + lane_id(); j < e; j += kWave) s += adjwgt[j];
+    s = wave_sum(s);
+    if (lane_id() != 0) return;
+    node_of[v] = 1;
+    label[v] = v;
+    fvw[v] = vwgt[v];
+    fwd[v] = s;
     if (v == 0) {
         nodes[1].start = 0;
         nodes[1].end = n;
@@ -83,30 +100,43 @@ __global__ void __launch_bounds__(256) k_ip_setup(const int32_t *__restrict__ ac
     }
 }
 
-// Exclusive offsets of trials and scratch over the active nodes (one block).
-__global__ void k_ip_offsets(const int32_t *__restrict__ act, int32_t nact, Node *nodes, int32_t lds_cap,
-                             bool heap, int32_t *total)
+// Exclusive offsets of trials, scratch and dense matrices over the active
+// nodes: running sums in one block, 256 nodes a step (one thread walking the nodes
+// took 145 us for 500 of them).
+__global__ void __launch_bounds__(256) k_ip_offsets(const int32_t *__restrict__ act, int32_t nact, Node *nodes,
+                                                    int32_t lds_cap, bool heap, int32_t *total)
 {
-    if (threadIdx.x != 0) return;
-    int32_t t = 0;
-    int64_t w = 0, s = 0;
-    for (int32_t a = 0; a < nact; a++) {
-        Node &nd = nodes[act[a]];
-        int64_t nn = nd.end - nd.start;
-        nd.trial_off = t;
-        nd.woff = w;
-        nd.soff = s;
-        t += nd.T;
-        w += (int64_t)nd.T * nn;
-        if (nn > lds_cap) s += (int64_t)nd.T * ((trial_bytes(nn, heap) + 255) & ~255ll);
+    __shared__ int64_t sh[256 / kWave];
+    int64_t t = 0, w = 0, s = 0, d = 0, b = 0;
+    for (int32_t a0 = 0; a0 < nact; a0 += 256) {
+        const int32_t a = a0 + threadIdx.x;
+        Node *nd = a < nact ? &nodes[act[a]] : nullptr;
+        const int64_t nn = nd ? nd->end - nd->start : 0, tr = nd ? nd->T : 0;
+        const int64_t sc = nn > lds_cap ? tr * ((trial_bytes(nn, heap, false) + 255) & ~255ll) : 0;
+        int64_t at, tot;
+        at = block_exclusive_scan<int64_t>(tr, sh, &tot) + t;
+        t += tot;
+        if (nd) nd->trial_off = (int32_t)at;
+        at = block_exclusive_scan<int64_t>(tr * nn, sh, &tot) + w;
+        w += tot;
+        if (nd) nd->woff = at;
+        at = block_exclusive_scan<int64_t>(sc, sh, &tot) + s;
+        s += tot;
+        if (nd) nd->soff = at;
+        at = block_exclusive_scan<int64_t>(nn * ((nn + 3) & ~3ll), sh, &tot) + d;
+        d += tot;
+        if (nd) nd->doff = at;
+        at = block_exclusive_scan<int64_t>(nn * ((nn + 31) / 32), sh, &tot) + b;
+        b += tot;
+        if (nd) nd->boff = at;
     }
-    *total = t;
+    if (threadIdx.x == 0) *total = (int32_t)t;
 }
 
 struct TrialMem {
     uint8_t *where, *moved;
     int32_t *ed, *id, *queue;
-    int32_t *loc, *hkey[2], *hval[2];   // heap FM only
+    int32_t *loc, *hkey[2], *hval[2];
 };
 
 // ---- device priority queue (hunyuangraph_GPU_priorityqueue.h:27-225), run by
@@ -194,50 +224,65 @@ __device__ inline void fence_wave()
     __syncthreads();
 }
 
-// One GGGP + FM trial per wave (hunyuangraph_gpu_BFS_warp_2wayrefine_noedit[_sampling],
-// :2426-3659).  Lane 0 runs the serial BFS; vertex scans, the FM arg-max
-// (gain desc, id asc) and neighbour updates are spread over the 64 lanes.
-// The boundary flag is derived: bnd(v) = deg(v) == 0 || ed[v] > 0, which is
-// the invariant the reference's incremental updates maintain.
-template <bool HEAP>
-__global__ void __launch_bounds__(kWave) k_ip_trials(const int32_t *__restrict__ act, int32_t nact,
-                                                     const Node *__restrict__ nodes, const int32_t *total,
-                                                     const eid_t *__restrict__ fx, const vid_t *__restrict__ fadj,
-                                                     const wgt_t *__restrict__ fw, const wgt_t *__restrict__ fvw,
-                                                     uint64_t seed, int32_t fm_passes, int32_t fm_kind,
-                                                     int32_t lds_cap,
-                                                     uint8_t *__restrict__ trial_where, char *__restrict__ gscratch,
-                                                     int64_t *__restrict__ tcut)
+// Trial gw of the depth: its node (the last active node whose trials start at
+// or before gw).
+__device__ inline int32_t trial_node(const int32_t *__restrict__ act, int32_t nact, const Node *__restrict__ nodes,
+                                     int32_t gw)
 {
-    extern __shared__ char lds[];
-    int32_t gw = blockIdx.x;
-    if (gw >= *total) return;
-    int lane = threadIdx.x;
     int32_t lo = 0, hi = nact - 1;
     while (lo < hi) {
         int32_t mid = (lo + hi + 1) >> 1;
         if (nodes[act[mid]].trial_off <= gw) lo = mid; else hi = mid - 1;
     }
-    const int32_t nid = act[lo];
+    return act[lo];
+}
+
+// Start vertex of trial t (sampled when the node has more vertices than trials).
+__device__ inline int32_t trial_start(const Node &nd, int32_t nid, int32_t n, int32_t t, uint64_t seed, int32_t &draw)
+{
+    if (nd.T >= n) return t;
+    int32_t len = n / nd.T, rem = n % nd.T, left;
+    if (t < rem) { len++; left = t * len; }
+    else left = rem * (len + 1) + (t - rem) * len;
+    return left + (int32_t)(trial_rng(seed, (uint32_t)nid, t, draw++) % (uint64_t)len);
+}
+
+// One GGGP + FM trial per wave (hunyuangraph_gpu_BFS_warp_2wayrefine_noedit[_sampling],
+// :2426-3659) with the queue-driven FM.  Every lane runs the serial BFS;
+// vertex scans and neighbour updates are spread over the 64 lanes.
+// The boundary flag is derived: bnd(v) = deg(v) == 0 || ed[v] > 0, which is
+// the invariant the reference's incremental updates maintain.
+__global__ void __launch_bounds__(kWave) k_ip_trials_heap(const int32_t *__restrict__ act, int32_t nact,
+                                                          const Node *__restrict__ nodes, const int32_t *total,
+                                                          const eid_t *__restrict__ fx,
+                                                          const vid_t *__restrict__ fadj,
+                                                          const wgt_t *__restrict__ fw, const wgt_t *__restrict__ fvw,
+                                                          uint64_t seed, int32_t fm_passes, int32_t fm_kind,
+                                                          int32_t lds_cap, uint8_t *__restrict__ trial_where,
+                                                          char *__restrict__ gscratch, int64_t *__restrict__ tcut)
+{
+    extern __shared__ char lds[];
+    int32_t gw = blockIdx.x;
+    if (gw >= *total) return;
+    int lane = threadIdx.x;
+    const int32_t nid = trial_node(act, nact, nodes, gw);
     const Node nd = nodes[nid];
     const int32_t t = gw - nd.trial_off;
     const int32_t n = nd.end - nd.start, s0 = nd.start;
     char *base;
     if (n <= lds_cap) base = lds;
-    else base = gscratch + nd.soff + (int64_t)t * ((trial_bytes(n, HEAP) + 255) & ~255ll);
+    else base = gscratch + nd.soff + (int64_t)t * ((trial_bytes(n, true, false) + 255) & ~255ll);
     TrialMem M;
     M.where = (uint8_t *)base;
     M.moved = M.where + n;
     M.ed = (int32_t *)(base + (((int64_t)2 * n + 3) & ~3ll));
     M.id = M.ed + n;
     M.queue = M.id + n;
-    if (HEAP) {
-        M.loc = M.queue + n;
-        M.hkey[0] = M.loc + n;
-        M.hval[0] = M.hkey[0] + (n + 1);
-        M.hkey[1] = M.hval[0] + (n + 1);
-        M.hval[1] = M.hkey[1] + (n + 1);
-    }
+    M.loc = M.queue + n;
+    M.hkey[0] = M.loc + n;
+    M.hval[0] = M.hkey[0] + (n + 1);
+    M.hkey[1] = M.hval[0] + (n + 1);
+    M.hval[1] = M.hkey[1] + (n + 1);
     const int64_t tv = nd.tv, onemin = nd.onemin, onemax = nd.onemax, ideal0 = nd.ideal0;
 
     for (int32_t i = lane; i < n; i += kWave) { M.where[i] = 1; M.moved[i] = 0; }
@@ -249,15 +294,8 @@ __global__ void __launch_bounds__(kWave) k_ip_trials(const int32_t *__restrict__
     // neighbours appended in row order (ballot ranks), as a serial scan would.
     int64_t pw0 = 0, pw1 = tv;
     {
-        int32_t draw = 0, start;
-        if (nd.T >= n) {
-            start = t;
-        } else {
-            int32_t len = n / nd.T, rem = n % nd.T, left;
-            if (t < rem) { len++; left = t * len; }
-            else left = rem * (len + 1) + (t - rem) * len;
-            start = left + (int32_t)(trial_rng(seed, (uint32_t)nid, t, draw++) % (uint64_t)len);
-        }
+        int32_t draw = 0;
+        const int32_t start = trial_start(nd, nid, n, t, seed, draw);
         int32_t first = 0, last = 1, nleft = n - 1, drain = 0;
         if (lane == 0) {
             M.queue[0] = start;
@@ -319,8 +357,7 @@ __global__ void __launch_bounds__(kWave) k_ip_trials(const int32_t *__restrict__
     fence_wave();
 
     // ed / id and the cut (compute_v_ed_id_bnd, :23-62).  From here on
-    // moved[v] holds bit 0 = moved in this pass, bit 1 = v has no edges, so
-    // the FM arg-max scan reads only this trial's arrays.
+    // moved[v] holds bit 0 = moved in this pass, bit 1 = v has no edges.
     int64_t cutacc = 0;
     for (int32_t v = lane; v < n; v += kWave) {
         int32_t e = 0, in = 0;
@@ -357,188 +394,78 @@ __global__ void __launch_bounds__(kWave) k_ip_trials(const int32_t *__restrict__
     if (limit > 100) limit = 100;
     int32_t *swaps = M.queue;
 
-    if (HEAP) {
-        // FM driven by two priority queues (FM_2way_cut_refinement,
-        // hunyuangraph_GPU_initialpartition.h:160-300).  Lane 0 runs every
-        // queue operation in the serial order; the lanes share the gain
-        // updates of a move's row.  fm_kind 1: (gain desc, id asc) keys and
-        // the part bounds of the scan FM below, so the moves are the same;
-        // fm_kind 2: the reference's queue order and balance rule
-        // (|ideal0 - pw0| <= origdiff + avgvwgt, weights applied before the
-        // test as hunyuangraph_CPU_2wayrefine.h:133-145 does).
-        Heap q[2];
-        for (int s = 0; s < 2; s++) {
-            q[s].key = M.hkey[s];
-            q[s].val = M.hval[s];
-            q[s].loc = M.loc;
-            q[s].cnt = 0;
-            q[s].ties = fm_kind == 1;
-        }
-        const bool live_rule = fm_kind == 1;
-        const int64_t a20 = (pw[0] + pw[1]) / 20, a2n = 2 * (pw[0] + pw[1]) / n;
-        const int64_t avgvwgt = a20 < a2n ? a20 : a2n;
-        const int64_t origdiff = ideal[0] - pw[0] < 0 ? pw[0] - ideal[0] : ideal[0] - pw[0];
-        for (int32_t pass = 0; pass < fm_passes; pass++) {
-            int64_t mincutorder = -1;
-            int64_t newcut = cut, mincut = cut, initcut = cut;
-            int64_t d0 = ideal[0] - pw[0];
-            int64_t mindiff = d0 < 0 ? -d0 : d0;
-            if (lane == 0) {
-                q[0].cnt = q[1].cnt = 0;
-                for (int32_t v = 0; v < n; v++) {
-                    int32_t e = M.ed[v];
-                    if (e > 0 || (M.moved[v] & 2)) q[M.where[v]].insert(v, e - M.id[v]);
-                }
-            }
-            int32_t nswaps;
-            for (nswaps = 0; nswaps < n; nswaps++) {
-                int from = (ideal[0] - pw[0] < ideal[1] - pw[1]) ? 0 : 1;
-                int to = from ^ 1;
-                int32_t bv = -1, bg = 0;
-                if (lane == 0) {
-                    bv = q[from].top();
-                    if (bv >= 0) bg = M.ed[bv] - M.id[bv];
-                }
-                bv = __shfl(bv, 0, kWave);
-                bg = __shfl(bg, 0, kWave);
-                if (bv == -1) break;
-                int32_t wv = fvw[s0 + bv];
-                newcut -= bg;
-                bool accept;
-                if (live_rule) {
-                    int64_t dd = ideal[0] - pw[0];
-                    dd = dd < 0 ? -dd : dd;
-                    accept = (newcut < mincut && pw[to] + wv <= onemax && pw[from] - wv <= onemax) ||
-                             (newcut == mincut && dd < mindiff);
-                    if (accept) mindiff = dd;
-                    pw[to] += wv;
-                    pw[from] -= wv;
-                } else {
-                    pw[to] += wv;
-                    pw[from] -= wv;
-                    int64_t dd = ideal[0] - pw[0];
-                    dd = dd < 0 ? -dd : dd;
-                    accept = (newcut < mincut && dd <= origdiff + avgvwgt) || (newcut == mincut && dd < mindiff);
-                    if (accept) mindiff = dd;
-                }
-                if (accept) {
-                    mincut = newcut;
-                    mincutorder = nswaps;
-                } else if (nswaps - mincutorder > limit) {
-                    newcut += bg;
-                    pw[from] += wv;
-                    pw[to] -= wv;
-                    break;
-                }
-                if (lane == 0) {
-                    M.where[bv] = (uint8_t)to;
-                    M.moved[bv] |= 1;
-                    swaps[nswaps] = bv;
-                    int32_t tmp = M.ed[bv];
-                    M.ed[bv] = M.id[bv];
-                    M.id[bv] = tmp;
-                }
-                fence_wave();
-                const eid_t rb = fx[s0 + bv], re = fx[s0 + bv + 1];
-                for (eid_t j = rb + lane; j < re; j += kWave) {
-                    int32_t x = fadj[j] - s0;
-                    int32_t kw = (M.where[x] == from) ? -fw[j] : fw[j];
-                    M.id[x] += kw;     // rows hold no duplicates: one lane per neighbour
-                    M.ed[x] -= kw;
-                }
-                fence_wave();
-                if (lane == 0) {
-                    // queue upkeep in row order: a neighbour that left the
-                    // boundary is deleted, one that stays is re-keyed, one
-                    // that joined is inserted (moved vertices stay out)
-                    for (eid_t j = rb; j < re; j++) {
-                        int32_t x = fadj[j] - s0;
-                        uint8_t st = M.moved[x];
-                        if (st & 1) continue;
-                        int32_t e = M.ed[x];
-                        int32_t kw = (M.where[x] == from) ? -fw[j] : fw[j];
-                        bool was = e + kw > 0;
-                        int sx = M.where[x];
-                        if (was) {
-                            if (e == 0) q[sx].remove(x);
-                            else q[sx].update(x, e - M.id[x]);
-                        } else if (e > 0) {
-                            q[sx].insert(x, e - M.id[x]);
-                        }
-                    }
-                }
-                fence_wave();
-            }
-            for (int32_t i = lane; i < nswaps; i += kWave) M.moved[swaps[i]] &= 2;
-            fence_wave();
-            for (nswaps--; nswaps > mincutorder; nswaps--) {
-                int32_t v = swaps[nswaps];
-                int from = M.where[v];
-                int to = from ^ 1;
-                int32_t wv = fvw[s0 + v];
-                fence_wave();
-                if (lane == 0) {
-                    M.where[v] = (uint8_t)to;
-                    int32_t tmp = M.ed[v];
-                    M.ed[v] = M.id[v];
-                    M.id[v] = tmp;
-                }
-                pw[to] += wv;
-                pw[from] -= wv;
-                fence_wave();
-                for (eid_t j = fx[s0 + v] + lane; j < fx[s0 + v + 1]; j += kWave) {
-                    int32_t x = fadj[j] - s0;
-                    int32_t kw = (M.where[x] == from) ? -fw[j] : fw[j];
-                    M.id[x] += kw;
-                    M.ed[x] -= kw;
-                }
-                fence_wave();
-            }
-            cut = mincut;
-            if (mincutorder <= 0 || mincut == initcut) break;
-        }
+    // FM driven by two priority queues (FM_2way_cut_refinement,
+    // hunyuangraph_GPU_initialpartition.h:160-300).  Lane 0 runs every
+    // queue operation in the serial order; the lanes share the gain
+    // updates of a move's row.  fm_kind 1: (gain desc, id asc) keys and
+    // the part bounds of the scan FM, so the moves are the same;
+    // fm_kind 2: the reference's queue order and balance rule
+    // (|ideal0 - pw0| <= origdiff + avgvwgt, weights applied before the
+    // test as hunyuangraph_CPU_2wayrefine.h:133-145 does).
+    Heap q[2];
+    for (int s = 0; s < 2; s++) {
+        q[s].key = M.hkey[s];
+        q[s].val = M.hval[s];
+        q[s].loc = M.loc;
+        q[s].cnt = 0;
+        q[s].ties = fm_kind == 1;
     }
-
-    for (int32_t pass = 0; pass < (HEAP ? 0 : fm_passes); pass++) {
+    const bool live_rule = fm_kind == 1;
+    const int64_t a20 = (pw[0] + pw[1]) / 20, a2n = 2 * (pw[0] + pw[1]) / n;
+    const int64_t avgvwgt = a20 < a2n ? a20 : a2n;
+    const int64_t origdiff = ideal[0] - pw[0] < 0 ? pw[0] - ideal[0] : ideal[0] - pw[0];
+    for (int32_t pass = 0; pass < fm_passes; pass++) {
         int64_t mincutorder = -1;
         int64_t newcut = cut, mincut = cut, initcut = cut;
         int64_t d0 = ideal[0] - pw[0];
         int64_t mindiff = d0 < 0 ? -d0 : d0;
+        if (lane == 0) {
+            q[0].cnt = q[1].cnt = 0;
+            for (int32_t v = 0; v < n; v++) {
+                int32_t e = M.ed[v];
+                if (e > 0 || (M.moved[v] & 2)) q[M.where[v]].insert(v, e - M.id[v]);
+            }
+        }
         int32_t nswaps;
         for (nswaps = 0; nswaps < n; nswaps++) {
             int from = (ideal[0] - pw[0] < ideal[1] - pw[1]) ? 0 : 1;
             int to = from ^ 1;
             int32_t bv = -1, bg = 0;
-            for (int32_t u = lane; u < n; u += kWave) {
-                uint8_t st = M.moved[u];
-                if (M.where[u] != from || (st & 1)) continue;
-                int32_t e = M.ed[u];
-                bool bnd = e > 0 || (st & 2);
-                if (!bnd) continue;
-                int32_t g = e - M.id[u];
-                if (bv == -1 || g > bg) { bv = u; bg = g; }
+            if (lane == 0) {
+                bv = q[from].top();
+                if (bv >= 0) bg = M.ed[bv] - M.id[bv];
             }
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                int32_t ov = __shfl_xor(bv, o, kWave), og = __shfl_xor(bg, o, kWave);
-                if (ov != -1 && (bv == -1 || og > bg || (og == bg && ov < bv))) { bv = ov; bg = og; }
-            }
+            bv = __shfl(bv, 0, kWave);
+            bg = __shfl(bg, 0, kWave);
             if (bv == -1) break;
             int32_t wv = fvw[s0 + bv];
             newcut -= bg;
-            int64_t dd = ideal[0] - pw[0];
-            dd = dd < 0 ? -dd : dd;
-            if ((newcut < mincut && pw[to] + wv <= onemax && pw[from] - wv <= onemax) ||
-                (newcut == mincut && dd < mindiff)) {
+            bool accept;
+            if (live_rule) {
+                int64_t dd = ideal[0] - pw[0];
+                dd = dd < 0 ? -dd : dd;
+                accept = (newcut < mincut && pw[to] + wv <= onemax && pw[from] - wv <= onemax) ||
+                         (newcut == mincut && dd < mindiff);
+                if (accept) mindiff = dd;
+                pw[to] += wv;
+                pw[from] -= wv;
+            } else {
+                pw[to] += wv;
+                pw[from] -= wv;
+                int64_t dd = ideal[0] - pw[0];
+                dd = dd < 0 ? -dd : dd;
+                accept = (newcut < mincut && dd <= origdiff + avgvwgt) || (newcut == mincut && dd < mindiff);
+                if (accept) mindiff = dd;
+            }
+            if (accept) {
                 mincut = newcut;
-                mindiff = dd;
                 mincutorder = nswaps;
             } else if (nswaps - mincutorder > limit) {
                 newcut += bg;
+                pw[from] += wv;
+                pw[to] -= wv;
                 break;
             }
-            pw[to] += wv;
-            pw[from] -= wv;
             if (lane == 0) {
                 M.where[bv] = (uint8_t)to;
                 M.moved[bv] |= 1;
@@ -548,11 +475,33 @@ __global__ void __launch_bounds__(kWave) k_ip_trials(const int32_t *__restrict__
                 M.id[bv] = tmp;
             }
             fence_wave();
-            for (eid_t j = fx[s0 + bv] + lane; j < fx[s0 + bv + 1]; j += kWave) {
+            const eid_t rb = fx[s0 + bv], re = fx[s0 + bv + 1];
+            for (eid_t j = rb + lane; j < re; j += kWave) {
                 int32_t x = fadj[j] - s0;
                 int32_t kw = (M.where[x] == from) ? -fw[j] : fw[j];
-                atomicAdd(&M.id[x], kw);
-                atomicAdd(&M.ed[x], -kw);
+                M.id[x] += kw;     // rows hold no duplicates: one lane per neighbour
+                M.ed[x] -= kw;
+            }
+            fence_wave();
+            if (lane == 0) {
+                // queue upkeep in row order: a neighbour that left the
+                // boundary is deleted, one that stays is re-keyed, one
+                // that joined is inserted (moved vertices stay out)
+                for (eid_t j = rb; j < re; j++) {
+                    int32_t x = fadj[j] - s0;
+                    uint8_t st = M.moved[x];
+                    if (st & 1) continue;
+                    int32_t e = M.ed[x];
+                    int32_t kw = (M.where[x] == from) ? -fw[j] : fw[j];
+                    bool was = e + kw > 0;
+                    int sx = M.where[x];
+                    if (was) {
+                        if (e == 0) q[sx].remove(x);
+                        else q[sx].update(x, e - M.id[x]);
+                    } else if (e > 0) {
+                        q[sx].insert(x, e - M.id[x]);
+                    }
+                }
             }
             fence_wave();
         }
@@ -576,8 +525,8 @@ __global__ void __launch_bounds__(kWave) k_ip_trials(const int32_t *__restrict__
             for (eid_t j = fx[s0 + v] + lane; j < fx[s0 + v + 1]; j += kWave) {
                 int32_t x = fadj[j] - s0;
                 int32_t kw = (M.where[x] == from) ? -fw[j] : fw[j];
-                atomicAdd(&M.id[x], kw);
-                atomicAdd(&M.ed[x], -kw);
+                M.id[x] += kw;
+                M.ed[x] -= kw;
             }
             fence_wave();
         }
@@ -588,6 +537,827 @@ __global__ void __launch_bounds__(kWave) k_ip_trials(const int32_t *__restrict__
     uint8_t *out = trial_where + nd.woff + (int64_t)t * n;
     for (int32_t i = lane; i < n; i += kWave) out[i] = M.where[i];
     if (lane == 0) tcut[gw] = cut;
+}
+
+// ---------------------------------------------------------------- scan FM
+
+// One GGGP + FM trial per block of NT threads, the FM choosing each move by
+// an arg-max scan.  A trial is a serial chain (a BFS step, then an FM move at
+// a time), so its time is the latency of one step times the steps, and each
+// step is made of as few round trips as its data allow:
+//  * the row offsets sit in LDS with the trial, so a row's entries are one
+//    load away, several per lane at once, and the BFS loads the next row while
+//    it works through this one;
+//  * a vertex keeps its external weight ed and its row's weight wd (summed
+//    once per node by k_ip_edges), so its gain is 2 ed - wd and a move changes
+//    one word per neighbour; the BFS keeps ed as it goes, so no pass over all
+//    rows follows it;
+//  * the arg-max reads four vertices per thread and step and reduces on the
+//    VALU;
+//  * 256 threads for node graphs of kWideTrial vertices and more, one wave
+//    below, where a step has no work for more.
+// Used where the dense trials below are not: node graphs of more than kDenseN
+// vertices, or rows that do not ascend.
+constexpr int32_t kWideTrial = 128;
+constexpr uint8_t kStSide = 1, kStMoved = 2, kStAlone = 4;   // state byte: side, queued or moved, no edges
+
+// The node's graph in the forest arrays.
+struct TrialRows {
+    const vid_t *adj;    // the node's entries (forest positions)
+    const wgt_t *w, *vw;
+    int32_t s0;
+    // entries first, first + step, ... of [.., e): neighbour -1 past the end
+    template <int P>
+    __device__ void load(int32_t first, int32_t e, int step, int32_t (&x)[P], int32_t (&wt)[P]) const
+    {
+#pragma unroll
+        for (int q = 0; q < P; q++) {
+            const int32_t j = first + q * step;
+            x[q] = j < e ? adj[j] - s0 : -1;
+            wt[q] = j < e ? w[j] : 0;
+        }
+    }
+};
+
+// The trial's arrays: (ed, wd) per vertex, row offsets from the node's first
+// entry, queue / swap list, state bytes.
+template <class Q>
+struct ScanMem {
+    int2 *ew;
+    int32_t *off;
+    Q *queue;
+    uint8_t *st;
+    __device__ ScanMem(char *base, int32_t n)
+    {
+        const int64_t n4 = (n + 3) & ~3;
+        ew = (int2 *)base;
+        off = (int32_t *)(base + 8 * n4);
+        queue = (Q *)(off + n4 + 4);
+        st = (uint8_t *)(queue + n4);
+    }
+    // marks v queued; whether it was not before (one of several lanes that
+    // mark the same vertex sees it fresh); old: the state byte before
+    __device__ bool mark(int32_t v, uint32_t &old) const
+    {
+        const int sh = 8 * (v & 3);
+        old = (atomicOr((uint32_t *)st + (v >> 2), (uint32_t)kStMoved << sh) >> sh) & 255u;
+        return !(old & kStMoved);
+    }
+};
+
+// GGGP: BFS from a start vertex, moving vertices to side 0 in BFS order, run by
+// one wave: every lane follows the same control flow on the same values; rows
+// are taken 64 entries at a time and the unvisited neighbours appended in row
+// order (ballot ranks), as a serial scan would.  ed is kept current.  Returns
+// side 0's weight.
+template <class Q>
+__device__ inline int64_t trial_grow(const TrialRows &G, const ScanMem<Q> &M, int32_t n, const Node &nd,
+                                     int32_t nid, int32_t t, uint64_t seed)
+{
+    constexpr int P = 4;   // 64-entry pieces of a row in flight
+    const int lane = lane_id();
+    const int64_t onemin = nd.onemin, onemax = nd.onemax;
+    int64_t pw0 = 0, pw1 = nd.tv;
+    int32_t draw = 0;
+    const int32_t start = trial_start(nd, nid, n, t, seed, draw);
+    int32_t first = 0, last = 1, nleft = n - 1, drain = 0;
+    if (lane == 0) {
+        M.queue[0] = (Q)start;
+        M.st[start] |= kStMoved;
+    }
+    wave_lds_sync();
+    // the next vertex in the queue: its position, row and weight, loaded ahead
+    int32_t ahead = -1, av = 0, aw = 0, ab = 0, ae = 0, ax[P], at[P];
+    for (;;) {
+        if (first == last) {
+            if (nleft == 0 || drain) break;
+            // restart from the r-th unvisited vertex in id order
+            int32_t r = (int32_t)(trial_rng(seed, (uint32_t)nid, t, draw++) % (uint64_t)nleft);
+            int32_t v = -1;
+            for (int32_t b0 = 0; b0 < n; b0 += kWave) {
+                int32_t u = b0 + lane;
+                bool un = u < n && !(M.st[u] & kStMoved);
+                uint64_t bal = __ballot(un);
+                int32_t cnt = __popcll(bal);
+                if (r < cnt) {
+                    uint64_t pick = __ballot(un && __popcll(bal & lanemask_lt()) == r);
+                    v = b0 + (__ffsll((long long)pick) - 1);
+                    break;
+                }
+                r -= cnt;
+            }
+            if (lane == 0) {
+                M.queue[0] = (Q)v;
+                M.st[v] |= kStMoved;
+            }
+            wave_lds_sync();
+            first = 0;
+            last = 1;
+            nleft--;
+            ahead = -1;
+        }
+        int32_t v, wv, rb, re, x[P], w[P];
+        if (ahead == first) {
+            v = av;
+            wv = aw;
+            rb = ab;
+            re = ae;
+#pragma unroll
+            for (int q = 0; q < P; q++) {
+                x[q] = ax[q];
+                w[q] = at[q];
+            }
+        } else {
+            v = wave_read((int32_t)M.queue[first], 0);
+            rb = wave_read(M.off[v], 0);
+            re = wave_read(M.off[v + 1], 0);
+            wv = G.vw[v];
+            G.load(rb + lane, re, kWave, x, w);
+        }
+        first++;
+        if (first < last) {
+            ahead = first;
+            av = wave_read((int32_t)M.queue[first], 0);
+            ab = wave_read(M.off[av], 0);
+            ae = wave_read(M.off[av + 1], 0);
+            aw = G.vw[av];
+            G.load(ab + lane, ae, kWave, ax, at);
+        }
+        wv = wave_read(wv, 0);
+        if (pw0 > 0 && pw1 - wv < onemin) { drain = 1; continue; }
+        pw0 += wv;
+        pw1 -= wv;
+        const bool stop = pw1 <= onemax;
+        if (lane == 0) {
+            M.st[v] &= (uint8_t)~kStSide;
+            const int2 e = M.ew[v];
+            M.ew[v] = make_int2(e.y - e.x, e.y);
+        }
+        drain = 0;
+        // the row: neighbours of side 1 gain an external edge, those of side 0
+        // lose one; the unvisited ones join the queue (not after the last vertex)
+        for (int32_t j0 = rb; j0 < re; j0 += P * kWave) {
+            if (j0 > rb) G.load(j0 + lane, re, kWave, x, w);
+            bool fresh[P];
+#pragma unroll
+            for (int q = 0; q < P; q++) {
+                fresh[q] = false;
+                if (x[q] < 0) continue;
+                uint32_t old;
+                fresh[q] = M.mark(x[q], old);
+                atomicAdd(&M.ew[x[q]].x, (old & kStSide) ? w[q] : -w[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < P; q++) {
+                const uint64_t bal = __ballot(fresh[q]);
+                if (fresh[q]) M.queue[last + __popcll(bal & lanemask_lt())] = (Q)x[q];
+                last += __popcll(bal);
+                nleft -= __popcll(bal);
+            }
+        }
+        wave_lds_sync();
+        if (stop) break;
+    }
+    return pw0;
+}
+
+// Moves v (a vertex of side `from`) to the other side: its external and
+// internal weight change places and its neighbours' external weight changes
+// by each edge.  x, w hold the row's first P*NT entries (x = -1 past the end).
+template <int NT, int P, class Q>
+__device__ inline void trial_move(const TrialRows &G, const ScanMem<Q> &M, int32_t v, int from, int32_t rb,
+                                  int32_t re, int32_t (&x)[P], int32_t (&w)[P])
+{
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        const int2 e = M.ew[v];
+        M.ew[v] = make_int2(e.y - e.x, e.y);
+    }
+    for (int32_t j0 = rb; j0 < re; j0 += P * NT) {
+        if (j0 > rb) G.load(j0 + tid, re, NT, x, w);
+#pragma unroll
+        for (int q = 0; q < P; q++) {
+            if (x[q] < 0) continue;
+            atomicAdd(&M.ew[x[q]].x, (M.st[x[q]] & kStSide) == from ? w[q] : -w[q]);
+        }
+    }
+}
+
+template <int NT>
+struct TrialShared {
+    int2 best[2][NT / kWave];   // each wave's (gain, vertex), by parity of the move
+    int64_t sum[NT / kWave];
+    int64_t pw0;
+};
+
+// The trial in arrays at `base`; returns its cut.  Every thread of the block
+// calls it and follows the same control flow.
+template <int NT, class Q>
+__device__ inline int64_t scan_trial(const TrialRows &G, char *base, int32_t n, const Node &nd, int32_t nid, int32_t t,
+                                     const eid_t *__restrict__ fx, const int32_t *__restrict__ fwd, uint64_t seed,
+                                     int32_t fm_passes, TrialShared<NT> &S)
+{
+    constexpr int NW = NT / kWave;
+    constexpr int P = NT == kWave ? 4 : 2;   // row entries per thread in flight
+    const int tid = threadIdx.x, lane = lane_id();
+    const ScanMem<Q> M(base, n);
+    const eid_t fb = fx[G.s0];
+    for (int32_t i = tid; i <= n; i += NT) M.off[i] = (int32_t)(fx[G.s0 + i] - fb);
+    for (int32_t i = tid; i < ((n + 3) & ~3); i += NT) {
+        M.st[i] = kStSide;
+        M.ew[i] = make_int2(0, i < n ? fwd[G.s0 + i] : 0);   // the padding stays out of the arg-max: ed 0, not alone
+    }
+    __syncthreads();
+    if (tid < kWave) {
+        const int64_t w0 = trial_grow<Q>(G, M, n, nd, nid, t, seed);
+        if (tid == 0) S.pw0 = w0;
+    }
+    __syncthreads();
+    // side weights (an array indexed by the side would go to scratch memory)
+    int64_t pw0 = S.pw0, pw1 = nd.tv - S.pw0;
+    const int64_t ideal0 = nd.ideal0, ideal1 = nd.tv - nd.ideal0;
+    const int64_t onemax = nd.onemax;
+
+    // the cut (compute_v_ed_id_bnd, :23-62); from here on kStMoved means
+    // moved in this pass
+    int64_t cutacc = 0;
+    for (int32_t v = tid; v < n; v += NT) {
+        const int2 e = M.ew[v];
+        M.st[v] = (uint8_t)((M.st[v] & kStSide) | (M.off[v] == M.off[v + 1] ? kStAlone : 0));
+        cutacc += e.x;
+    }
+    cutacc = wave_sum(cutacc);
+    if (lane == 0) S.sum[tid / kWave] = cutacc;
+    __syncthreads();
+    int64_t cut = 0;
+#pragma unroll
+    for (int i = 0; i < NW; i++) cut += S.sum[i];
+    cut /= 2;
+
+    int64_t limit = n / 100;
+    if (limit < 15) limit = 15;
+    if (limit > 100) limit = 100;
+    Q *swaps = M.queue;
+    for (int32_t pass = 0; pass < fm_passes; pass++) {
+        int64_t mincutorder = -1;
+        int64_t newcut = cut, mincut = cut, initcut = cut;
+        int64_t d0 = ideal0 - pw0;
+        int64_t mindiff = d0 < 0 ? -d0 : d0;
+        int32_t nswaps;
+        for (nswaps = 0; nswaps < n; nswaps++) {
+            const int from = (ideal0 - pw0 < ideal1 - pw1) ? 0 : 1;
+            // the boundary vertex of side `from`, not moved in this pass, of
+            // largest gain (2 ed - wd; |gain| < 2^30), the smallest id among equals
+            int32_t g = INT32_MIN, bv = INT32_MAX;
+            for (int32_t u0 = tid * 4; u0 < n; u0 += NT * 4) {
+                const int4 a = *(const int4 *)(M.ew + u0), b = *(const int4 *)(M.ew + u0 + 2);
+                const uint32_t s4 = *(const uint32_t *)(M.st + u0);
+                const int32_t ed[4] = {a.x, a.z, b.x, b.z}, wd[4] = {a.y, a.w, b.y, b.w};
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const uint32_t st = (s4 >> (8 * q)) & 255u;
+                    const bool can = ((st & (kStSide | kStMoved)) == (uint32_t)from) & ((ed[q] > 0) | ((st & kStAlone) != 0));
+                    const int32_t gq = can ? 2 * ed[q] - wd[q] : INT32_MIN;
+                    bv = gq > g ? u0 + q : bv;
+                    g = gq > g ? gq : g;
+                }
+            }
+            const int32_t gm = lanes_reduce<kWave>(g, [](int32_t a, int32_t b) { return a > b ? a : b; });
+            bv = lanes_reduce<kWave>(g == gm ? bv : INT32_MAX, [](int32_t a, int32_t b) { return a < b ? a : b; });
+            g = gm;
+            if constexpr (NW > 1) {
+                int2 *slot = S.best[nswaps & 1];
+                if (lane == 0) slot[tid / kWave] = make_int2(g, bv);
+                __syncthreads();
+                g = INT32_MIN;
+                bv = INT32_MAX;
+#pragma unroll
+                for (int i = 0; i < NW; i++) {   // waves hold ascending ids only within a step: compare them
+                    const int2 o = slot[i];
+                    const bool take = (o.x > g) | ((o.x == g) & (o.y < bv));
+                    g = take ? o.x : g;
+                    bv = take ? o.y : bv;
+                }
+            }
+            // the same in every lane: kept in scalar registers, so that the
+            // serial decisions below are scalar branches
+            bv = wave_read(bv, 0);
+            const int32_t bg = wave_read(g, 0);
+            if (bg == INT32_MIN) break;
+            const int32_t rb = wave_read(M.off[bv], 0), re = wave_read(M.off[bv + 1], 0);
+            const int32_t wv = wave_read(G.vw[bv], 0);
+            int32_t x[P], w[P];   // the row, on its way while the move is judged
+            G.load(rb + tid, re, NT, x, w);
+            newcut -= bg;
+            int64_t dd = ideal0 - pw0;
+            dd = dd < 0 ? -dd : dd;
+            const int64_t into = (from ? pw0 : pw1) + wv, outof = (from ? pw1 : pw0) - wv;
+            // selects instead of short-circuit branches: those were compiled into
+            // code that kept the old mincutorder where the second test alone held
+            const bool keep = ((newcut < mincut) & (into <= onemax) & (outof <= onemax)) |
+                              ((newcut == mincut) & (dd < mindiff));
+            if (!keep && nswaps - mincutorder > limit) break;
+            mincut = keep ? newcut : mincut;
+            mindiff = keep ? dd : mindiff;
+            mincutorder = keep ? nswaps : mincutorder;
+            pw0 = from ? into : outof;
+            pw1 = from ? outof : into;
+            if (tid == 0) {
+                M.st[bv] = (uint8_t)((M.st[bv] ^ kStSide) | kStMoved);
+                swaps[nswaps] = (Q)bv;
+            }
+            trial_move<NT, P, Q>(G, M, bv, from, rb, re, x, w);
+            __syncthreads();
+        }
+        __syncthreads();   // the swap list is whole
+        for (int32_t i = tid; i < nswaps; i += NT) M.st[swaps[i]] &= (uint8_t)~kStMoved;
+        __syncthreads();
+        for (nswaps--; nswaps > mincutorder; nswaps--) {
+            const int32_t v = wave_read((int32_t)swaps[nswaps], 0);
+            const int from = wave_read((int32_t)M.st[v], 0) & kStSide;
+            const int32_t rb = wave_read(M.off[v], 0), re = wave_read(M.off[v + 1], 0);
+            const int32_t wv = wave_read(G.vw[v], 0);
+            int32_t x[P], w[P];
+            G.load(rb + tid, re, NT, x, w);
+            __syncthreads();   // every thread has read v's side
+            if (tid == 0) M.st[v] ^= kStSide;
+            pw0 += from ? wv : -wv;
+            pw1 += from ? -wv : wv;
+            trial_move<NT, P, Q>(G, M, v, from, rb, re, x, w);
+            __syncthreads();
+        }
+        cut = mincut;
+        if (mincutorder <= 0 || mincut == initcut) break;
+    }
+    return cut;
+}
+
+template <int NT>
+__global__ void __launch_bounds__(NT) k_ip_trials(const int32_t *__restrict__ act, int32_t nact,
+                                                  const Node *__restrict__ nodes, const int32_t *total,
+                                                  const eid_t *__restrict__ fx, const vid_t *__restrict__ fadj,
+                                                  const wgt_t *__restrict__ fw, const wgt_t *__restrict__ fvw,
+                                                  const int32_t *__restrict__ fwd, uint64_t seed, int32_t fm_passes,
+                                                  int32_t lds_cap,
+                                                  uint8_t *__restrict__ trial_where, char *__restrict__ gscratch,
+                                                  int64_t *__restrict__ tcut)
+{
+    extern __shared__ __align__(16) char lds[];
+    __shared__ TrialShared<NT> S;
+    const int32_t gw = blockIdx.x;
+    if (gw >= *total) return;
+    const int32_t nid = trial_node(act, nact, nodes, gw);
+    const Node nd = nodes[nid];
+    const int32_t t = gw - nd.trial_off, n = nd.end - nd.start;
+    const eid_t fb = fx[nd.start];
+    const TrialRows G{fadj + fb, fw + fb, fvw + nd.start, nd.start};
+    const uint8_t *st;
+    int64_t cut;
+    if (n <= lds_cap) {   // a 16-bit queue: lds_cap < 2^16
+        cut = scan_trial<NT, uint16_t>(G, lds, n, nd, nid, t, fx, fwd, seed, fm_passes, S);
+        st = ScanMem<uint16_t>(lds, n).st;
+    } else {
+        char *base = gscratch + nd.soff + (int64_t)t * ((trial_bytes(n, false, false) + 255) & ~255ll);
+        cut = scan_trial<NT, int32_t>(G, base, n, nd, nid, t, fx, fwd, seed, fm_passes, S);
+        st = ScanMem<int32_t>(base, n).st;
+    }
+    uint8_t *out = trial_where + nd.woff + (int64_t)t * n;
+    for (int32_t i = threadIdx.x; i < n; i += NT) out[i] = st[i] & kStSide;
+    if (threadIdx.x == 0) tcut[gw] = cut;
+}
+
+// ---------------------------------------------------------------- dense scan FM
+
+// The same trial on a dense copy of the node's graph, for coarsest graphs of
+// up to kDenseN vertices with strictly ascending rows.  A trial is bound by the
+// latency of its serial steps; on lists a step was index load, weight load,
+// LDS atomics per neighbour, then a scan of LDS.  Here
+//  * a thread owns 4 or 8 vertices for the whole trial, their state in
+//    registers: S0 (edge weight to side 0), row weight, side, moved;
+//  * moving v adds or subtracts row v of the weight matrix W: one 16-byte load
+//    per 4 vertices, no indices and no atomics, whatever the row's length; the
+//    sums do not depend on the order, so a pass is undone, and the sums after
+//    the BFS are made, with many rows in flight;
+//  * a BFS step is one word of the adjacency bit matrix per lane, masked with
+//    the unvisited ones;
+//  * a move takes one barrier (none with one wave).
+// The matrices are built once per depth (5-9 us).  All depths of a partition
+// (one wave per trial on lists -> this): R-MAT 2^22, k = 256 (999 vertices,
+// 297k entries) 5.6 -> 1.6 ms, R-MAT 2^17, k = 1000 (1945 vertices) 17.5 ->
+// 3.8 ms, 3-D RGG 2^20, k = 64 (430 vertices) 3.3 -> 1.2 ms.
+constexpr int32_t kDenseN = 4096;
+
+struct DenseNode {
+    const int32_t *W;      // n rows of `stride` words (a multiple of 4, zero past n)
+    const uint32_t *B;     // n rows of `words` words
+    const wgt_t *vw;
+    const int32_t *wd;
+    int32_t n, stride, words;
+};
+
+__host__ __device__ inline int64_t dense_stride(int64_t n) { return (n + 3) & ~3ll; }
+__host__ __device__ inline int64_t dense_words(int64_t n) { return (n + 31) / 32; }
+
+// Rows of the weight and bit matrices of the depth's active nodes: a block per
+// vertex spreads its list row in LDS and writes it out in order.
+__global__ void __launch_bounds__(256) k_ip_dense(int32_t n, const int32_t *__restrict__ node_of,
+                                                  const Node *__restrict__ nodes, const eid_t *__restrict__ fx,
+                                                  const vid_t *__restrict__ fadj, const wgt_t *__restrict__ fw,
+                                                  int32_t *__restrict__ W, uint32_t *__restrict__ B)
+{
+    extern __shared__ int32_t row[];
+    const int32_t v = blockIdx.x, tid = threadIdx.x;
+    const Node &nd = nodes[node_of[v]];
+    if (nd.k < 2) return;
+    const int32_t nn = nd.end - nd.start, s0 = nd.start;
+    const int32_t stride = (int32_t)dense_stride(nn), words = (int32_t)dense_words(nn);
+    for (int32_t i = tid; i < words * 32; i += 256) row[i] = 0;
+    __syncthreads();
+    const eid_t e = fx[v + 1];
+#pragma unroll 4
+    for (eid_t j = fx[v] + tid; j < e; j += 256) row[fadj[j] - s0] = fw[j];
+    __syncthreads();
+    int32_t *wr = W + nd.doff + (int64_t)(v - s0) * stride;
+    for (int32_t i = tid; i < stride; i += 256) wr[i] = row[i];
+    uint32_t *br = B + nd.boff + (int64_t)(v - s0) * words;
+    for (int32_t i0 = tid & ~(kWave - 1); i0 < words * 32; i0 += 256) {   // whole waves, 64 entries each
+        const int32_t i = i0 + lane_id();
+        const uint64_t m = __ballot(i < words * 32 && row[i] != 0);
+        if (lane_id() < 2 && i0 / 32 + lane_id() < words) br[i0 / 32 + lane_id()] = (uint32_t)(m >> (32 * lane_id()));
+    }
+}
+
+// trial_grow on the bit matrix (WPL words per lane): lists the vertices of side
+// 0 in `taken` and sets their side bytes to 0; returns their number and weight.
+template <int WPL>
+__device__ inline int32_t dense_grow(const DenseNode &D, uint16_t *queue, uint16_t *taken, uint8_t *side,
+                                     const Node &nd, int32_t nid, int32_t t, uint64_t seed, int64_t &w0)
+{
+    const int lane = lane_id();
+    const int32_t n = D.n;
+    const int64_t onemin = nd.onemin, onemax = nd.onemax;
+    int64_t pw0 = 0, pw1 = nd.tv;
+    int32_t draw = 0, nt = 0;
+    const int32_t start = trial_start(nd, nid, n, t, seed, draw);
+    int32_t first = 0, last = 1, nleft = n - 1, drain = 0;
+    uint32_t open[WPL];   // unvisited vertices among this lane's 32 * WPL
+#pragma unroll
+    for (int q = 0; q < WPL; q++) {
+        const int32_t left = n - (lane * WPL + q) * 32;
+        open[q] = left >= 32 ? ~0u : (left > 0 ? (1u << left) - 1u : 0u);
+    }
+    auto visit = [&](int32_t v) {
+        if (lane == 0) queue[0] = (uint16_t)v;
+#pragma unroll
+        for (int q = 0; q < WPL; q++)
+            if (v / 32 == lane * WPL + q) open[q] &= ~(1u << (v & 31));
+    };
+    auto load_row = [&](int32_t v, uint32_t (&b)[WPL]) {
+#pragma unroll
+        for (int q = 0; q < WPL; q++) {
+            const int32_t i = lane * WPL + q;
+            b[q] = i < D.words ? D.B[(int64_t)v * D.words + i] : 0u;
+        }
+    };
+    visit(start);
+    wave_lds_sync();
+    int32_t ahead = -1, av = 0, aw = 0;   // the next vertex of the queue, loaded ahead
+    uint32_t ab[WPL];
+    for (;;) {
+        if (first == last) {
+            if (nleft == 0 || drain) break;
+            // restart from the r-th unvisited vertex in id order
+            int32_t r = (int32_t)(trial_rng(seed, (uint32_t)nid, t, draw++) % (uint64_t)nleft);
+            int32_t own = 0;
+#pragma unroll
+            for (int q = 0; q < WPL; q++) own += __popc(open[q]);
+            const int32_t before = wave_inclusive_scan(own) - own;
+            int32_t v = -1;
+            if (r >= before && r < before + own) {
+                r -= before;
+#pragma unroll
+                for (int q = 0; q < WPL; q++) {
+                    uint32_t b = open[q];
+                    const int32_t c = __popc(b);
+                    if (v < 0 && r < c) {
+                        for (; r > 0; r--) b &= b - 1;
+                        v = (lane * WPL + q) * 32 + (__ffs(b) - 1);
+                    }
+                    r -= c;
+                }
+            }
+            v = wave_max(v);
+            visit(v);
+            wave_lds_sync();
+            first = 0;
+            last = 1;
+            nleft--;
+            ahead = -1;
+        }
+        int32_t v, wv;
+        uint32_t b[WPL];
+        if (ahead == first) {
+            v = av;
+            wv = aw;
+#pragma unroll
+            for (int q = 0; q < WPL; q++) b[q] = ab[q];
+        } else {
+            v = wave_read((int32_t)queue[first], 0);
+            wv = D.vw[v];
+            load_row(v, b);
+        }
+        first++;
+        if (first < last) {
+            ahead = first;
+            av = wave_read((int32_t)queue[first], 0);
+            aw = D.vw[av];
+            load_row(av, ab);
+        }
+        wv = wave_read(wv, 0);
+        if (pw0 > 0 && pw1 - wv < onemin) { drain = 1; continue; }
+        pw0 += wv;
+        pw1 -= wv;
+        if (lane == 0) {
+            side[v] = 0;
+            taken[nt] = (uint16_t)v;
+        }
+        nt++;
+        if (pw1 <= onemax) break;
+        drain = 0;
+        // the unvisited neighbours join the queue in id (row) order
+        int32_t cnt = 0;
+#pragma unroll
+        for (int q = 0; q < WPL; q++) {
+            b[q] &= open[q];
+            open[q] &= ~b[q];
+            cnt += __popc(b[q]);
+        }
+        const int32_t incl = wave_inclusive_scan(cnt), tot = wave_read(incl, kWave - 1);
+        int32_t at = last + incl - cnt;
+#pragma unroll
+        for (int q = 0; q < WPL; q++) {
+            uint32_t f = b[q];
+            while (f) {
+                queue[at++] = (uint16_t)((lane * WPL + q) * 32 + (__ffs(f) - 1));
+                f &= f - 1;
+            }
+        }
+        last += tot;
+        nleft -= tot;
+        wave_lds_sync();
+    }
+    w0 = pw0;
+    return nt;
+}
+
+template <int NT>
+struct DenseShared {
+    int2 best[2][NT / kWave];   // each wave's (gain, vertex), by parity of the move
+    int64_t sum[NT / kWave];
+    int64_t pw0;
+    int32_t ntaken;
+};
+
+template <int NT>
+__device__ inline void trial_sync()
+{
+    if constexpr (NT == kWave) wave_lds_sync();   // (the block's other waves have left)
+    else __syncthreads();
+}
+
+// LDS of a dense trial: queue / swap list and taken list (u16), side bytes.
+__host__ __device__ inline int64_t dense_bytes(int64_t n) { return 5 * dense_stride(n) + 16; }
+
+template <int NT, int V, int NTMAX>
+__device__ inline int64_t dense_trial(const DenseNode &D, char *lds, const Node &nd, int32_t nid, int32_t t,
+                                      uint64_t seed, int32_t fm_passes, DenseShared<NTMAX> &S,
+                                      uint8_t *__restrict__ out)
+{
+    constexpr int NW = NT / kWave, C = V / 4;
+    const int tid = threadIdx.x, lane = lane_id();
+    const int32_t n = D.n, n4 = D.stride;
+    uint16_t *queue = (uint16_t *)lds, *taken = queue + n4;
+    uint8_t *sideb = (uint8_t *)(taken + n4);
+    for (int32_t i = tid * 4; i < n4; i += NT * 4) *(uint32_t *)(sideb + i) = 0x01010101u;
+    trial_sync<NT>();
+    if (tid < kWave) {
+        int64_t w0;
+        const int32_t nt = n <= 2048 ? dense_grow<1>(D, queue, taken, sideb, nd, nid, t, seed, w0)
+                                     : dense_grow<2>(D, queue, taken, sideb, nd, nid, t, seed, w0);
+        if (tid == 0) {
+            S.pw0 = w0;
+            S.ntaken = nt;
+        }
+    }
+    trial_sync<NT>();
+    int64_t pw0 = S.pw0, pw1 = nd.tv - S.pw0;
+    const int64_t ideal0 = nd.ideal0, ideal1 = nd.tv - nd.ideal0;
+    const int64_t onemax = nd.onemax;
+
+    // the thread's vertices: chunk c holds u = c*4*NT + 4*tid .. + 3
+    int32_t s[V], wd[V];
+    uint32_t side = 0, gone = 0, alone = 0;   // bits: side 1; outside the node; no edges
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int32_t u0 = c * 4 * NT + 4 * tid;
+        const uint32_t s4 = u0 < n4 ? *(const uint32_t *)(sideb + u0) : 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int i = c * 4 + j;
+            const bool in = u0 + j < n;
+            s[i] = 0;
+            wd[i] = in ? D.wd[u0 + j] : 0;
+            side |= (in ? (s4 >> (8 * j)) & 1u : 0u) << i;
+            gone |= (in ? 0u : 1u) << i;
+            alone |= (in && wd[i] == 0 ? 1u : 0u) << i;
+        }
+    }
+    // s += sign * row v; w[] holds the row's pieces
+    auto load = [&](int32_t v, int4 (&w)[C]) {
+        const int32_t *r = D.W + (int64_t)v * n4;
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const int32_t u0 = c * 4 * NT + 4 * tid;
+            w[c] = u0 < n4 ? *(const int4 *)(r + u0) : make_int4(0, 0, 0, 0);
+        }
+    };
+    auto add = [&](int sign, const int4 (&w)[C]) {
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            s[c * 4] += sign * w[c].x;
+            s[c * 4 + 1] += sign * w[c].y;
+            s[c * 4 + 2] += sign * w[c].z;
+            s[c * 4 + 3] += sign * w[c].w;
+        }
+    };
+    // sums over lists of rows: R rows in flight
+    constexpr int R = V == 4 ? 4 : 2;
+    {
+        const int32_t nt = S.ntaken;
+        for (int32_t i = 0; i < nt; i += R) {
+            int4 w[R][C];
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                load(wave_read((int32_t)taken[i + r < nt ? i + r : i], 0), w[r]);
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                if (i + r < nt) add(1, w[r]);
+        }
+    }
+    // the cut: every cut edge once, from its end in side 1
+    int64_t cut = 0;
+#pragma unroll
+    for (int i = 0; i < V; i++) cut += (side >> i) & 1u ? s[i] : 0;
+    cut = wave_sum(cut);
+    if constexpr (NW > 1) {
+        if (lane == 0) S.sum[tid / kWave] = cut;
+        __syncthreads();
+        cut = 0;
+#pragma unroll
+        for (int i = 0; i < NW; i++) cut += S.sum[i];
+    }
+
+    int64_t limit = n / 100;
+    if (limit < 15) limit = 15;
+    if (limit > 100) limit = 100;
+    uint16_t *swaps = queue;   // vertex, with the side it left in bit 15
+    for (int32_t pass = 0; pass < fm_passes; pass++) {
+        int64_t mincutorder = -1;
+        int64_t newcut = cut, mincut = cut, initcut = cut;
+        int64_t d0 = ideal0 - pw0;
+        int64_t mindiff = d0 < 0 ? -d0 : d0;
+        uint32_t out_of_play = gone;   // and moved in this pass
+        int32_t nswaps;
+        for (nswaps = 0; nswaps < n; nswaps++) {
+            const int from = (ideal0 - pw0 < ideal1 - pw1) ? 0 : 1;
+            // the boundary vertex of side `from`, not moved in this pass, of
+            // largest gain (2 ed - wd; |gain| < 2^30), the smallest id among equals
+            const uint32_t play = (from ? side : ~side) & ~out_of_play;
+            int32_t g = INT32_MIN, bv = INT32_MAX;
+#pragma unroll
+            for (int i = 0; i < V; i++) {
+                const int32_t ed = from ? s[i] : wd[i] - s[i];
+                const bool can = ((play >> i) & 1u) != 0 && (ed > 0 || ((alone >> i) & 1u) != 0);
+                const int32_t gi = can ? 2 * ed - wd[i] : INT32_MIN;
+                bv = gi > g ? (i / 4) * 4 * NT + 4 * tid + (i & 3) : bv;
+                g = gi > g ? gi : g;
+            }
+            const int32_t gm = lanes_reduce<kWave>(g, [](int32_t a, int32_t b) { return a > b ? a : b; });
+            bv = lanes_reduce<kWave>(g == gm ? bv : INT32_MAX, [](int32_t a, int32_t b) { return a < b ? a : b; });
+            g = gm;
+            if constexpr (NW > 1) {
+                int2 *slot = S.best[nswaps & 1];
+                if (lane == 0) slot[tid / kWave] = make_int2(g, bv);
+                __syncthreads();
+                g = INT32_MIN;
+                bv = INT32_MAX;
+#pragma unroll
+                for (int i = 0; i < NW; i++) {
+                    const int2 o = slot[i];
+                    const bool take = (o.x > g) | ((o.x == g) & (o.y < bv));
+                    g = take ? o.x : g;
+                    bv = take ? o.y : bv;
+                }
+            }
+            // the same in every lane: kept in scalar registers, so that the
+            // serial decisions below are scalar branches
+            bv = wave_read(bv, 0);
+            const int32_t bg = wave_read(g, 0);
+            if (bg == INT32_MIN) break;
+            int4 w[C];   // the row, on its way while the move is judged
+            load(bv, w);
+            const int32_t wv = wave_read(D.vw[bv], 0);
+            newcut -= bg;
+            int64_t dd = ideal0 - pw0;
+            dd = dd < 0 ? -dd : dd;
+            const int64_t into = (from ? pw0 : pw1) + wv, outof = (from ? pw1 : pw0) - wv;
+            // selects instead of short-circuit branches: those were compiled into
+            // code that kept the old mincutorder where the second test alone held
+            const bool keep = ((newcut < mincut) & (into <= onemax) & (outof <= onemax)) |
+                              ((newcut == mincut) & (dd < mindiff));
+            if (!keep && nswaps - mincutorder > limit) break;
+            mincut = keep ? newcut : mincut;
+            mindiff = keep ? dd : mindiff;
+            mincutorder = keep ? nswaps : mincutorder;
+            pw0 = from ? into : outof;
+            pw1 = from ? outof : into;
+            const uint32_t own = (bv >> 2) % NT == tid ? 1u << ((bv / (4 * NT)) * 4 + (bv & 3)) : 0u;
+            side ^= own;
+            out_of_play |= own;
+            if (tid == 0) swaps[nswaps] = (uint16_t)(bv | (from << 15));
+            add(from ? 1 : -1, w);
+        }
+        trial_sync<NT>();   // the swap list is whole
+        for (int32_t i = (int32_t)mincutorder + 1; i < nswaps; i += R) {
+            int4 w[R][C];
+            int32_t x[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                x[r] = wave_read((int32_t)swaps[i + r < nswaps ? i + r : i], 0);
+                load(x[r] & 0x7FFF, w[r]);
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if (i + r >= nswaps) break;
+                const int32_t v = x[r] & 0x7FFF, back = x[r] >> 15;   // back to side `back`
+                const int32_t wv = wave_read(D.vw[v], 0);
+                pw0 += back ? -wv : wv;
+                pw1 += back ? wv : -wv;
+                side ^= (v >> 2) % NT == tid ? 1u << ((v / (4 * NT)) * 4 + (v & 3)) : 0u;
+                add(back ? -1 : 1, w[r]);
+            }
+        }
+        cut = mincut;
+        if (mincutorder <= 0 || mincut == initcut) break;
+        trial_sync<NT>();   // every wave has read the swap list
+    }
+#pragma unroll
+    for (int i = 0; i < V; i++) {
+        const int32_t u = (i / 4) * 4 * NT + 4 * tid + (i & 3);
+        if (u < n) out[u] = (uint8_t)((side >> i) & 1u);
+    }
+    return cut;
+}
+
+// A block of NTMAX threads per trial; node graphs of up to 256 vertices keep
+// one wave of it (4 vertices a thread), larger ones 4 or 8 vertices a thread
+// (up to 8 * NTMAX vertices).
+template <int NTMAX>
+__global__ void __launch_bounds__(NTMAX) k_ip_trials_dense(const int32_t *__restrict__ act, int32_t nact,
+                                                           const Node *__restrict__ nodes, const int32_t *total,
+                                                           const int32_t *__restrict__ W,
+                                                           const uint32_t *__restrict__ B,
+                                                           const wgt_t *__restrict__ fvw,
+                                                           const int32_t *__restrict__ fwd, uint64_t seed,
+                                                           int32_t fm_passes, uint8_t *__restrict__ trial_where,
+                                                           int64_t *__restrict__ tcut)
+{
+    extern __shared__ __align__(16) char lds[];
+    __shared__ DenseShared<NTMAX> S;
+    const int32_t gw = blockIdx.x;
+    if (gw >= *total) return;
+    const int32_t nid = trial_node(act, nact, nodes, gw);
+    const Node nd = nodes[nid];
+    const int32_t t = gw - nd.trial_off;
+    DenseNode D;
+    D.n = nd.end - nd.start;
+    D.stride = (int32_t)dense_stride(D.n);
+    D.words = (int32_t)dense_words(D.n);
+    D.W = W + nd.doff;
+    D.B = B + nd.boff;
+    D.vw = fvw + nd.start;
+    D.wd = fwd + nd.start;
+    uint8_t *out = trial_where + nd.woff + (int64_t)t * D.n;
+    int64_t cut;
+    if (D.n <= 4 * kWave) {
+        if (threadIdx.x >= kWave) return;
+        cut = dense_trial<kWave, 4, NTMAX>(D, lds, nd, nid, t, seed, fm_passes, S, out);
+    } else if (D.n <= 4 * NTMAX) {
+        cut = dense_trial<NTMAX, 4, NTMAX>(D, lds, nd, nid, t, seed, fm_passes, S, out);
+    } else {
+        cut = dense_trial<NTMAX, 8, NTMAX>(D, lds, nd, nid, t, seed, fm_passes, S, out);
+    }
+    if (threadIdx.x == 0) tcut[gw] = cut;
 }
 
 // Arg-min cut over a node's trials, first minimum wins (:3713-3812).
@@ -669,80 +1439,85 @@ __global__ void k_ip_f0(int32_t n, const int8_t *__restrict__ side, int32_t *__r
 // Order-preserving split (hunyuangraph_GPU_splitgraph.h:802-944): side-0
 // vertices first, then side-1, each in their old order, inside the node's
 // range.  Rows keep only same-side entries; finished nodes drop their rows.
-__global__ void k_ip_pos(int32_t n, const int32_t *__restrict__ node_of, const Node *__restrict__ nodes,
-                         const int8_t *__restrict__ side, const int32_t *__restrict__ s0, const eid_t *__restrict__ fx,
-                         const vid_t *__restrict__ fadj, int32_t *__restrict__ pos, int32_t *__restrict__ nnode_of,
-                         int32_t *__restrict__ nlabel, const int32_t *__restrict__ label, wgt_t *__restrict__ nfvw,
-                         const wgt_t *__restrict__ fvw, int64_t *__restrict__ ndeg)
+// A wave per vertex: the rows of the coarsest graph are long (a thread per
+// row took 97 us a launch for 2000 rows of about 200 entries).
+__global__ void __launch_bounds__(kRowBS) k_ip_pos(int32_t n, const int32_t *__restrict__ node_of,
+                                                   const Node *__restrict__ nodes, const int8_t *__restrict__ side,
+                                                   const int32_t *__restrict__ s0, const eid_t *__restrict__ fx,
+                                                   const vid_t *__restrict__ fadj, int32_t *__restrict__ pos,
+                                                   int32_t *__restrict__ nnode_of, int32_t *__restrict__ nlabel,
+                                                   const int32_t *__restrict__ label, wgt_t *__restrict__ nfvw,
+                                                   const wgt_t *__restrict__ fvw, int64_t *__restrict__ ndeg)
 {
-    int32_t v = (int32_t)((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (v >= n) return;
-    int32_t id = node_of[v];
-    int8_t sd = side[v];
-    int32_t p;
-    int64_t d = 0;
-    if (sd < 0) {
-        p = v;
-        nnode_of[p] = id;
-    } else {
+    const int32_t v = (int32_t)gindex<kWave>();
+    if (v >= n) return;   // whole waves
+    const int lane = lane_id();
+    const int32_t id = node_of[v];
+    const int8_t sd = side[v];
+    int32_t p = v, d = 0, nid = id;
+    if (sd >= 0) {
         const Node &nd = nodes[id];
-        int32_t before = nd.start > 0 ? s0[nd.start - 1] : 0;
-        int32_t rank0 = (s0[v] - (sd == 0 ? 1 : 0)) - before;
-        int32_t rank1 = (v - nd.start) - rank0;
+        const int32_t before = nd.start > 0 ? s0[nd.start - 1] : 0;
+        const int32_t rank0 = (s0[v] - (sd == 0 ? 1 : 0)) - before;
+        const int32_t rank1 = (v - nd.start) - rank0;
         p = sd == 0 ? nd.start + rank0 : nd.start + nd.cnt0 + rank1;
-        nnode_of[p] = 2 * id + sd;
-        eid_t j = fx[v];
+        nid = 2 * id + sd;
         const eid_t je = fx[v + 1];
-        for (; j + 8 <= je; j += 8) {   // eight entries' loads in flight
-            int32_t x[8];
-#pragma unroll
-            for (int t = 0; t < 8; t++) x[t] = fadj[j + t];
-#pragma unroll
-            for (int t = 0; t < 8; t++) d += side[x[t]] == sd;
-        }
-        for (; j < je; j++) d += side[fadj[j]] == sd;
+#pragma unroll 4
+        for (eid_t j = fx[v] + lane; j < je; j += kWave) d += side[fadj[j]] == sd;
+        d = wave_sum(d);
     }
-    pos[v] = p;
-    nlabel[p] = label[v];
-    nfvw[p] = fvw[v];
-    ndeg[p] = d;
+    if (lane == 0) {
+        nnode_of[p] = nid;
+        pos[v] = p;
+        nlabel[p] = label[v];
+        nfvw[p] = fvw[v];
+        ndeg[p] = d;
+    }
 }
 
-__global__ void k_ip_edges(int32_t n, const int8_t *__restrict__ side, const int32_t *__restrict__ pos,
-                           const eid_t *__restrict__ fx, const vid_t *__restrict__ fadj, const wgt_t *__restrict__ fw,
-                           const eid_t *__restrict__ nfx, vid_t *__restrict__ nfadj, wgt_t *__restrict__ nfw)
+// The same-side entries of each row, in row order, at the row's new place, and
+// their total weight: a wave per row, ranked by ballots.
+__global__ void __launch_bounds__(kRowBS) k_ip_edges(int32_t n, const int8_t *__restrict__ side,
+                                                     const int32_t *__restrict__ pos, const eid_t *__restrict__ fx,
+                                                     const vid_t *__restrict__ fadj, const wgt_t *__restrict__ fw,
+                                                     const eid_t *__restrict__ nfx, vid_t *__restrict__ nfadj,
+                                                     wgt_t *__restrict__ nfw, int32_t *__restrict__ nfwd)
 {
-    int32_t v = (int32_t)((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (v >= n) return;
-    int8_t sd = side[v];
+    constexpr int P = 4;   // 64-entry pieces in flight
+    const int32_t v = (int32_t)gindex<kWave>();
+    if (v >= n) return;   // whole waves
+    const int lane = lane_id();
+    const int8_t sd = side[v];
     if (sd < 0) return;
-    eid_t o = nfx[pos[v]];
-    eid_t j = fx[v];
+    const int32_t np = pos[v];
+    eid_t o = nfx[np];
+    int32_t wsum = 0;
     const eid_t je = fx[v + 1];
-    for (; j + 8 <= je; j += 8) {   // eight entries' loads in flight, written in row order
-        int32_t x[8], w[8], sx[8];
+    for (eid_t j0 = fx[v]; j0 < je; j0 += P * kWave) {
+        int32_t x[P], w[P];
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-            x[t] = fadj[j + t];
-            w[t] = fw[j + t];
+        for (int q = 0; q < P; q++) {
+            const eid_t j = j0 + lane + q * kWave;
+            x[q] = j < je ? fadj[j] : -1;
+            w[q] = j < je ? fw[j] : 0;
         }
 #pragma unroll
-        for (int t = 0; t < 8; t++) sx[t] = side[x[t]] == sd ? pos[x[t]] : -1;
+        for (int q = 0; q < P; q++) x[q] = x[q] >= 0 && side[x[q]] == sd ? pos[x[q]] : -1;
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-            if (sx[t] < 0) continue;
-            nfadj[o] = sx[t];
-            nfw[o] = w[t];
-            o++;
+        for (int q = 0; q < P; q++) {
+            const uint64_t m = __ballot(x[q] >= 0);
+            if (x[q] >= 0) {
+                const eid_t at = o + __popcll(m & lanemask_lt());
+                nfadj[at] = x[q];
+                nfw[at] = w[q];
+                wsum += w[q];
+            }
+            o += __popcll(m);
         }
     }
-    for (; j < je; j++) {
-        int32_t x = fadj[j];
-        if (side[x] != sd) continue;
-        nfadj[o] = pos[x];
-        nfw[o] = fw[j];
-        o++;
-    }
+    wsum = wave_sum(wsum);
+    if (lane == 0) nfwd[np] = wsum;
 }
 
 struct TreeNode { int32_t id, k, fpart; };
@@ -804,9 +1579,9 @@ void initial_partition(Ctx &c, const DevGraph &g, int32_t k, const Params &p, in
     double ub = std::pow((double)p.ub_num / (double)p.ub_den, 1.0 / std::log((double)k));
     const bool heap = fm_uses_heap(p.fm_kind, n);
     const int32_t fm_kind = p.fm_kind < 0 ? (heap ? 1 : 0) : p.fm_kind;
-    int32_t lds_cap = (kLdsBudget - 64) / (kTrialBytesPerVertex + (heap ? kHeapBytesPerVertex : 0));
+    int32_t lds_cap = heap ? (kHeapLdsBudget - 64) / kHeapBytesPerVertex : kScanLdsN;
     int32_t lds_n = std::min(n, lds_cap);
-    size_t lds_bytes = (size_t)trial_bytes(lds_n, heap) + 16;
+    size_t lds_bytes = (size_t)trial_bytes(lds_n, heap, true) + 16;
 
     size_t mark = c.arena.right_mark();
     Node *nodes = c.arena.ralloc<Node>((size_t)ntab);
@@ -823,17 +1598,25 @@ void initial_partition(Ctx &c, const DevGraph &g, int32_t k, const Params &p, in
     int32_t *total = c.arena.ralloc<int32_t>(1);
     int64_t maxtrials = (int64_t)std::min(p.trials, n);
     uint8_t *trial_where = c.arena.ralloc<uint8_t>((size_t)(maxtrials * n));
+    // dense trials: the graph as matrices, rebuilt per depth node by node
+    const bool dense = !heap && g.ascending && n <= kDenseN;
+    int32_t *W = nullptr;
+    uint32_t *B = nullptr;
+    if (dense) {
+        W = c.arena.ralloc<int32_t>((size_t)(n * (dense_stride(n) + 3)));
+        B = c.arena.ralloc<uint32_t>((size_t)(n * (dense_words(n) + 1)));
+    }
     char *gscratch = nullptr;
     if (n > lds_cap) {
         // sum over nodes of T * round256(trial_bytes(nn)): trial_bytes is affine
-        // in nn with a constant below 20, and at most n / lds_cap + 1 nodes
-        // use global scratch
-        size_t gs = (size_t)maxtrials * ((size_t)trial_bytes(n, heap) + 512 * ((size_t)(n / lds_cap) + 1));
+        // in nn but for a constant below 80 a node, and at most n / lds_cap + 1
+        // nodes use global scratch
+        size_t gs = (size_t)maxtrials * ((size_t)trial_bytes(n, heap, false) + 512 * ((size_t)(n / lds_cap) + 1));
         gscratch = c.arena.ralloc<char>(gs);
     }
     // trials of one depth: sum of min(trials, n_node) <= n
     int64_t *tcut = c.arena.ralloc<int64_t>((size_t)n + 1);
-    int32_t *node_of[2], *label[2];
+    int32_t *node_of[2], *label[2], *fwd[2];
     wgt_t *fvw[2], *fw[2];
     eid_t *fx[2];
     vid_t *fadj[2];
@@ -842,6 +1625,7 @@ void initial_partition(Ctx &c, const DevGraph &g, int32_t k, const Params &p, in
         node_of[b] = c.arena.ralloc<int32_t>((size_t)n);
         label[b] = c.arena.ralloc<int32_t>((size_t)n);
         fvw[b] = c.arena.ralloc<wgt_t>((size_t)n);
+        fwd[b] = c.arena.ralloc<int32_t>((size_t)n);
         fx[b] = c.arena.ralloc<eid_t>((size_t)n + 1);
         fadj[b] = c.arena.ralloc<vid_t>((size_t)mm);
         fw[b] = c.arena.ralloc<wgt_t>((size_t)mm);
@@ -852,7 +1636,8 @@ void initial_partition(Ctx &c, const DevGraph &g, int32_t k, const Params &p, in
     int64_t *ndeg = c.arena.ralloc<int64_t>((size_t)n);
 
     unsigned gv = grid_for(n, 256);
-    k_ip_init<<<gv, 256, 0, c.stream>>>(n, g.vwgt, node_of[0], label[0], fvw[0], nodes);
+    k_ip_init<<<grid_groups(n, kWave), kRowBS, 0, c.stream>>>(n, g.vwgt, g.xadj, g.adjwgt, node_of[0], label[0],
+                                                             fvw[0], fwd[0], nodes);
     HGP_LAUNCH_CHECK();
     HGP_CHECK_HIP(hipMemcpyAsync(fx[0], g.xadj, sizeof(eid_t) * ((size_t)n + 1), hipMemcpyDeviceToDevice, c.stream));
     if (g.m > 0) {
@@ -867,15 +1652,41 @@ void initial_partition(Ctx &c, const DevGraph &g, int32_t k, const Params &p, in
         const int32_t *act = act_all + act_off[d];
         k_ip_setup<<<nact, 256, 0, c.stream>>>(act, nodes, fvw[cb], ub, p.trials);
         HGP_LAUNCH_CHECK();
-        k_ip_offsets<<<1, 64, 0, c.stream>>>(act, nact, nodes, lds_cap, heap, total);
+        k_ip_offsets<<<1, 256, 0, c.stream>>>(act, nact, nodes, lds_cap, heap, total);
         HGP_LAUNCH_CHECK();
+        if (dense) {
+            KScope ks(c, "k_ip_dense", 0.0);
+            k_ip_dense<<<(unsigned)n, 256, 4 * 32 * dense_words(n), c.stream>>>(n, node_of[cb], nodes, fx[cb],
+                                                                               fadj[cb], fw[cb], W, B);
+            HGP_LAUNCH_CHECK();
+        }
         int64_t waves = std::min<int64_t>((int64_t)nact * p.trials, n);
-        KScope ks(c, "k_ip_trials", 0.0);
-        auto trials_kernel = heap ? k_ip_trials<true> : k_ip_trials<false>;
-        trials_kernel<<<(unsigned)std::max<int64_t>(waves, 1), kWave, lds_bytes, c.stream>>>(
-            act, nact, nodes, total, fx[cb], fadj[cb], fw[cb], fvw[cb], p.seed, p.fm_passes, fm_kind, lds_cap,
-            trial_where, gscratch, tcut);
-        HGP_LAUNCH_CHECK();
+        {
+            KScope ks(c, "k_ip_trials", 0.0);
+            const unsigned grid = (unsigned)std::max<int64_t>(waves, 1);
+            // the average node graph of the depth decides the block size
+            const bool wide = n / nact >= kWideTrial;
+            if (heap)
+                k_ip_trials_heap<<<grid, kWave, lds_bytes, c.stream>>>(act, nact, nodes, total, fx[cb], fadj[cb],
+                                                                       fw[cb], fvw[cb], p.seed, p.fm_passes, fm_kind,
+                                                                       lds_cap, trial_where, gscratch, tcut);
+            else if (dense && n <= 2048)
+                k_ip_trials_dense<256><<<grid, 256, dense_bytes(n), c.stream>>>(
+                    act, nact, nodes, total, W, B, fvw[cb], fwd[cb], p.seed, p.fm_passes, trial_where, tcut);
+            else if (dense)
+                k_ip_trials_dense<512><<<grid, 512, dense_bytes(n), c.stream>>>(
+                    act, nact, nodes, total, W, B, fvw[cb], fwd[cb], p.seed, p.fm_passes, trial_where, tcut);
+            else if (wide)
+                k_ip_trials<256><<<grid, 256, lds_bytes, c.stream>>>(act, nact, nodes, total, fx[cb], fadj[cb],
+                                                                     fw[cb], fvw[cb], fwd[cb], p.seed, p.fm_passes,
+                                                                     lds_cap, trial_where, gscratch, tcut);
+            else
+                k_ip_trials<kWave><<<grid, kWave, lds_bytes, c.stream>>>(act, nact, nodes, total, fx[cb], fadj[cb],
+                                                                         fw[cb], fvw[cb], fwd[cb], p.seed,
+                                                                         p.fm_passes, lds_cap, trial_where, gscratch,
+                                                                         tcut);
+            HGP_LAUNCH_CHECK();
+        }
         k_ip_select<<<nact, 256, 0, c.stream>>>(act, nodes, tcut);
         HGP_LAUNCH_CHECK();
         k_ip_side<<<gv, 256, 0, c.stream>>>(n, node_of[cb], nodes, trial_where, label[cb], where, side);
@@ -887,11 +1698,12 @@ void initial_partition(Ctx &c, const DevGraph &g, int32_t k, const Params &p, in
         HGP_LAUNCH_CHECK();
         scan_inclusive(c, f0, f0, n);
         int nb = cb ^ 1;
-        k_ip_pos<<<gv, 256, 0, c.stream>>>(n, node_of[cb], nodes, side, f0, fx[cb], fadj[cb], pos, node_of[nb],
+        k_ip_pos<<<grid_groups(n, kWave), kRowBS, 0, c.stream>>>(n, node_of[cb], nodes, side, f0, fx[cb], fadj[cb], pos, node_of[nb],
                                            label[nb], label[cb], fvw[nb], fvw[cb], ndeg);
         HGP_LAUNCH_CHECK();
         offsets_from_counts(c, ndeg, fx[nb], n);
-        k_ip_edges<<<gv, 256, 0, c.stream>>>(n, side, pos, fx[cb], fadj[cb], fw[cb], fx[nb], fadj[nb], fw[nb]);
+        k_ip_edges<<<grid_groups(n, kWave), kRowBS, 0, c.stream>>>(n, side, pos, fx[cb], fadj[cb], fw[cb], fx[nb], fadj[nb], fw[nb],
+                                                                    fwd[nb]);
         HGP_LAUNCH_CHECK();
         cb = nb;
     }
