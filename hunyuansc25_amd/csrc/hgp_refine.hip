@@ -8,6 +8,7 @@
 // (part, gain bucket, vertex id) via a stable radix sort, so the result does
 // not depend on scheduling.
 #include "hgp_graph.hpp"
+#include "hgp_jet.hpp"
 #include "hgp_prims.hpp"
 
 #include "hunyuangraph.h"
@@ -23,17 +24,6 @@ namespace {
 constexpr int kBS = 256;
 constexpr int kMaxWaves = 1024 / kWave;   // waves of the largest block here
 constexpr int32_t kNoGain = INT32_MIN;
-
-enum Mode : int32_t { kModeLP = 0, kModeRW = 1, kModeRS = 2 };
-
-struct JetCtl {
-    int64_t cut, best_cut, best_max, maxwgt, opt, maxdest;
-    unsigned long long delta2;      // 2 x cut change (two's complement)
-    int32_t count, balance_counter, mode, done, iters, patience;
-    int32_t ncand, nunder, copy_best, filt_num;   // ncand: 1 if an LP candidate exists
-    int64_t nsorted;                // candidates of RW/RS
-    int64_t nevict;
-};
 
 // Part ids of neighbours are gathered from a narrow copy of where/dest (uint8
 // for k <= 256, else uint16): 1-2 bytes per vertex keep the gathered array
@@ -141,13 +131,6 @@ struct HubConn {
         for (int t = 0; t < T; t++) move(h[t], w[t], pv, dv);
     }
 };
-
-// Writes the (where, dest) word of v.
-__device__ inline void store_pair(uint16_t *p16, uint32_t *p32, int32_t v, int32_t w, int32_t d)
-{
-    if (p16) p16[v] = (uint16_t)((uint32_t)w | ((uint32_t)d << 8));
-    else p32[v] = (uint32_t)w | ((uint32_t)d << 16);
-}
 
 // The afterburner's view of a neighbour: pregain (low 32 bits), where and
 // dest (16 bits each above it), one 8-byte gather per neighbour.
@@ -261,8 +244,6 @@ __device__ inline void jet_next(JetCtl &C, int32_t k, const int64_t *__restrict_
             if (balanced) C.balance_counter = 0; else C.balance_counter++;
             C.ncand = 0;
             C.delta2 = 0;
-            C.nsorted = 0;
-            C.nevict = 0;
         }
     }
     __syncthreads();
@@ -1243,157 +1224,6 @@ __global__ void k_lp_finish(int32_t n, const JetCtl *ctl, const uint8_t *__restr
         dest[v] = w;
     }
     store_pair(pd16, pd32, v, w, d);
-}
-
-// ---------------------------------------------------------------- rebalancers
-
-// After the sort by (key, id): each candidate's weight (scanned next into
-// the prefix weights of its part's candidates) and the first position of
-// each part in the sorted list.
-__global__ void k_rb_weights(int32_t n, int32_t k, const uint32_t *__restrict__ key, const uint32_t *__restrict__ val,
-                             const wgt_t *__restrict__ vwgt, int64_t *__restrict__ w, int32_t *__restrict__ pstart)
-{
-    int32_t i = (int32_t)((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= n) return;
-    const uint32_t kk = key[i];
-    const bool cand = kk < (uint32_t)k * kMaxBuckets;
-    w[i] = cand ? vwgt[val[i]] : 0;
-    if (cand) {
-        uint32_t p = kk / kMaxBuckets;
-        if (i == 0 || key[i - 1] / kMaxBuckets != p) pstart[p] = i;
-    }
-}
-
-// Evict a candidate iff the candidates ahead of it in its part weigh less
-// than the part's excess (filter_scores_below_cutoff :3344-3366 for RW,
-// find_score_cutoffs/filter_below_cutoffs :2641-2691 for RS).  RW keeps the
-// destination chosen in selection; RS only flags the evicted ones.
-__global__ void k_rb_evict(int32_t n, int32_t k, const uint32_t *__restrict__ key, const uint32_t *__restrict__ val,
-                           const int64_t *__restrict__ wsc, const wgt_t *__restrict__ vwgt,
-                           const int32_t *__restrict__ pstart, const int64_t *__restrict__ pwgts, const JetCtl *ctl,
-                           const int32_t *__restrict__ where, int32_t *__restrict__ dest, uint8_t *__restrict__ ev,
-                           uint16_t *__restrict__ pd16, uint32_t *__restrict__ pd32)
-{
-    int32_t i = (int32_t)((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= n) return;
-    uint32_t kk = key[i];
-    int32_t v = (int32_t)val[i];
-    if (kk >= (uint32_t)k * kMaxBuckets) {
-        ev[i] = 0;
-        return;
-    }
-    int32_t p = (int32_t)(kk / kMaxBuckets);
-    int32_t s = pstart[p];
-    int64_t before = wsc[i] - vwgt[v] - (s > 0 ? wsc[s - 1] : 0);
-    bool evict = before < pwgts[p] - ctl->maxwgt;
-    ev[i] = evict ? 1 : 0;
-    if (ctl->mode != kModeRW || !evict) {
-        int32_t w = where[v];
-        dest[v] = w;
-        store_pair(pd16, pd32, v, w, w);
-    }
-}
-
-// Cookie cutter (:2710-2745): slice the evicted list (in sorted order) into
-// consecutive runs, part by part, each filling maxwgt - pwgts.  The parts
-// stay sequential (a slice starts where the last one ended); one wave finds
-// each slice end.  Vertex weights are >= 1, so bs is strictly increasing: a
-// slice of capacity 0 (or an exhausted list) ends where it starts, and the
-// first prefix reaching bs[start] + cap lies within cap entries of start.
-// Over (start, limit], limit = min(ne, start + cap), the serial binary search
-// ends on hi = the first index whose prefix reaches find (limit if none) and
-// lo = hi - 1; the wave finds that hi by 64-way narrowing (each round one
-// load per lane and a ballot), then keeps the nearer of lo and hi.
-__global__ void __launch_bounds__(kWave) k_rs_cookie(int32_t k, const int64_t *__restrict__ bs,
-                                                     const int64_t *__restrict__ ne_ptr,
-                                                     const int64_t *__restrict__ pwgts, const JetCtl *ctl,
-                                                     int32_t *__restrict__ es, int32_t *__restrict__ ee)
-{
-    extern __shared__ int64_t room[];   // maxwgt - pwgts[p], clamped at 0
-    if (blockIdx.x != 0) return;
-    const int lane = lane_id();
-    const int32_t ne = (int32_t)*ne_ptr;
-    const int64_t maxwgt = ctl->maxwgt;
-    for (int32_t p = lane; p < k; p += kWave) room[p] = maxwgt > pwgts[p] ? maxwgt - pwgts[p] : 0;
-    __syncthreads();
-    int32_t start = 0;
-    int64_t bstart = bs[0];   // bs[start], carried from slice to slice
-    for (int32_t p = 0; p < k; p++) {
-        if (start >= ne) {   // the list is used up: every later slice is empty
-            for (int32_t q = p + lane; q < k; q += kWave) es[q] = ee[q] = ne;
-            break;
-        }
-        if (lane == 0) es[p] = start;
-        const int64_t cap = room[p];
-        int32_t end = start;
-        if (cap > 0 && start < ne) {
-            const int64_t find = bstart + cap;
-            const int32_t limit = (int32_t)min((int64_t)ne, (int64_t)start + cap);
-            int32_t L = start + 1, H = limit;   // the answer lies in [L, H]; H stands for "none below H"
-            while (L < H) {
-                const int32_t span = H - L;
-                const int32_t step = span <= kWave ? 1 : (span + kWave - 1) / kWave;
-                const int32_t pos = L + lane * step;
-                const bool ge = pos < H && bs[pos] >= find;
-                const uint64_t m = __ballot(ge);
-                if (step == 1) {   // every index of [L, H) was tested
-                    if (m) H = L + (__ffsll((long long)m) - 1);
-                    break;
-                }
-                if (m == 0) {   // every sample below find: past the last one that lies below H
-                    const int32_t nsamp = (span + step - 1) / step;
-                    L = L + (nsamp - 1) * step + 1;
-                    continue;
-                }
-                const int f = __ffsll((long long)m) - 1;
-                if (f == 0) {
-                    H = L;
-                    break;
-                }
-                H = L + f * step;
-                L = L + (f - 1) * step + 1;
-            }
-            const int32_t hi = H, lo = H - 1;
-            const int64_t bh = bs[hi], bl = bs[lo];
-            int64_t dh = bh - find, dl = bl - find;
-            dh = dh < 0 ? -dh : dh;
-            dl = dl < 0 ? -dl : dl;
-            end = dh < dl ? hi : lo;
-            bstart = dh < dl ? bh : bl;
-        }
-        if (lane == 0) ee[p] = end;
-        start = end;
-    }
-}
-
-// select_dest_parts_rs (:2747-2766) over the compacted evicted list.
-__global__ void k_rs_assign(int32_t k, const int64_t *__restrict__ ne_ptr, const int32_t *__restrict__ elist,
-                            const uint32_t *__restrict__ val, const int32_t *__restrict__ es,
-                            const int32_t *__restrict__ ee, const int32_t *__restrict__ where,
-                            int32_t *__restrict__ dest, uint16_t *__restrict__ pd16, uint32_t *__restrict__ pd32)
-{
-    int32_t i = (int32_t)((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= *ne_ptr) return;
-    int32_t lo = 0, hi = k - 1;
-    while (lo < hi) {
-        int32_t mid = (lo + hi + 1) >> 1;
-        if (es[mid] <= i) lo = mid; else hi = mid - 1;
-    }
-    int32_t v = (int32_t)val[elist[i]];
-    int32_t w = where[v];
-    if (i < ee[lo] && lo != w) {
-        dest[v] = lo;
-        store_pair(pd16, pd32, v, w, lo);
-    }
-}
-
-__global__ void k_gather_w(const int64_t *__restrict__ ne_ptr, const int32_t *__restrict__ elist,
-                           const uint32_t *__restrict__ val, const wgt_t *__restrict__ vwgt, int64_t *__restrict__ bs)
-{
-    int32_t i = (int32_t)((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    int64_t ne = *ne_ptr;
-    if (i == 0) bs[0] = 0;
-    if (i < ne) bs[i + 1] = vwgt[val[elist[i]]];
 }
 
 // ---------------------------------------------------------------- moves
@@ -2484,9 +2314,6 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
     int64_t maxwgt = ((int64_t)p.ub_num * tvwgt) / ((int64_t)p.ub_den * k);
     int64_t *pwgts = c.arena.ralloc<int64_t>((size_t)k);
     int32_t *under = c.arena.ralloc<int32_t>((size_t)k);
-    int32_t *es = c.arena.ralloc<int32_t>((size_t)k);
-    int32_t *ee = c.arena.ralloc<int32_t>((size_t)k);
-    int32_t *pstart = c.arena.ralloc<int32_t>((size_t)k);
     JetCtl *ctl = c.arena.ralloc<JetCtl>(1);
     int32_t *dest = c.arena.ralloc<int32_t>((size_t)n);
     int32_t *pregain = c.arena.ralloc<int32_t>((size_t)n);
@@ -2494,10 +2321,6 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
     uint8_t *lock = c.arena.ralloc<uint8_t>((size_t)n);
     uint8_t *sel = c.arena.ralloc<uint8_t>((size_t)n);
     uint32_t *key = c.arena.ralloc<uint32_t>((size_t)n);
-    uint32_t *val = c.arena.ralloc<uint32_t>((size_t)n);
-    int64_t *wsc = c.arena.ralloc<int64_t>((size_t)n);
-    int32_t *elist = c.arena.ralloc<int32_t>((size_t)n);
-    int64_t *bs = c.arena.ralloc<int64_t>((size_t)n + 1);
     // compact copies for the neighbour gathers: where alone (selection),
     // where and dest in one word (move accounting), pregain, where and dest
     // in 8 bytes (afterburner)
@@ -2515,7 +2338,6 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
         fill<int32_t>(c, conn, (int64_t)g.segs.nmulti * k, 0);
         fill<int64_t>(c, macc, g.segs.nmulti, 0);
     }
-    int64_t *d_ne = c.arena.ralloc<int64_t>(1);
     fill<uint8_t>(c, lock, n, 0);
     HGP_CHECK_HIP(hipMemcpyAsync(best, where, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToDevice, c.stream));
     part_weights(c, n, g.vwgt, where, k, pwgts);
@@ -2549,8 +2371,6 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
     unsigned gv = grid_for(n, kBS);
     if (tiny) {
         // the whole loop in one block
-        uint32_t *k2 = c.arena.ralloc<uint32_t>((size_t)n);
-        uint32_t *v2 = c.arena.ralloc<uint32_t>((size_t)n);
         TinyArgs T;
         T.A = SelArgs{k,    g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, pwgts, lock, under, ctl,
                       dest, pregain, key, nullptr, wq, ab, pd16, pd32};
@@ -2559,20 +2379,20 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
         T.where = where;
         T.under = under;
         T.best = best;
-        T.pstart = pstart;
-        T.elist = elist;
-        T.es = es;
-        T.ee = ee;
+        T.pstart = c.arena.ralloc<int32_t>((size_t)k);
+        T.elist = c.arena.ralloc<int32_t>((size_t)n);
+        T.es = c.arena.ralloc<int32_t>((size_t)k);
+        T.ee = c.arena.ralloc<int32_t>((size_t)k);
         T.sel = sel;
         T.lock = lock;
         T.w8 = w8;
         T.w16 = w16;
-        T.val = val;
-        T.k2 = k2;
-        T.v2 = v2;
+        T.val = c.arena.ralloc<uint32_t>((size_t)n);
+        T.k2 = c.arena.ralloc<uint32_t>((size_t)n);
+        T.v2 = c.arena.ralloc<uint32_t>((size_t)n);
         T.pwgts = pwgts;
-        T.wsc = wsc;
-        T.bs = bs;
+        T.wsc = c.arena.ralloc<int64_t>((size_t)n);
+        T.bs = c.arena.ralloc<int64_t>((size_t)n + 1);
         const size_t lds = tiny_lds(k);
         {
             KScope ks(c, "k_jet_tiny", 0.0);
@@ -2588,6 +2408,9 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
         k_jet_next<<<1, kBS, 0, c.stream>>>(ctl, k, pwgts, under, 1, mirror);
         HGP_LAUNCH_CHECK();
     }
+    const RbView rbv{n, k, key, g.vwgt, where, dest, pd16, pd32, pwgts, ctl};
+    RbScratch rbs{};
+    if (!tiny) rbs = rebalance_scratch(c, n, k);
     // The rest of an iteration once its mode is known: the mode's moves, the
     // move accounting, the commit and the bookkeeping.
     auto issue_rest = [&](int32_t mode, int32_t iters) {
@@ -2640,23 +2463,7 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
             k_lp_finish<<<gv, kBS, 0, c.stream>>>(n, ctl, sel, where, dest, lock, pd16, pd32);
             HGP_LAUNCH_CHECK();
         } else {
-            radix_sort_index(c, key, val, n, 0, bits_for((uint64_t)k * kMaxBuckets));
-            k_rb_weights<<<gv, kBS, 0, c.stream>>>(n, k, key, val, g.vwgt, wsc, pstart);
-            HGP_LAUNCH_CHECK();
-            scan_inclusive(c, wsc, wsc, n);
-            k_rb_evict<<<gv, kBS, 0, c.stream>>>(n, k, key, val, wsc, g.vwgt, pstart, pwgts, ctl, where, dest, sel,
-                                                 pd16, pd32);
-            HGP_LAUNCH_CHECK();
-            if (mode == kModeRS) {
-                compact_indices(c, sel, n, elist, d_ne);
-                k_gather_w<<<gv, kBS, 0, c.stream>>>(d_ne, elist, val, g.vwgt, bs);
-                HGP_LAUNCH_CHECK();
-                scan_inclusive(c, bs + 1, bs + 1, n);
-                k_rs_cookie<<<1, kWave, sizeof(int64_t) * (size_t)k, c.stream>>>(k, bs, d_ne, pwgts, ctl, es, ee);
-                HGP_LAUNCH_CHECK();
-                k_rs_assign<<<gv, kBS, 0, c.stream>>>(k, d_ne, elist, val, es, ee, where, dest, pd16, pd32);
-                HGP_LAUNCH_CHECK();
-            }
+            rebalance(c, rbv, rbs, mode);
         }
         // fixed: ids, where, dest (12 B per row); moved rows add xadj, vwgt and 16 B per entry
         if (int64_t nb = g.bins.few() ? g.bins.short_rows() : 0) {
