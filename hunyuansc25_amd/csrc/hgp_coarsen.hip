@@ -220,19 +220,23 @@ __global__ void k_accept(int32_t n, const int32_t *__restrict__ prop, int32_t *_
     if (__syncthreads_or(got) && threadIdx.x == 0) *progress = 1;   // only "any progress" is read
 }
 
-__global__ void __launch_bounds__(kBS) k_count_matched(int32_t n, const int32_t *__restrict__ match,
-                                                       unsigned long long *cnt)
+// (one atomic a block on one word: few, large blocks)
+constexpr int kCountBS = 1024;
+
+__global__ void __launch_bounds__(kCountBS) k_count_matched(int32_t n, const int32_t *__restrict__ match,
+                                                            unsigned long long *cnt)
 {
-    __shared__ uint32_t part[kBS / kWave];
+    __shared__ uint32_t part[kCountBS / kWave];
     uint32_t c = 0;
-    for (int64_t v = (int64_t)blockIdx.x * kBS + threadIdx.x; v < n; v += (int64_t)gridDim.x * kBS)
+#pragma unroll 4
+    for (int64_t v = (int64_t)blockIdx.x * kCountBS + threadIdx.x; v < n; v += (int64_t)gridDim.x * kCountBS)
         c += match[v] >= 0;
     c = wave_sum(c);
     if (lane_id() == 0) part[threadIdx.x / kWave] = c;
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t t = 0;
-        for (int i = 0; i < kBS / kWave; i++) t += part[i];
+        for (int i = 0; i < kCountBS / kWave; i++) t += part[i];
         if (t) atomicAdd(cnt, (unsigned long long)t);
     }
 }
@@ -1358,8 +1362,8 @@ __global__ void __launch_bounds__(kRowBS) k_seg_compact(const int32_t *__restric
 int64_t count_matched(Ctx &c, int32_t n, const int32_t *match, int64_t *d_cnt)
 {
     fill<int64_t>(c, d_cnt, 1, 0);
-    unsigned blocks = (unsigned)std::min<int64_t>(((int64_t)n + kBS - 1) / kBS, 1024);
-    k_count_matched<<<blocks, kBS, 0, c.stream>>>(n, match, (unsigned long long *)d_cnt);
+    unsigned blocks = (unsigned)std::min<int64_t>(((int64_t)n + 4 * kCountBS - 1) / (4 * kCountBS), 256);
+    k_count_matched<<<blocks, kCountBS, 0, c.stream>>>(n, match, (unsigned long long *)d_cnt);
     HGP_LAUNCH_CHECK();
     read_scalars(c, d_cnt, sizeof(int64_t));
     return c.pinned[0];

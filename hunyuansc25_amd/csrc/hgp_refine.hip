@@ -187,7 +187,7 @@ struct NextScratch {
 
 // Block-wide body (any block of whole waves, up to kMaxWaves): every thread
 // of the block calls it.
-__device__ inline void jet_next(JetCtl &C, int32_t k, const int64_t *__restrict__ pwgts, int32_t *__restrict__ under,
+__device__ inline void jet_next(JetCtl &C, int32_t k, const int64_t *pwgts, int32_t *__restrict__ under,
                                 int32_t first, NextScratch &S)
 {
     const int nw = blockDim.x / kWave;
@@ -249,15 +249,34 @@ __device__ inline void jet_next(JetCtl &C, int32_t k, const int64_t *__restrict_
     __syncthreads();
 }
 
-// mirror (host memory mapped for the device, may be null) receives a copy of
-// the control block for the host to read once the kernel has completed, in
-// place of a copy launch.
-__global__ void __launch_bounds__(kBS) k_jet_next(JetCtl *ctl, int32_t k, const int64_t *__restrict__ pwgts,
-                                                  int32_t *__restrict__ under, int32_t first, JetCtl *mirror)
+// First adds the iteration's move sums to the part weights and the control
+// block.  mirror (host memory mapped for the device, may be null) receives a
+// copy of the control block for the host to read once the kernel has
+// completed, in place of a copy launch.
+constexpr int kNextBS = 512;
+
+__global__ void __launch_bounds__(kNextBS) k_jet_next(JetCtl *ctl, int32_t k, int64_t *pwgts, MoveSums ms,
+                                                      int32_t *__restrict__ under, int32_t first, JetCtl *mirror)
 {
     __shared__ NextScratch S;
     __shared__ int32_t was_done;
     if (threadIdx.x == 0) was_done = ctl->done;
+    if (!first) {   // (nothing was added when the loop has ended)
+        for (int32_t q = threadIdx.x; q <= k; q += kNextBS) {
+            int64_t *const r = ms.rep + q;
+            const int64_t old = q < k ? pwgts[q] : (int64_t)ctl->delta2;
+            int64_t x[8], d = old;
+#pragma unroll
+            for (int i = 0; i < 8; i++) x[i] = i < ms.count ? r[(size_t)i * ms.stride] : 0;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                d += x[i];
+                if (x[i]) r[(size_t)i * ms.stride] = 0;
+            }
+            if (q < k) pwgts[q] = d;
+            else ctl->delta2 = (unsigned long long)d;
+        }
+    }
     __syncthreads();
     if (!was_done) jet_next(*ctl, k, pwgts, under, first, S);
     __syncthreads();
@@ -1250,7 +1269,7 @@ __global__ void __launch_bounds__(kRowBS) k_move_delta_g(const int32_t *__restri
                                                          const wgt_t *__restrict__ vwgt,
                                                          const int32_t *__restrict__ where,
                                                          const int32_t *__restrict__ dest, PairParts pq, HubConn hc,
-                                                         JetCtl *ctl, int64_t *__restrict__ pwgts,
+                                                         const JetCtl *ctl, MoveSums ms,
                                                          unsigned long long *kb)
 {
     extern __shared__ unsigned long long pdelta[];
@@ -1325,9 +1344,10 @@ __global__ void __launch_bounds__(kRowBS) k_move_delta_g(const int32_t *__restri
     }
     kb_flush(kb, kbytes);
     __syncthreads();
+    unsigned long long *const out = ms.mine();
     for (int i = threadIdx.x; i < k; i += kRowBS)
-        if (pdelta[i]) atomicAdd((unsigned long long *)&pwgts[i], pdelta[i]);
-    if (threadIdx.x == 0 && bdelta) atomicAdd(&ctl->delta2, bdelta);
+        if (pdelta[i]) atomicAdd(&out[i], pdelta[i]);
+    if (threadIdx.x == 0 && bdelta) atomicAdd(&out[k], bdelta);
 }
 
 // Rows of 33..512 entries: 64 rows per wave at a time, only the moved ones
@@ -1341,7 +1361,7 @@ __global__ void __launch_bounds__(kRowBS) k_move_delta_w(const int32_t *__restri
                                                          const wgt_t *__restrict__ vwgt,
                                                          const int32_t *__restrict__ where,
                                                          const int32_t *__restrict__ dest, PairParts pq, HubConn hc,
-                                                         JetCtl *ctl, int64_t *__restrict__ pwgts, int32_t rpw,
+                                                         const JetCtl *ctl, MoveSums ms, int32_t rpw,
                                                          unsigned long long *kb)
 {
     extern __shared__ unsigned long long pdelta[];
@@ -1412,9 +1432,10 @@ __global__ void __launch_bounds__(kRowBS) k_move_delta_w(const int32_t *__restri
     if (lane_id() == 0 && d2) atomicAdd(&bdelta, (unsigned long long)d2);
     kb_flush(kb, kbytes);
     __syncthreads();
+    unsigned long long *const out = ms.mine();
     for (int i = threadIdx.x; i < k; i += kRowBS)
-        if (pdelta[i]) atomicAdd((unsigned long long *)&pwgts[i], pdelta[i]);
-    if (threadIdx.x == 0 && bdelta) atomicAdd(&ctl->delta2, bdelta);
+        if (pdelta[i]) atomicAdd(&out[i], pdelta[i]);
+    if (threadIdx.x == 0 && bdelta) atomicAdd(&out[k], bdelta);
 }
 
 // Long rows by segments; the part weights move with the row's first segment.
@@ -1425,7 +1446,7 @@ __global__ void __launch_bounds__(kSegBlk) k_move_delta_seg(RowSegs S, int32_t k
                                                            const wgt_t *__restrict__ vwgt,
                                                            const int32_t *__restrict__ where,
                                                            const int32_t *__restrict__ dest, PairParts pq, HubConn hc,
-                                                           JetCtl *ctl, int64_t *__restrict__ pwgts,
+                                                           const JetCtl *ctl, MoveSums ms,
                                                            unsigned long long *kb)
 {
     extern __shared__ unsigned long long pdelta[];
@@ -1463,9 +1484,10 @@ __global__ void __launch_bounds__(kSegBlk) k_move_delta_seg(RowSegs S, int32_t k
     if (threadIdx.x == 0 && d2) atomicAdd(&bdelta, (unsigned long long)d2);
     kb_flush(kb, kbytes);
     __syncthreads();
+    unsigned long long *const out = ms.mine();
     for (int i = threadIdx.x; i < k; i += kSegBlk)
-        if (pdelta[i]) atomicAdd((unsigned long long *)&pwgts[i], pdelta[i]);
-    if (threadIdx.x == 0 && bdelta) atomicAdd(&ctl->delta2, bdelta);
+        if (pdelta[i]) atomicAdd(&out[i], pdelta[i]);
+    if (threadIdx.x == 0 && bdelta) atomicAdd(&out[k], bdelta);
 }
 
 // Applies dest and refreshes the narrow copy of where.  First, when the
@@ -1580,17 +1602,20 @@ inline unsigned seg_grid(const RowSegs &S) { return (unsigned)std::min<int64_t>(
 __global__ void k_half(int64_t *d) { *d /= 2; }
 
 // Persistent blocks sum their vertices' weights per part in LDS and flush one
-// atomic per block and touched part.
-__global__ void __launch_bounds__(kBS) k_pwgts(int32_t n, int32_t k, const wgt_t *__restrict__ vwgt,
+// atomic per block and touched part: few and large blocks, since the flushes
+// of the blocks into one line wait for each other (22 ns a block).
+constexpr int kPwBS = 1024;
+
+__global__ void __launch_bounds__(kPwBS) k_pwgts(int32_t n, int32_t k, const wgt_t *__restrict__ vwgt,
                                                const int32_t *__restrict__ where, unsigned long long *pw)
 {
     extern __shared__ unsigned long long hist[];
-    for (int i = threadIdx.x; i < k; i += kBS) hist[i] = 0;
+    for (int i = threadIdx.x; i < k; i += kPwBS) hist[i] = 0;
     __syncthreads();
-    for (int64_t v = (int64_t)blockIdx.x * kBS + threadIdx.x; v < n; v += (int64_t)gridDim.x * kBS)
+    for (int64_t v = (int64_t)blockIdx.x * kPwBS + threadIdx.x; v < n; v += (int64_t)gridDim.x * kPwBS)
         atomicAdd(&hist[where[v]], (unsigned long long)(int64_t)vwgt[v]);
     __syncthreads();
-    for (int i = threadIdx.x; i < k; i += kBS)
+    for (int i = threadIdx.x; i < k; i += kPwBS)
         if (hist[i]) atomicAdd(&pw[i], hist[i]);
 }
 
@@ -1737,8 +1762,8 @@ void part_weights(Ctx &c, int32_t n, const wgt_t *vwgt, const int32_t *where, in
 {
     fill<int64_t>(c, pwgts, k, 0);
     if (n <= 0) return;
-    unsigned blocks = (unsigned)std::min<int64_t>(((int64_t)n + kBS - 1) / kBS, 1024);
-    k_pwgts<<<blocks, kBS, sizeof(unsigned long long) * (size_t)k, c.stream>>>(n, k, vwgt, where,
+    unsigned blocks = (unsigned)std::min<int64_t>(((int64_t)n + 4 * kPwBS - 1) / (4 * kPwBS), 256);
+    k_pwgts<<<blocks, kPwBS, sizeof(unsigned long long) * (size_t)k, c.stream>>>(n, k, vwgt, where,
                                                                               (unsigned long long *)pwgts);
     HGP_LAUNCH_CHECK();
 }
@@ -2401,11 +2426,23 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
         }
         read_scalars(c, ctl, sizeof(JetCtl));
     }
+    MoveSums ms;
+    if (!tiny) {
+        // One copy while few blocks flush (a block takes at least 256 rows or a
+        // segment), up to 8: k_jet_next reads them in one go (32 copies cost it
+        // 1.3 us more an iteration than they saved).
+        const int64_t blocks = std::min<int64_t>(4096, (int64_t)n / 256 + g.segs.nseg);
+        ms.count = 1;
+        while (ms.count < 8 && ms.count * 128 < blocks) ms.count *= 2;
+        ms.stride = (k + 1 + 15) / 16 * 16;
+        ms.rep = c.arena.ralloc<int64_t>((size_t)ms.count * (size_t)ms.stride);
+        fill<int64_t>(c, ms.rep, (int64_t)ms.count * ms.stride, 0);
+    }
     // k_jet_next leaves a copy of the control block in the pinned buffer
     JetCtl *mirror = nullptr;
     if (!tiny) HGP_CHECK_HIP(hipHostGetDevicePointer((void **)&mirror, c.pinned, 0));
     if (!tiny) {
-        k_jet_next<<<1, kBS, 0, c.stream>>>(ctl, k, pwgts, under, 1, mirror);
+        k_jet_next<<<1, kNextBS, 0, c.stream>>>(ctl, k, pwgts, ms, under, 1, mirror);
         HGP_LAUNCH_CHECK();
     }
     const RbView rbv{n, k, key, g.vwgt, where, dest, pd16, pd32, pwgts, ctl};
@@ -2470,7 +2507,7 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
             KScope ks(c, "k_move_delta_few", 12.0 * (double)nb, true);
             int32_t rpw = rows_per_wave(nb);
             k_move_delta_w<<<wave_blocks(nb, rpw, 2048), kRowBS, sizeof(unsigned long long) * (size_t)k, c.stream>>>(
-                g.bins.list(0), nb, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, pwgts, rpw,
+                g.bins.list(0), nb, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, ms, rpw,
                 ks.dev());
             HGP_LAUNCH_CHECK();
         }
@@ -2478,21 +2515,21 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
             KScope ks(c, "k_move_delta_s", 12.0 * (double)nb, true);
             int64_t blocks = std::min<int64_t>((nb + kRowBS - 1) / kRowBS, 2048);
             k_move_delta_g<8><<<(unsigned)blocks, kRowBS, sizeof(unsigned long long) * (size_t)k, c.stream>>>(
-                g.bins.list(0), nb, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, pwgts, ks.dev());
+                g.bins.list(0), nb, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, ms, ks.dev());
             HGP_LAUNCH_CHECK();
         }
         if (int64_t nb = g.bins.few() ? 0 : g.bins.count(1)) {
             KScope ks(c, "k_move_delta_m", 12.0 * (double)nb, true);
             int64_t blocks = std::min<int64_t>((nb + kRowBS - 1) / kRowBS, 2048);
             k_move_delta_g<32><<<(unsigned)blocks, kRowBS, sizeof(unsigned long long) * (size_t)k, c.stream>>>(
-                g.bins.list(1), nb, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, pwgts, ks.dev());
+                g.bins.list(1), nb, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, ms, ks.dev());
             HGP_LAUNCH_CHECK();
         }
         if (int64_t nb = g.bins.few() ? 0 : g.bins.count(2)) {
             KScope ks(c, "k_move_delta_w", 12.0 * (double)nb, true);
             int32_t rpw = rows_per_wave(nb);
             k_move_delta_w<<<wave_blocks(nb, rpw, 2048), kRowBS, sizeof(unsigned long long) * (size_t)k, c.stream>>>(
-                g.bins.list(2), nb, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, pwgts, rpw,
+                g.bins.list(2), nb, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, ms, rpw,
                 ks.dev());
             HGP_LAUNCH_CHECK();
         }
@@ -2500,7 +2537,7 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
             KScope ks(c, "k_move_delta_seg", 24.0 * (double)g.segs.nseg, true);
             unsigned blocks = (unsigned)std::min<int64_t>(g.segs.nseg, 4096);
             k_move_delta_seg<<<blocks, kSegBlk, sizeof(unsigned long long) * (size_t)k, c.stream>>>(
-                g.segs, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, pwgts, ks.dev());
+                g.segs, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, ms, ks.dev());
             HGP_LAUNCH_CHECK();
         }
         {
@@ -2518,7 +2555,7 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
         }
         k_move_commit<<<gv, kBS, 0, c.stream>>>(n, ctl, dest, where, w8, w16, best);
         HGP_LAUNCH_CHECK();
-        k_jet_next<<<1, kBS, 0, c.stream>>>(ctl, k, pwgts, under, 0, mirror);
+        k_jet_next<<<1, kNextBS, 0, c.stream>>>(ctl, k, pwgts, ms, under, 0, mirror);
         HGP_LAUNCH_CHECK();
     };
     auto issue_select = [&] {
