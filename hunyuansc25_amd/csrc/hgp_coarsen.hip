@@ -123,6 +123,58 @@ __global__ void __launch_bounds__(kRowBS) k_propose(const int32_t *__restrict__ 
     kb_flush(kb, kbytes);
 }
 
+// Rows of <= 8 entries: a lane per row, the row in its registers, so a wave's 64
+// rows share one chain of loads (8 lanes per row: 95 us for the first round of
+// a 1.5M-vertex mesh).
+__global__ void __launch_bounds__(kRowBS) k_propose_t(const int32_t *__restrict__ ids, int64_t cnt,
+                                                      const eid_t *__restrict__ xadj,
+                                                      const vid_t *__restrict__ adjncy,
+                                                      const wgt_t *__restrict__ adjwgt,
+                                                      const int32_t *__restrict__ avail, int32_t maxvwgt,
+                                                      uint64_t s1, int32_t *__restrict__ prop,
+                                                      const int32_t *prev_progress, int32_t first,
+                                                      unsigned long long *kb)
+{
+    constexpr int T = (int)kBinSmall;
+    const int64_t i = (int64_t)blockIdx.x * kRowBS + threadIdx.x;
+    const int32_t v = i < cnt ? ids[i] : -1;
+    const int32_t wv = v >= 0 ? avail[v] : -1;
+    if (prev_progress && *prev_progress == 0) return;
+    uint64_t kbytes = 0;
+    if (v >= 0) {
+        if (wv < 0) {
+            prop[v] = -1;
+        } else if (!keeps_proposal(first, v, avail, prop)) {
+            const eid_t b = xadj[v];
+            const int32_t d = (int32_t)(xadj[v + 1] - b);
+            const uint64_t tv = mix64(s1 ^ (uint64_t)(uint32_t)v);
+            int32_t u[T], w[T], wu[T];
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                u[t] = -1;
+                w[t] = 0;
+                if (t < d) {
+                    u[t] = adjncy[b + t];
+                    w[t] = adjwgt[b + t];
+                }
+            }
+            gather_slots<T>(avail, u, wu, -1);
+            EdgeKey best{-1, 0, 0, 0u};
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                if (u[t] < 0 || u[t] == v || wu[t] < 0) continue;
+                if ((int64_t)wu[t] + wv >= maxvwgt) continue;
+                EdgeKey e{w[t], u[t] < v ? u[t] : v, u[t] < v ? v : u[t], 0u};
+                e.h = edge_hash_row(s1, tv, v, u[t]);
+                if (BetterEdge()(e, best)) best = e;
+            }
+            prop[v] = best.w < 0 ? -1 : (best.lo == v ? best.hi : best.lo);
+            kbytes = 16 + 12 * (uint64_t)d;
+        }
+    }
+    kb_flush(kb, kbytes);
+}
+
 // Class-2 rows by segments (a hub row is shared by several blocks): the
 // segment of a single-segment row writes the proposal; the segments of a
 // multi row leave their best edge in sbest for k_propose_fin.
@@ -1443,7 +1495,7 @@ int64_t match_level(Ctx &c, const DevGraph &g, int32_t maxvwgt, uint64_t seed, i
                 KScope ks(c, names[cl], 12.0 * (double)cnt, true);
                 const int32_t *ids = g.bins.list(cl);
                 if (cl == 0)
-                    k_propose<8><<<grid_groups(cnt, 8), kRowBS, 0, c.stream>>>(ids, cnt, g.xadj, g.adjncy, g.adjwgt,
+                    k_propose_t<<<grid_groups(cnt, 1), kRowBS, 0, c.stream>>>(ids, cnt, g.xadj, g.adjncy, g.adjwgt,
                                                                                avail, maxvwgt, s1, prop, prev,
                                                                                r == 0, ks.dev());
                 else if (cl == 1)

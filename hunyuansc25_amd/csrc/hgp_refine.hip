@@ -466,94 +466,88 @@ __device__ inline void load_targets(const SelArgs &A, int32_t mode, int64_t maxw
     __syncthreads();
 }
 
-// Rows of <= G entries (G = 8): each wave screens 64 rows (one per lane),
-// settles the ineligible ones lane by lane, then takes the eligible ones 64/G
-// at a time, G lanes and one entry per lane each.  The entry loads of all
-// passes are issued before the first pass is reduced.  A lane's connectivity
-// to its entry's part is summed over the group with shuffles (no LDS).
-template <int G>
-__global__ void __launch_bounds__(kRowBS) k_jet_select_g(const int32_t *__restrict__ ids, int64_t cnt, SelArgs A)
+// Rows of <= 8 entries (class s): a lane per row, the row's entries in its
+// registers and the sums per part by comparing them pairwise, so a wave's 64
+// rows share one chain of loads and nothing is exchanged between lanes.  The
+// part weights come from LDS, and a chunk's ids and parts are on their way
+// before the control block has arrived.  (8 lanes per row with shuffles, eight
+// passes a wave: 12 us at 65k rows and 80 us at 1.5M.)
+constexpr int kRowT = (int)kBinSmall;
+
+__global__ void __launch_bounds__(kRowBS) k_jet_select_t(const int32_t *__restrict__ ids, int64_t cnt, SelArgs A)
 {
-    extern __shared__ uint8_t tg[];     // k part flags
-    __shared__ int32_t slots[kRowBS];   // per wave: lanes holding eligible rows, in rank order
+    extern __shared__ int64_t pw[];   // k part weights, then k part flags
     const JetCtl &C = *A.ctl;
+    int64_t i = (int64_t)blockIdx.x * kRowBS + threadIdx.x;
+    int32_t v = i < cnt ? ids[i] : -1;
+    SelRow r;
+    if (v >= 0) r.p = A.where[v];
     if (C.done) return;
     const int32_t mode = C.mode;
     const int64_t maxwgt = C.maxwgt, opt = C.opt;
-    load_targets(A, mode, maxwgt, tg);
-    constexpr int RP = kWave / G;   // rows per pass
-    constexpr int NP = kWave / RP;  // passes that cover 64 rows
-    static_assert(NP <= 8, "the passes' entries are held in registers at once");
-    const int lane = lane_id(), grp = lane / G, gl = lane % G;
-    int32_t *sl = slots + (threadIdx.x / kWave) * kWave;
-    const int64_t wid = ((int64_t)blockIdx.x * kRowBS + threadIdx.x) / kWave;
-    const int64_t nwaves = ((int64_t)gridDim.x * kRowBS) / kWave;
+    uint8_t *tg = (uint8_t *)(pw + A.k);
+    for (int q = threadIdx.x; q < A.k; q += kRowBS) {
+        const int64_t x = A.pwgts[q];
+        pw[q] = x;
+        tg[q] = mode == kModeLP || (mode == kModeRW && x < maxwgt) ? 1 : 0;   // sel_target
+    }
+    __syncthreads();
     int32_t ncand = 0;
     uint64_t kbytes = 0;
-    for (int64_t base = wid * kWave; base < cnt; base += nwaves * kWave) {
-        // one row per lane: screen, settle the ineligible ones, fetch the bounds of the others
-        int64_t i = base + lane;
-        int32_t mv = i < cnt ? ids[i] : -1;
-        SelRow mr;
-        if (mv >= 0) mr = sel_row(A, mode, mv);
-        bool mel = mv >= 0 && sel_eligible(mode, maxwgt, opt, mr);
-        if (mv >= 0 && !mel) sel_decide(A, C, mode, mv, mr, false, 0, PartKey{0, -1});
-        eid_t mb = 0, me = 0;
-        if (mel) {
-            mb = A.xadj[mv];
-            me = A.xadj[mv + 1];
+    for (;;) {
+        bool el = false;
+        if (v >= 0) {
+            if (mode == kModeLP) {
+                r.lk = A.lock[v];
+                el = true;
+            } else {
+                r.pwp = pw[r.p];
+                if (r.pwp > maxwgt) {
+                    r.vw = A.vwgt[v];
+                    el = sel_eligible(mode, maxwgt, opt, r);
+                }
+            }
         }
-        uint64_t bal = __ballot(mel);
-        const int ne = __popcll(bal);
-        if (mel) sl[__popcll(bal & lanemask_lt())] = lane;
-        wave_lds_sync();
-        const int np = (ne + RP - 1) / RP;
-        int32_t src[NP], rl[NP], u[NP], w[NP], q[NP];
+        int32_t u[kRowT], w[kRowT], q[kRowT];
+        const eid_t b = el ? A.xadj[v] : 0;
+        const int32_t d = el ? (int32_t)(A.xadj[v + 1] - b) : 0;
 #pragma unroll
-        for (int t = 0; t < NP; t++) {
+        for (int t = 0; t < kRowT; t++) {
             u[t] = -1;
             w[t] = 0;
-            src[t] = -1;
-            rl[t] = 0;
-            if (t < np) {   // wave-uniform
-                int r = t * RP + grp;
-                int s = r < ne ? sl[r] : 0;
-                eid_t b = __shfl(mb, s, kWave), e = __shfl(me, s, kWave);
-                if (r < ne) {
-                    src[t] = s;
-                    rl[t] = (int32_t)(e - b);
-                }
-                if (r < ne && b + gl < e) {
-                    u[t] = A.adjncy[b + gl];
-                    w[t] = A.adjwgt[b + gl];
-                }
+            if (t < d) {
+                u[t] = A.adjncy[b + t];
+                w[t] = A.adjwgt[b + t];
             }
         }
         A.wq.gather(u, q);
+        // the next chunk's rows, loaded while this one is decided
+        const int32_t cv = v;
+        const SelRow cr = r;
+        i += (int64_t)gridDim.x * kRowBS;
+        v = i < cnt ? ids[i] : -1;
+        if (cv >= 0) {
+            int32_t pc = 0;
+            PartKey best{0, -1};
 #pragma unroll
-        for (int t = 0; t < NP; t++) {
-            if (t < np) {
-                int s = src[t] >= 0 ? src[t] : 0;
-                int32_t v = __shfl(mv, s, kWave);
-                const SelRow rr = shfl_row(mr, s);
-                const int32_t p = rr.p;
-                int32_t conn = w[t];
+            for (int t = 0; t < kRowT; t++) pc += q[t] == cr.p ? w[t] : 0;
+            if (mode != kModeRS) {
 #pragma unroll
-                for (int o = 1; o < G; o++) {
-                    int32_t qq = __shfl_xor(q[t], o, G), ww = __shfl_xor(w[t], o, G);
-                    if (qq == q[t]) conn += ww;
-                }
-                int32_t pc = group_sum<G>(q[t] == p ? w[t] : 0);
-                PartKey best{0, -1};
-                if (q[t] >= 0 && q[t] != p && tg[q[t]]) best = PartKey{conn, q[t]};
-                best = group_best<G>(best, BetterPart());
-                if (src[t] >= 0 && gl == 0) {
-                    ncand += sel_decide(A, C, mode, v, rr, true, pc, best);
-                    kbytes += 16 + 12 * (uint64_t)rl[t];
+                for (int t = 0; t < kRowT; t++) {
+                    int32_t c = 0;
+#pragma unroll
+                    for (int x = 0; x < kRowT; x++) c += q[x] == q[t] ? w[x] : 0;
+                    const bool ok = q[t] >= 0 && q[t] != cr.p && tg[q[t] >= 0 ? q[t] : 0];
+                    const bool better = ok && (c > best.c || (c == best.c && c > 0 && q[t] < best.q));
+                    best.c = better ? c : best.c;
+                    best.q = better ? q[t] : best.q;
                 }
             }
+            ncand += sel_decide(A, C, mode, cv, cr, el, pc, best);
+            if (el) kbytes += 16 + 12 * (uint64_t)d;
         }
-        wave_lds_sync();
+        if ((int64_t)(i - threadIdx.x) >= cnt) break;   // the same for the whole block
+        if (v >= 0) r.p = A.where[v];
     }
     sel_count(A, mode, ncand);
     kb_flush(A.kb, kbytes);
@@ -1072,6 +1066,53 @@ __global__ void __launch_bounds__(kRowBS) k_afterburner(const int32_t *__restric
     kb_flush(kb, kbytes);
 }
 
+// Rows of <= 8 entries: a lane per row (see k_jet_select_t).
+__global__ void __launch_bounds__(kRowBS) k_afterburner_t(const int32_t *__restrict__ ids, int64_t cnt,
+                                                          const eid_t *__restrict__ xadj,
+                                                          const vid_t *__restrict__ adjncy,
+                                                          const wgt_t *__restrict__ adjwgt,
+                                                          const int32_t *__restrict__ where,
+                                                          const int32_t *__restrict__ dest,
+                                                          const uint64_t *__restrict__ ab,
+                                                          const int32_t *__restrict__ pregain, const JetCtl *ctl,
+                                                          uint8_t *__restrict__ sel, unsigned long long *kb)
+{
+    const int64_t i = (int64_t)blockIdx.x * kRowBS + threadIdx.x;
+    const int32_t v = i < cnt ? ids[i] : -1;
+    const int32_t ig = v >= 0 ? pregain[v] : kNoGain;
+    if (ctl->done || ctl->mode != kModeLP) return;
+    uint64_t kbytes = 0;
+    if (v >= 0) {
+        bool keep = false;
+        if (ig != kNoGain) {
+            const int32_t p = where[v], best = dest[v];
+            const eid_t b = xadj[v];
+            const int32_t d = (int32_t)(xadj[v + 1] - b);
+            int32_t u[kRowT], w[kRowT];
+            uint64_t x[kRowT];
+#pragma unroll
+            for (int t = 0; t < kRowT; t++) {
+                u[t] = -1;
+                w[t] = 0;
+                if (t < d) {
+                    u[t] = adjncy[b + t];
+                    w[t] = adjwgt[b + t];
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < kRowT; t++) x[t] = u[t] >= 0 ? ab[u[t]] : 0ull;
+            int64_t change = 0;
+#pragma unroll
+            for (int t = 0; t < kRowT; t++)
+                if (u[t] >= 0) change += ab_change(v, ig, p, best, u[t], w[t], x[t]);
+            keep = (int64_t)ig + change >= 0;
+            kbytes = 24 + 16 * (uint64_t)d;
+        }
+        sel[v] = keep ? 1 : 0;
+    }
+    kb_flush(kb, kbytes);
+}
+
 // Rows of 33..512 entries: 64 rows per wave at a time; non-candidates are
 // settled lane by lane, candidates of <= kQuarterRow entries four at a time
 // (a 16-lane quarter and 8 entries per lane each), longer ones one row at a
@@ -1251,9 +1292,9 @@ __global__ void k_lp_finish(int32_t n, const JetCtl *ctl, const uint8_t *__restr
 // applying dest[] (edges between two moved vertices are seen from both ends,
 // so each side counts once and one-sided edges twice) and the part-weight
 // updates.  Both are summed in LDS and flushed with one atomic per block and
-// touched part.  Rows of <= G entries (G = 8 or 32): each wave screens 64
-// rows, then walks the moved ones 64/G at a time (G lanes, one entry per lane
-// each), the entry loads of all passes issued before the first is used.
+// touched part.  Rows of 9..G entries (G = 32): each wave screens 64 rows, then
+// walks the moved ones 64/G at a time (G lanes, one entry per lane each), the
+// entry loads of all passes issued before the first is used.
 __device__ inline int64_t move_d2(int32_t pv, int32_t dv, int32_t pu, int32_t du, int32_t w)
 {
     bool um = pu != du;
@@ -1347,6 +1388,71 @@ __global__ void __launch_bounds__(kRowBS) k_move_delta_g(const int32_t *__restri
     unsigned long long *const out = ms.mine();
     for (int i = threadIdx.x; i < k; i += kRowBS)
         if (pdelta[i]) atomicAdd(&out[i], pdelta[i]);
+    if (threadIdx.x == 0 && bdelta) atomicAdd(&out[k], bdelta);
+}
+
+// Rows of <= 8 entries: a lane per row (see k_jet_select_t).
+__global__ void __launch_bounds__(kRowBS) k_move_delta_t(const int32_t *__restrict__ ids, int64_t cnt, int32_t k,
+                                                         const eid_t *__restrict__ xadj,
+                                                         const vid_t *__restrict__ adjncy,
+                                                         const wgt_t *__restrict__ adjwgt,
+                                                         const wgt_t *__restrict__ vwgt,
+                                                         const int32_t *__restrict__ where,
+                                                         const int32_t *__restrict__ dest, PairParts pq, HubConn hc,
+                                                         const JetCtl *ctl, MoveSums ms, unsigned long long *kb)
+{
+    extern __shared__ unsigned long long pdelta[];
+    __shared__ unsigned long long bdelta;
+    int64_t i = (int64_t)blockIdx.x * kRowBS + threadIdx.x;
+    int32_t v = i < cnt ? ids[i] : -1, pv = 0, dv = 0;
+    if (v >= 0) {
+        pv = where[v];
+        dv = dest[v];
+    }
+    if (ctl->done) return;
+    for (int q = threadIdx.x; q < k; q += kRowBS) pdelta[q] = 0;
+    if (threadIdx.x == 0) bdelta = 0;
+    __syncthreads();
+    uint64_t kbytes = 0;
+    int64_t d2 = 0;
+    while (v >= 0) {
+        if (pv != dv) {
+            const eid_t b = xadj[v];
+            const int32_t d = (int32_t)(xadj[v + 1] - b);
+            const int64_t wv = vwgt[v];
+            int32_t u[kRowT], w[kRowT], pu[kRowT], du[kRowT];
+#pragma unroll
+            for (int t = 0; t < kRowT; t++) {
+                u[t] = -1;
+                w[t] = 0;
+                if (t < d) {
+                    u[t] = adjncy[b + t];
+                    w[t] = adjwgt[b + t];
+                }
+            }
+            pq.gather(u, pu, du);
+            atomicAdd(&pdelta[pv], (unsigned long long)(-wv));
+            atomicAdd(&pdelta[dv], (unsigned long long)wv);
+#pragma unroll
+            for (int t = 0; t < kRowT; t++)
+                if (u[t] >= 0) d2 += move_d2(pv, dv, pu[t], du[t], w[t]);
+            hc.moved<kRowT>(u, w, pv, dv);
+            kbytes += 20 + 16 * (uint64_t)d;
+        }
+        i += (int64_t)gridDim.x * kRowBS;
+        v = i < cnt ? ids[i] : -1;
+        if (v >= 0) {
+            pv = where[v];
+            dv = dest[v];
+        }
+    }
+    d2 = wave_sum(d2);
+    if (lane_id() == 0 && d2) atomicAdd(&bdelta, (unsigned long long)d2);
+    kb_flush(kb, kbytes);
+    __syncthreads();
+    unsigned long long *const out = ms.mine();
+    for (int q = threadIdx.x; q < k; q += kRowBS)
+        if (pdelta[q]) atomicAdd(&out[q], pdelta[q]);
     if (threadIdx.x == 0 && bdelta) atomicAdd(&out[k], bdelta);
 }
 
@@ -1679,8 +1785,11 @@ void launch_select(Ctx &c, const DevGraph &g, int32_t k, const int32_t *where, c
     if (b.count(0) && !b.few()) {
         KScope ks(c, "k_jet_select_s", 24.0 * (double)b.count(0), true);
         A.kb = ks.dev();
-        unsigned blocks = (unsigned)std::min<int64_t>((b.count(0) + kRowBS - 1) / kRowBS, 16384);
-        k_jet_select_g<8><<<blocks, kRowBS, tg_bytes, c.stream>>>(b.list(0), b.count(0), A);
+        // one chunk a block until the chip is full, then as many as a block's part
+        // weights are worth (k reads against 256 rows)
+        unsigned blocks = (unsigned)std::min<int64_t>((b.count(0) + kRowBS - 1) / kRowBS, k <= 256 ? 4096 : 2048);
+        k_jet_select_t<<<blocks, kRowBS, sizeof(int64_t) * (size_t)k + tg_bytes, c.stream>>>(b.list(0), b.count(0),
+                                                                                            A);
         HGP_LAUNCH_CHECK();
     }
     // class m: 16-lane groups while k is small enough for their LDS rows;
@@ -2464,7 +2573,7 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
                 }
                 if (int64_t nb = g.bins.few() ? 0 : g.bins.count(0)) {
                     KScope ks(c, "k_afterburner_s", 9.0 * (double)nb, true);
-                    k_afterburner<8><<<grid_groups(nb, 8), kRowBS, 0, c.stream>>>(
+                    k_afterburner_t<<<grid_groups(nb, 1), kRowBS, 0, c.stream>>>(
                         g.bins.list(0), nb, g.xadj, g.adjncy, g.adjwgt, where, dest, ab, pregain, ctl, sel, ks.dev());
                     HGP_LAUNCH_CHECK();
                 }
@@ -2514,7 +2623,7 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
         if (int64_t nb = g.bins.few() ? 0 : g.bins.count(0)) {
             KScope ks(c, "k_move_delta_s", 12.0 * (double)nb, true);
             int64_t blocks = std::min<int64_t>((nb + kRowBS - 1) / kRowBS, 2048);
-            k_move_delta_g<8><<<(unsigned)blocks, kRowBS, sizeof(unsigned long long) * (size_t)k, c.stream>>>(
+            k_move_delta_t<<<(unsigned)blocks, kRowBS, sizeof(unsigned long long) * (size_t)k, c.stream>>>(
                 g.bins.list(0), nb, k, g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, dest, pq, hc, ctl, ms, ks.dev());
             HGP_LAUNCH_CHECK();
         }
