@@ -440,16 +440,6 @@ __device__ inline int32_t sel_decide(const SelArgs &A, const JetCtl &C, int32_t 
     return o.cand;
 }
 
-__device__ inline SelRow shfl_row(const SelRow &r, int src)
-{
-    SelRow o;
-    o.p = __shfl(r.p, src, kWave);
-    o.vw = __shfl(r.vw, src, kWave);
-    o.lk = __shfl(r.lk, src, kWave);
-    o.pwp = __shfl(r.pwp, src, kWave);
-    return o;
-}
-
 // LP only needs to know whether any candidate exists: one store per block
 // that has some (every thread of the block calls this).
 __device__ inline void sel_count(const SelArgs &A, int32_t mode, int32_t ncand)
@@ -553,78 +543,138 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_t(const int32_t *__restri
     kb_flush(A.kb, kbytes);
 }
 
-// Rows of 9..32 entries (class m): 16-lane groups, four rows per wave at a
-// time, each group with its own k-int LDS row.  The groups of a wave run in
-// lockstep, so a wave-level fence orders each group's accumulation, reads
-// and clearing.  Used when k <= kQuarterK.
+// Rows of 9..32 entries (class m), used when k <= kQuarterK: 16-lane groups,
+// four rows per wave at a time, each group with its own k-int LDS row.  A wave
+// screens 64 rows (one per lane) and takes the eligible ones four at a time with
+// the entry loads of kMidPasses passes out before the first is used, so 64
+// rows share a few memory round trips; what is left per pass is a short chain
+// through LDS.  Each row's result goes back to its lane through LDS, and the 64
+// lanes decide at once.  (A group that fetched its rows one by one, a chain of
+// five round trips each: 163 us for 1M rows of a 3-D RGG.)
+// The groups of a wave run in lockstep, so a wave-level fence orders each
+// group's accumulation, reads and clearing.
 constexpr int kQuarterG = 16;
 constexpr int32_t kQuarterK = 512;
+constexpr int kMidPasses = 8;
 // The long rows (> 512 entries) keep connectivity rows while k is at most
 // this: a k-int row is then at most the size of the shortest long row's
 // entries, and the selection reads it instead of the row.
 constexpr int32_t kTrackMaxK = 512;
 
-__global__ void __launch_bounds__(kRowBS) k_jet_select_q(const int32_t *__restrict__ ids, int64_t cnt, SelArgs A)
+// LDS of k_jet_select_m: a k-int row per group, rows an odd number of banks
+// apart, and the part flags.
+inline size_t sel_m_lds(int32_t k) { return sizeof(int32_t) * (kRowBS / kQuarterG) * (size_t)(k | 1); }
+
+__global__ void __launch_bounds__(kRowBS) k_jet_select_m(const int32_t *__restrict__ ids, int64_t cnt, int32_t rpw,
+                                                         SelArgs A)
 {
-    extern __shared__ int32_t acc[];   // k ints per group, then k part flags
-    constexpr int G = kQuarterG, NG = kRowBS / G, E = (int)(kBinHalf / G);
+    extern __shared__ int32_t acc[];
+    constexpr int G = kQuarterG, NG = kRowBS / G, NQ = kWave / G, E = (int)(kBinHalf / G), NP = kMidPasses;
+    __shared__ int32_t slots[kRowBS];   // per wave: lanes holding eligible rows, in rank order
+    __shared__ int3 results[kRowBS];    // per row: connectivity to the own part, best other part
     const JetCtl &C = *A.ctl;
+    const int lane = lane_id(), wv = threadIdx.x / kWave, grp = lane / G, gl = lane % G;
+    const int64_t nwaves = (int64_t)gridDim.x * (kRowBS / kWave);
+    int64_t base = ((int64_t)blockIdx.x * (kRowBS / kWave) + wv) * rpw;
+    int32_t nv = lane < rpw && base + lane < cnt ? ids[base + lane] : -1;
     if (C.done) return;
     const int32_t mode = C.mode;
     const int64_t maxwgt = C.maxwgt, opt = C.opt;
-    const int k = A.k, gid = threadIdx.x / G, gl = threadIdx.x % G;
-    int32_t *my = acc + (size_t)gid * k;
-    uint8_t *tg = (uint8_t *)(acc + (size_t)NG * k);
+    const int k = A.k, stride = k | 1;
+    int32_t *my = acc + (size_t)(wv * NQ + grp) * stride;
+    uint8_t *tg = (uint8_t *)(acc + (size_t)NG * stride);
+    int32_t *sl = slots + wv * kWave;
+    int3 *res = results + wv * kWave;
     for (int i = gl; i < k; i += G) my[i] = 0;
     load_targets(A, mode, maxwgt, tg);
     int32_t ncand = 0;
     uint64_t kbytes = 0;
-    for (int64_t row = (int64_t)blockIdx.x * NG + gid; row < cnt; row += (int64_t)gridDim.x * NG) {
-        const int32_t v = ids[row];
-        const SelRow r = sel_row(A, mode, v);
-        const int32_t p = r.p;
-        if (!sel_eligible(mode, maxwgt, opt, r)) {
-            if (gl == 0) sel_decide(A, C, mode, v, r, false, 0, PartKey{0, -1});
-            continue;
+    for (; base < cnt; base += nwaves * rpw) {
+        const int32_t mv = nv;
+        SelRow mr;
+        if (mv >= 0) mr = sel_row(A, mode, mv);
+        const int64_t nb = base + nwaves * rpw;
+        nv = lane < rpw && nb + lane < cnt ? ids[nb + lane] : -1;   // the next rows
+        const bool mel = mv >= 0 && sel_eligible(mode, maxwgt, opt, mr);
+        // the row's first entry (offsets are below 2^31), its length and part
+        int32_t mb = 0, mpd = 0;
+        if (mel) {
+            const eid_t b = A.xadj[mv];
+            mb = (int32_t)b;
+            mpd = (int32_t)(A.xadj[mv + 1] - b) | (mr.p << 8);
+            kbytes += 16 + 12 * (uint64_t)(mpd & 255);
         }
-        const eid_t b = A.xadj[v], e = A.xadj[v + 1];
-        int32_t u[E], w[E], q[E];
-        load_entries<E, G>(A.adjncy, A.adjwgt, b, e, gl, u, w);
-        A.wq.gather(u, q);
-        if (gl == 0) kbytes += 16 + 12 * (uint64_t)(e - b);
-        if (mode == kModeRS) {
-            int32_t own = 0;
-#pragma unroll
-            for (int t = 0; t < E; t++) own += q[t] == p ? w[t] : 0;
-            own = group_sum<G>(own);
-            if (gl == 0) sel_decide(A, C, mode, v, r, true, own, PartKey{0, -1});
-            continue;
-        }
-#pragma unroll
-        for (int t = 0; t < E; t++)
-            if (q[t] >= 0) atomicAdd(&my[q[t]], w[t]);
+        const uint64_t bal = __ballot(mel);
+        const int ne = __popcll(bal);
+        if (mel) sl[__popcll(bal & lanemask_lt())] = lane;
         wave_lds_sync();
-        const int32_t pc = my[p];
-        PartKey best{0, -1};
+        for (int r0 = 0; r0 < ne; r0 += NP * NQ) {
+            int32_t u[NP][E], w[NP][E], q[NP][E], src[NP], pt[NP];
 #pragma unroll
-        for (int t = 0; t < E; t++) {
-            if (q[t] >= 0 && q[t] != p && tg[q[t]]) {
-                PartKey cand{my[q[t]], q[t]};
-                if (BetterPart()(cand, best)) best = cand;
+            for (int t = 0; t < NP; t++) {
+                const int r = r0 + t * NQ + grp;
+                src[t] = r < ne ? sl[r] : -1;
+                const int s = src[t] >= 0 ? src[t] : 0;
+                const int32_t b = __shfl(mb, s, kWave), pd = __shfl(mpd, s, kWave);   // every lane shuffles
+                const int32_t d = src[t] >= 0 ? pd & 255 : 0;
+                pt[t] = pd >> 8;
+#pragma unroll
+                for (int x = 0; x < E; x++) {
+                    u[t][x] = -1;
+                    w[t][x] = 0;
+                    if (gl + x * G < d) {
+                        u[t][x] = __builtin_nontemporal_load(A.adjncy + b + gl + x * G);
+                        w[t][x] = __builtin_nontemporal_load(A.adjwgt + b + gl + x * G);
+                    }
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < NP; t++) A.wq.gather(u[t], q[t]);
+#pragma unroll
+            for (int t = 0; t < NP; t++) {
+                if (r0 + t * NQ >= ne) break;   // the same for the whole wave
+                const int32_t p = pt[t];
+                const bool lead = src[t] >= 0 && gl == 0;
+                if (mode == kModeRS) {
+                    int32_t own = 0;
+#pragma unroll
+                    for (int x = 0; x < E; x++) own += q[t][x] == p ? w[t][x] : 0;
+                    own = group_sum<G>(own);
+                    if (lead) res[src[t]] = make_int3(own, 0, -1);
+                    continue;
+                }
+#pragma unroll
+                for (int x = 0; x < E; x++)
+                    if (q[t][x] >= 0) atomicAdd(&my[q[t][x]], w[t][x]);
+                wave_lds_sync();
+                const int32_t pc = my[p];
+                PartKey best{0, -1};
+#pragma unroll
+                for (int x = 0; x < E; x++) {
+                    if (q[t][x] >= 0 && q[t][x] != p && tg[q[t][x]]) {
+                        PartKey cand{my[q[t][x]], q[t][x]};
+                        if (BetterPart()(cand, best)) best = cand;
+                    }
+                }
+                best = group_best<G>(best, BetterPart());
+                wave_lds_sync();
+#pragma unroll
+                for (int x = 0; x < E; x++)
+                    if (q[t][x] >= 0) my[q[t][x]] = 0;
+                if (lead) res[src[t]] = make_int3(pc, best.c, best.q);
+                wave_lds_sync();
             }
         }
-        best = group_best<G>(best, BetterPart());
         wave_lds_sync();
-#pragma unroll
-        for (int t = 0; t < E; t++)
-            if (q[t] >= 0) my[q[t]] = 0;
+        if (mv >= 0) {
+            const int3 x = mel ? res[lane] : make_int3(0, 0, -1);
+            ncand += sel_decide(A, C, mode, mv, mr, mel, x.x, PartKey{x.y, x.z});
+        }
         wave_lds_sync();
-        if (gl == 0) ncand += sel_decide(A, C, mode, v, r, true, pc, best);
     }
     sel_count(A, mode, ncand);
     kb_flush(A.kb, kbytes);
 }
-
 
 // Rows of 9..512 entries (classes 1 and 2): a wave takes 64 rows of the list
 // at a time, decides the ineligible ones lane by lane and then walks the
@@ -633,7 +683,8 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_q(const int32_t *__restri
 // own k-int LDS row, so that one chain of loads and gathers serves four rows;
 // the longer rows (and all rows without Q) go one at a time with their
 // entries in registers (8 per lane, loaded in phases) and a k-int LDS row per
-// wave.  Waves loop on their own, without block barriers.
+// wave.  A row's result goes back to its lane through LDS and the 64 lanes
+// decide at once.  Waves loop on their own, without block barriers.
 constexpr int64_t kQuarterRow = kQuarterG * 8;
 
 template <bool Q>
@@ -642,6 +693,7 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
 {
     extern __shared__ int32_t acc[];   // k ints per wave (4k with Q), then k part flags
     constexpr int S = (int)(kBinMid / kWave), NQ = Q ? kWave / kQuarterG : 1;
+    __shared__ int3 results[kRowBS];   // per row: connectivity to the own part, best other part
     const JetCtl &C = *A.ctl;
     if (C.done) return;
     const int32_t mode = C.mode;
@@ -653,6 +705,7 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
     uint8_t *tg = (uint8_t *)(acc + (size_t)nw * NQ * k);
     for (int i = lane; i < NQ * k; i += kWave) my[i] = 0;
     load_targets(A, mode, maxwgt, tg);
+    int3 *res = results + wv * kWave;
     int32_t ncand = 0;
     uint64_t kbytes = 0;
     for (int64_t base = ((int64_t)blockIdx.x * nw + wv) * rpw; base < cnt; base += (int64_t)gridDim.x * nw * rpw) {
@@ -661,15 +714,17 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
         SelRow mr;
         if (mv >= 0) mr = sel_row(A, mode, mv);
         bool mel = mv >= 0 && sel_eligible(mode, maxwgt, opt, mr);
-        if (mv >= 0 && !mel) sel_decide(A, C, mode, mv, mr, false, 0, PartKey{0, -1});
-        eid_t mb = 0, me = 0;
+        // the row's first entry (offsets are below 2^31) and its length
+        int32_t mb = 0, md = 0;
         if (mel) {
-            mb = A.xadj[mv];
-            me = A.xadj[mv + 1];
+            const eid_t b = A.xadj[mv];
+            mb = (int32_t)b;
+            md = (int32_t)(A.xadj[mv + 1] - b);
+            kbytes += 16 + 12 * (uint64_t)md;
         }
         uint64_t todo = __ballot(mel);
         if constexpr (Q) {
-            uint64_t four = __ballot(mel && me - mb <= kQuarterRow);
+            uint64_t four = __ballot(mel && md <= kQuarterRow);
             todo &= ~four;
             while (four) {
                 int ql = -1;   // the lane (row) of this lane's quarter, -1 when the rows ran out
@@ -680,22 +735,19 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
                     if (g == quarter) ql = l;
                 }
                 const int src = ql >= 0 ? ql : 0;
-                const int32_t v = __shfl(mv, src, kWave);
-                const SelRow rr = shfl_row(mr, src);
-                const int32_t p = rr.p;
-                const eid_t b = __shfl(mb, src, kWave), e1 = __shfl(me, src, kWave);   // every lane shuffles
-                const eid_t e = ql >= 0 ? e1 : b;
+                const int32_t p = __shfl(mr.p, src, kWave);
+                const int32_t b = __shfl(mb, src, kWave), d0 = __shfl(md, src, kWave);   // every lane shuffles
+                const int32_t e = ql >= 0 ? b + d0 : b;
                 int32_t u[8], w[8], q[8];
                 load_entries<8, kQuarterG>(A.adjncy, A.adjwgt, b, e, gl, u, w);
                 A.wq.gather(u, q);
                 const bool lead = gl == 0 && ql >= 0;
-                if (lead) kbytes += 16 + 12 * (uint64_t)(e - b);
                 if (mode == kModeRS) {
                     int32_t own = 0;
 #pragma unroll
                     for (int t = 0; t < 8; t++) own += q[t] == p ? w[t] : 0;
                     own = group_sum<kQuarterG>(own);
-                    if (lead) sel_decide(A, C, mode, v, rr, true, own, PartKey{0, -1});
+                    if (lead) res[src] = make_int3(own, 0, -1);
                     continue;
                 }
                 int32_t *mq = my + (size_t)quarter * k;
@@ -703,7 +755,7 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
                 for (int t = 0; t < 8; t++)
                     if (q[t] >= 0) atomicAdd(&mq[q[t]], w[t]);
                 wave_lds_sync();
-                const int32_t pc = ql >= 0 ? mq[p] : 0;
+                const int32_t pc = mq[p];
                 PartKey best{0, -1};
 #pragma unroll
                 for (int t = 0; t < 8; t++) {
@@ -717,17 +769,14 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
 #pragma unroll
                 for (int t = 0; t < 8; t++)
                     if (q[t] >= 0) mq[q[t]] = 0;
+                if (lead) res[src] = make_int3(pc, best.c, best.q);
                 wave_lds_sync();
-                if (lead) ncand += sel_decide(A, C, mode, v, rr, true, pc, best);
             }
         }
         while (todo) {
-            int l = __ffsll((long long)todo) - 1;
+            const int l = __ffsll((long long)todo) - 1;
             todo &= todo - 1;
-            int32_t v = __shfl(mv, l, kWave);
-            const SelRow rr = shfl_row(mr, l);
-            const int32_t p = rr.p;
-            eid_t b = __shfl(mb, l, kWave), e = __shfl(me, l, kWave);
+            const int32_t p = wave_read(mr.p, l), b = wave_read(mb, l), e = b + wave_read(md, l);
             int32_t u[S], w[S], q[S];
             load_entries<S, kWave>(A.adjncy, A.adjwgt, b, e, lane, u, w);
             A.wq.gather(u, q);
@@ -737,10 +786,7 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
 #pragma unroll
                 for (int t = 0; t < S; t++) own += q[t] == p ? w[t] : 0;
                 own = wave_sum(own);
-                if (lane == 0) {
-                    sel_decide(A, C, mode, v, rr, true, own, PartKey{0, -1});
-                    kbytes += 16 + 12 * (uint64_t)(e - b);
-                }
+                if (lane == 0) res[l] = make_int3(own, 0, -1);
                 continue;
             }
 #pragma unroll
@@ -761,12 +807,15 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
 #pragma unroll
             for (int t = 0; t < S; t++)
                 if (q[t] >= 0) my[q[t]] = 0;
+            if (lane == 0) res[l] = make_int3(pc, best.c, best.q);
             wave_lds_sync();
-            if (lane == 0) {
-                ncand += sel_decide(A, C, mode, v, rr, true, pc, best);
-                kbytes += 16 + 12 * (uint64_t)(e - b);
-            }
         }
+        wave_lds_sync();
+        if (mv >= 0) {
+            const int3 x = mel ? res[lane] : make_int3(0, 0, -1);
+            ncand += sel_decide(A, C, mode, mv, mr, mel, x.x, PartKey{x.y, x.z});
+        }
+        wave_lds_sync();
     }
     sel_count(A, mode, ncand);
     kb_flush(A.kb, kbytes);
@@ -1797,12 +1846,11 @@ void launch_select(Ctx &c, const DevGraph &g, int32_t k, const int32_t *where, c
     // wave-per-row launch
     const bool quarter = !b.few() && k <= kQuarterK && b.count(1) > 0;
     if (quarter) {
-        KScope ks(c, "k_jet_select_q", 24.0 * (double)b.count(1), true);
+        KScope ks(c, "k_jet_select_m", 24.0 * (double)b.count(1), true);
         A.kb = ks.dev();
-        constexpr int NG = kRowBS / kQuarterG;
-        unsigned blocks = (unsigned)std::min<int64_t>((b.count(1) + NG - 1) / NG, 32768);
-        k_jet_select_q<<<blocks, kRowBS, sizeof(int32_t) * NG * (size_t)k + tg_bytes, c.stream>>>(b.list(1),
-                                                                                               b.count(1), A);
+        const int32_t rpw = rows_per_wave(b.count(1));
+        k_jet_select_m<<<wave_blocks(b.count(1), rpw, 4096), kRowBS, sel_m_lds(k) + tg_bytes, c.stream>>>(
+            b.list(1), b.count(1), rpw, A);
         HGP_LAUNCH_CHECK();
     }
     if (int64_t nw = b.few() ? 0 : (quarter ? 0 : b.count(1)) + b.count(2)) {
