@@ -437,9 +437,8 @@ void detach_fused(Ctx &c, size_t m0, size_t m1, FusedGraph &f)
     for (int32_t *&p : f.cmaps) rb(p);
     for (int32_t *&p : f.where) rb(p);
     TinyScratch &t = f.s;
-    rb(t.dest), rb(t.pregain), rb(t.best), rb(t.elist), rb(t.under), rb(t.es), rb(t.ee), rb(t.pstart);
-    rb(t.iters), rb(t.lock), rb(t.sel), rb(t.w8), rb(t.w16), rb(t.pd16), rb(t.pd32), rb(t.key), rb(t.val);
-    rb(t.k2), rb(t.v2), rb(t.ab), rb(t.wsc), rb(t.bs), rb(t.pwgts), rb(t.cut), rb(t.ctl);
+    rb(t.dest), rb(t.pregain), rb(t.best), rb(t.under), rb(t.iters), rb(t.lock), rb(t.sel), rb(t.w8), rb(t.w16);
+    rb(t.pd16), rb(t.pd32), rb(t.key), rb(t.ab), rb(t.bs), rb(t.pwgts), rb(t.cut), rb(t.ctl);
 }
 
 // Statistics of a fused batch graph from its level-0 partition part0.

@@ -101,13 +101,12 @@ constexpr int32_t kTinyMaxK = 256;
 // cut (int64; in: the coarsest partition's cut, out: the cut after the
 // last level) and the Jet iterations of each level (HGP_MAX_LEVELS ints).
 struct TinyScratch {
-    int32_t *dest = nullptr, *pregain = nullptr, *best = nullptr, *elist = nullptr;
-    int32_t *under = nullptr, *es = nullptr, *ee = nullptr, *pstart = nullptr, *iters = nullptr;
+    int32_t *dest = nullptr, *pregain = nullptr, *best = nullptr, *under = nullptr, *iters = nullptr;
     uint8_t *lock = nullptr, *sel = nullptr, *w8 = nullptr;
     uint16_t *w16 = nullptr, *pd16 = nullptr;
-    uint32_t *pd32 = nullptr, *key = nullptr, *val = nullptr, *k2 = nullptr, *v2 = nullptr;
+    uint32_t *pd32 = nullptr, *key = nullptr;
     uint64_t *ab = nullptr;
-    int64_t *wsc = nullptr, *bs = nullptr, *pwgts = nullptr, *cut = nullptr;
+    int64_t *bs = nullptr, *pwgts = nullptr, *cut = nullptr;
     void *ctl = nullptr;   // the Jet control block
 };
 TinyScratch alloc_tiny_scratch(Ctx &c, int32_t n, int32_t k);

@@ -10,6 +10,7 @@
 #include "hgp_graph.hpp"
 #include "hgp_jet.hpp"
 #include "hgp_prims.hpp"
+#include "hgp_rebalance_block.hpp"
 
 #include "hunyuangraph.h"
 
@@ -464,6 +465,42 @@ __device__ inline void load_targets(const SelArgs &A, int32_t mode, int64_t maxw
 // passes a wave: 12 us at 65k rows and 80 us at 1.5M.)
 constexpr int kRowT = (int)kBinSmall;
 
+__device__ inline void load_short_row(const vid_t *__restrict__ adjncy, const wgt_t *__restrict__ adjwgt, eid_t b,
+                                      int32_t d, int32_t (&u)[kRowT], int32_t (&w)[kRowT])
+{
+#pragma unroll
+    for (int t = 0; t < kRowT; t++) {
+        u[t] = -1;
+        w[t] = 0;
+        if (t < d) {
+            u[t] = adjncy[b + t];
+            w[t] = adjwgt[b + t];
+        }
+    }
+}
+
+// Connectivity to part p and, with `parts`, the best target part of a row
+// whose entries lie in parts q (-1: no entry).
+__device__ inline void short_row_sums(const int32_t (&q)[kRowT], const int32_t (&w)[kRowT], int32_t p, bool parts,
+                                      const uint8_t *tg, int32_t &pc, PartKey &best)
+{
+    pc = 0;
+    best = PartKey{0, -1};
+#pragma unroll
+    for (int t = 0; t < kRowT; t++) pc += q[t] == p ? w[t] : 0;
+    if (!parts) return;
+#pragma unroll
+    for (int t = 0; t < kRowT; t++) {
+        int32_t c = 0;
+#pragma unroll
+        for (int x = 0; x < kRowT; x++) c += q[x] == q[t] ? w[x] : 0;
+        const bool ok = q[t] >= 0 && q[t] != p && tg[q[t] >= 0 ? q[t] : 0];
+        const bool better = ok && (c > best.c || (c == best.c && c > 0 && q[t] < best.q));
+        best.c = better ? c : best.c;
+        best.q = better ? q[t] : best.q;
+    }
+}
+
 __global__ void __launch_bounds__(kRowBS) k_jet_select_t(const int32_t *__restrict__ ids, int64_t cnt, SelArgs A)
 {
     extern __shared__ int64_t pw[];   // k part weights, then k part flags
@@ -501,15 +538,7 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_t(const int32_t *__restri
         int32_t u[kRowT], w[kRowT], q[kRowT];
         const eid_t b = el ? A.xadj[v] : 0;
         const int32_t d = el ? (int32_t)(A.xadj[v + 1] - b) : 0;
-#pragma unroll
-        for (int t = 0; t < kRowT; t++) {
-            u[t] = -1;
-            w[t] = 0;
-            if (t < d) {
-                u[t] = A.adjncy[b + t];
-                w[t] = A.adjwgt[b + t];
-            }
-        }
+        load_short_row(A.adjncy, A.adjwgt, b, d, u, w);
         A.wq.gather(u, q);
         // the next chunk's rows, loaded while this one is decided
         const int32_t cv = v;
@@ -517,22 +546,9 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_t(const int32_t *__restri
         i += (int64_t)gridDim.x * kRowBS;
         v = i < cnt ? ids[i] : -1;
         if (cv >= 0) {
-            int32_t pc = 0;
-            PartKey best{0, -1};
-#pragma unroll
-            for (int t = 0; t < kRowT; t++) pc += q[t] == cr.p ? w[t] : 0;
-            if (mode != kModeRS) {
-#pragma unroll
-                for (int t = 0; t < kRowT; t++) {
-                    int32_t c = 0;
-#pragma unroll
-                    for (int x = 0; x < kRowT; x++) c += q[x] == q[t] ? w[x] : 0;
-                    const bool ok = q[t] >= 0 && q[t] != cr.p && tg[q[t] >= 0 ? q[t] : 0];
-                    const bool better = ok && (c > best.c || (c == best.c && c > 0 && q[t] < best.q));
-                    best.c = better ? c : best.c;
-                    best.q = better ? q[t] : best.q;
-                }
-            }
+            int32_t pc;
+            PartKey best;
+            short_row_sums(q, w, cr.p, mode != kModeRS, tg, pc, best);
             ncand += sel_decide(A, C, mode, cv, cr, el, pc, best);
             if (el) kbytes += 16 + 12 * (uint64_t)d;
         }
@@ -565,35 +581,24 @@ constexpr int32_t kTrackMaxK = 512;
 // apart, and the part flags.
 inline size_t sel_m_lds(int32_t k) { return sizeof(int32_t) * (kRowBS / kQuarterG) * (size_t)(k | 1); }
 
-__global__ void __launch_bounds__(kRowBS) k_jet_select_m(const int32_t *__restrict__ ids, int64_t cnt, int32_t rpw,
-                                                         SelArgs A)
+// The rows of one wave: ids[base .. base + rpw) (nv: this lane's id, loaded
+// already), then `step` further on.  my: this lane's group's zeroed k-int row,
+// sl and res: 64 words and 64 results of the wave.  Returns the lane's LP
+// candidates.
+template <int NP>
+__device__ inline int32_t select_mid(const SelArgs &A, const JetCtl &C, int32_t mode, int64_t maxwgt, int64_t opt,
+                                     const int32_t *__restrict__ ids, int64_t cnt, int64_t base, int64_t step,
+                                     int32_t rpw, int32_t nv, int32_t *my, const uint8_t *tg, int32_t *sl, int3 *res,
+                                     uint64_t &kbytes)
 {
-    extern __shared__ int32_t acc[];
-    constexpr int G = kQuarterG, NG = kRowBS / G, NQ = kWave / G, E = (int)(kBinHalf / G), NP = kMidPasses;
-    __shared__ int32_t slots[kRowBS];   // per wave: lanes holding eligible rows, in rank order
-    __shared__ int3 results[kRowBS];    // per row: connectivity to the own part, best other part
-    const JetCtl &C = *A.ctl;
-    const int lane = lane_id(), wv = threadIdx.x / kWave, grp = lane / G, gl = lane % G;
-    const int64_t nwaves = (int64_t)gridDim.x * (kRowBS / kWave);
-    int64_t base = ((int64_t)blockIdx.x * (kRowBS / kWave) + wv) * rpw;
-    int32_t nv = lane < rpw && base + lane < cnt ? ids[base + lane] : -1;
-    if (C.done) return;
-    const int32_t mode = C.mode;
-    const int64_t maxwgt = C.maxwgt, opt = C.opt;
-    const int k = A.k, stride = k | 1;
-    int32_t *my = acc + (size_t)(wv * NQ + grp) * stride;
-    uint8_t *tg = (uint8_t *)(acc + (size_t)NG * stride);
-    int32_t *sl = slots + wv * kWave;
-    int3 *res = results + wv * kWave;
-    for (int i = gl; i < k; i += G) my[i] = 0;
-    load_targets(A, mode, maxwgt, tg);
+    constexpr int G = kQuarterG, NQ = kWave / G, E = (int)(kBinHalf / G);
+    const int lane = lane_id(), grp = lane / G, gl = lane % G;
     int32_t ncand = 0;
-    uint64_t kbytes = 0;
-    for (; base < cnt; base += nwaves * rpw) {
+    for (; base < cnt; base += step) {
         const int32_t mv = nv;
         SelRow mr;
         if (mv >= 0) mr = sel_row(A, mode, mv);
-        const int64_t nb = base + nwaves * rpw;
+        const int64_t nb = base + step;
         nv = lane < rpw && nb + lane < cnt ? ids[nb + lane] : -1;   // the next rows
         const bool mel = mv >= 0 && sel_eligible(mode, maxwgt, opt, mr);
         // the row's first entry (offsets are below 2^31), its length and part
@@ -672,6 +677,33 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_m(const int32_t *__restri
         }
         wave_lds_sync();
     }
+    return ncand;
+}
+
+__global__ void __launch_bounds__(kRowBS) k_jet_select_m(const int32_t *__restrict__ ids, int64_t cnt, int32_t rpw,
+                                                         SelArgs A)
+{
+    extern __shared__ int32_t acc[];
+    constexpr int G = kQuarterG, NG = kRowBS / G, NQ = kWave / G;
+    __shared__ int32_t slots[kRowBS];   // per wave: lanes holding eligible rows, in rank order
+    __shared__ int3 results[kRowBS];    // per row: connectivity to the own part, best other part
+    const JetCtl &C = *A.ctl;
+    const int lane = lane_id(), wv = threadIdx.x / kWave, grp = lane / G, gl = lane % G;
+    const int64_t nwaves = (int64_t)gridDim.x * (kRowBS / kWave);
+    int64_t base = ((int64_t)blockIdx.x * (kRowBS / kWave) + wv) * rpw;
+    int32_t nv = lane < rpw && base + lane < cnt ? ids[base + lane] : -1;
+    if (C.done) return;
+    const int32_t mode = C.mode;
+    const int64_t maxwgt = C.maxwgt, opt = C.opt;
+    const int k = A.k, stride = k | 1;
+    int32_t *my = acc + (size_t)(wv * NQ + grp) * stride;
+    uint8_t *tg = (uint8_t *)(acc + (size_t)NG * stride);
+    int32_t *sl = slots + wv * kWave;
+    for (int i = gl; i < k; i += G) my[i] = 0;
+    load_targets(A, mode, maxwgt, tg);
+    uint64_t kbytes = 0;
+    const int32_t ncand = select_mid<kMidPasses>(A, C, mode, maxwgt, opt, ids, cnt, base, nwaves * rpw, rpw, nv, my, tg,
+                                                 sl, results + wv * kWave, kbytes);
     sel_count(A, mode, ncand);
     kb_flush(A.kb, kbytes);
 }
@@ -1139,15 +1171,7 @@ __global__ void __launch_bounds__(kRowBS) k_afterburner_t(const int32_t *__restr
             const int32_t d = (int32_t)(xadj[v + 1] - b);
             int32_t u[kRowT], w[kRowT];
             uint64_t x[kRowT];
-#pragma unroll
-            for (int t = 0; t < kRowT; t++) {
-                u[t] = -1;
-                w[t] = 0;
-                if (t < d) {
-                    u[t] = adjncy[b + t];
-                    w[t] = adjwgt[b + t];
-                }
-            }
+            load_short_row(adjncy, adjwgt, b, d, u, w);
 #pragma unroll
             for (int t = 0; t < kRowT; t++) x[t] = u[t] >= 0 ? ab[u[t]] : 0ull;
             int64_t change = 0;
@@ -1470,15 +1494,7 @@ __global__ void __launch_bounds__(kRowBS) k_move_delta_t(const int32_t *__restri
             const int32_t d = (int32_t)(xadj[v + 1] - b);
             const int64_t wv = vwgt[v];
             int32_t u[kRowT], w[kRowT], pu[kRowT], du[kRowT];
-#pragma unroll
-            for (int t = 0; t < kRowT; t++) {
-                u[t] = -1;
-                w[t] = 0;
-                if (t < d) {
-                    u[t] = adjncy[b + t];
-                    w[t] = adjwgt[b + t];
-                }
-            }
+            load_short_row(adjncy, adjwgt, b, d, u, w);
             pq.gather(u, pu, du);
             atomicAdd(&pdelta[pv], (unsigned long long)(-wv));
             atomicAdd(&pdelta[dv], (unsigned long long)wv);
@@ -1938,14 +1954,11 @@ void project(Ctx &c, int32_t n, const int32_t *cmap, const int32_t *where_c, int
 // in one block of kTinyBS threads: the same phases as the kernels above
 // (selection, afterburner, LP filter, RW/RS eviction with its sort and cookie
 // cutter, move accounting, commit, bookkeeping) separated by block barriers
-// instead of launches, and no host round trip per iteration.  Rows are
-// walked one per wave in chunks of 256 entries; per-vertex phases stride the
-// block.  The block's 16 waves walk rows one after another, so the path
+// instead of launches, and no host round trip per iteration.  The block's 16 waves walk rows one after another, so the path
 // pays off only while a level's rows are few: measured on grids, 3-D RGGs
 // and banded graphs, 512 vertices beat both 256 and 1024.
 constexpr int kTinyBS = 1024;
 constexpr int kTinyWaves = kTinyBS / kWave;
-constexpr int32_t kTinyN = 4096;   // chunk of the block-local scans and compactions
 constexpr int32_t kTinyK = 256;
 constexpr int kTinyChunk = 4;                         // entries per lane and chunk
 constexpr eid_t kTinyRow = (eid_t)kTinyChunk * kWave;  // row entries per chunk
@@ -1953,132 +1966,66 @@ constexpr eid_t kTinyRow = (eid_t)kTinyChunk * kWave;  // row entries per chunk
 struct TinyArgs {
     SelArgs A;                   // selection inputs and outputs (dest, pregain, key, ab, pairs, under, ctl)
     int32_t n, sort_bits;
-    int32_t *where, *under, *best, *pstart, *elist, *es, *ee;
+    const int32_t *ids;          // rows by degree class: [0, c0) <= 8 entries, [c0, c1) <= 32, the rest longer
+    int32_t c0, c1;
+    int32_t *where, *under, *best;
     uint8_t *sel, *lock, *w8;
     uint16_t *w16;
-    uint32_t *val, *k2, *v2;
-    int64_t *pwgts, *wsc, *bs;
+    int64_t *pwgts, *bs;
 };
 
+constexpr int kTinyGroups = kTinyBS / kQuarterG;
+
+// Dynamic LDS of the one-block loop for levels of up to n vertices: the
+// selection's k-int rows (one per 16-lane group) with each wave's slots and
+// results, or in another phase the rebalancer's arrays; then k words (cut-off
+// bases, part-weight changes) and the part flags.
+__host__ __device__ inline size_t tiny_sel_lds(int32_t k)
+{
+    return (sizeof(int32_t) * kTinyGroups * (size_t)(k | 1) + (sizeof(int32_t) + sizeof(int3)) * kTinyBS + 15) / 16 * 16;
+}
+template <int R>
+__host__ __device__ inline size_t tiny_work_lds(int32_t k)
+{
+    const size_t a = tiny_sel_lds(k), b = (sizeof(RbLds<R>) + 15) / 16 * 16;
+    return a > b ? a : b;
+}
+template <int R>
 inline size_t tiny_lds(int32_t k)
 {
-    return sizeof(int32_t) * (size_t)kTinyWaves * k + (((size_t)k + 7) / 8) * 8 + sizeof(int64_t) * (size_t)k;
+    return tiny_work_lds<R>(k) + sizeof(int64_t) * (size_t)k + ((size_t)k + 15) / 16 * 16;
 }
 
 struct TinyShared {
     NextScratch nx;
-    uint32_t cnt[256], base_d[256];
-    uint32_t wcnt[kTinyWaves][256];
-    uint32_t ssh[kTinyWaves + 1];
     int64_t lsh[kTinyWaves + 1];
     unsigned long long d2[kTinyWaves];
     int32_t done, mode;
 };
 
-// Inclusive scan of a[0..n) in place (n <= kTinyBS * 4), one block.
-__device__ inline void tiny_scan_i64(int64_t *a, int32_t n, TinyShared &S)
-{
-    constexpr int E = kTinyN / kTinyBS;
-    int64_t carry = 0;
-    for (int32_t base = 0; base < n; base += kTinyN) {   // chunks of kTinyN, the running sum carried
-        const int32_t m = min(n - base, kTinyN);
-        const int32_t b = threadIdx.x * E;
-        int64_t x[E], run = 0;
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            x[e] = b + e < m ? a[base + b + e] : 0;
-            run += x[e];
-        }
-        int64_t tot;
-        int64_t off = carry + block_exclusive_scan<int64_t>(run, S.lsh, &tot);
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            off += x[e];
-            if (b + e < m) a[base + b + e] = off;
-        }
-        carry += tot;
-        __syncthreads();
-    }
-}
-
-// Stable LSD radix sort of (key, val)[0..n) over bits [0, hi) in 8-bit
-// digits, one block; the result ends in key/val.
-__device__ inline void tiny_sort(uint32_t *key, uint32_t *val, uint32_t *k2, uint32_t *v2, int32_t n, int hi,
-                                 TinyShared &S)
-{
-    const int t = threadIdx.x, w = t / kWave;
-    uint32_t *sk = key, *sv = val, *dk = k2, *dv = v2;
-    for (int shift = 0; shift < hi; shift += 8) {
-        if (t < 256) S.cnt[t] = 0;
-        __syncthreads();
-        for (int32_t i = t; i < n; i += kTinyBS) atomicAdd(&S.cnt[(sk[i] >> shift) & 255u], 1u);
-        __syncthreads();
-        uint32_t ex = block_exclusive_scan<uint32_t>(t < 256 ? S.cnt[t] : 0u, S.ssh, nullptr);
-        if (t < 256) S.base_d[t] = ex;
-        __syncthreads();
-        for (int32_t first = 0; first < n; first += kTinyBS) {
-            for (int i = t; i < kTinyWaves * 256; i += kTinyBS) (&S.wcnt[0][0])[i] = 0;
-            __syncthreads();
-            int32_t i = first + t;
-            bool valid = i < n;
-            uint32_t kk = valid ? sk[i] : 0u, vv = valid ? sv[i] : 0u;
-            uint32_t d = (kk >> shift) & 255u;
-            uint64_t m = __ballot(valid);
-#pragma unroll
-            for (int bit = 0; bit < 8; bit++) {
-                bool on = (d >> bit) & 1u;
-                uint64_t bb = __ballot(on);
-                m &= on ? bb : ~bb;
-            }
-            uint64_t lower = m & lanemask_lt();
-            uint32_t rank = (uint32_t)__popcll(lower);
-            if (valid && lower == 0) S.wcnt[w][d] = (uint32_t)__popcll(m);
-            __syncthreads();
-            if (t < 256) {
-                uint32_t acc = S.base_d[t];
-                for (int ww = 0; ww < kTinyWaves; ww++) {
-                    uint32_t c = S.wcnt[ww][t];
-                    S.wcnt[ww][t] = acc;
-                    acc += c;
-                }
-                S.base_d[t] = acc;
-            }
-            __syncthreads();
-            if (valid) {
-                uint32_t pos = S.wcnt[w][d] + rank;
-                dk[pos] = kk;
-                dv[pos] = vv;
-            }
-            __syncthreads();
-        }
-        uint32_t *tk = sk; sk = dk; dk = tk;
-        uint32_t *tv = sv; sv = dv; dv = tv;
-    }
-    if (sk != key) {
-        for (int32_t i = t; i < n; i += kTinyBS) {
-            key[i] = sk[i];
-            val[i] = sv[i];
-        }
-    }
-    __syncthreads();
-}
-
-// The whole Jet loop of one level in the calling block (kTinyBS threads).
-// dyn: per-wave k-int conn rows | k part flags (8-byte padded) | k int64
-// deltas (tiny_lds(k) bytes of dynamic LDS).
-__device__ inline void jet_tiny_loop(const TinyArgs &T, int32_t *dyn, TinyShared &S)
+// The whole Jet loop of one level of at most 1024 R vertices in the calling
+// block (kTinyBS threads); dyn: tiny_lds<R>(k) bytes of dynamic LDS for the
+// launch's largest k, `work` of them the shared working area.  Rows go by degree class as in the kernels
+// above: a lane each up to 8 entries, 16 lanes up to 32, a wave beyond.  (A
+// wave per row, whatever its length, walked an 8192-vertex level in 512 serial
+// steps a phase.)
+template <int R>
+__device__ inline void jet_tiny_loop(const TinyArgs &T, char *dyn, size_t work, TinyShared &S)
 {
     const SelArgs &A = T.A;
     JetCtl &C = *A.ctl;
     const int32_t n = T.n, k = A.k;
     const int tid = threadIdx.x, lane = lane_id(), wv = tid / kWave;
-    int32_t *my = dyn + (size_t)wv * k;
-    uint8_t *tg = (uint8_t *)(dyn + (size_t)kTinyWaves * k);
-    unsigned long long *pdelta = (unsigned long long *)(dyn + (size_t)kTinyWaves * k + (((size_t)k + 7) / 8) * 2);
+    constexpr int G = kQuarterG, E = (int)(kBinHalf / G), R4 = 4;   // R4: rows per group in flight
+    const int grp = tid / G, gl = tid % G;
+    int32_t *conn = (int32_t *)dyn, *my = conn + (size_t)grp * (k | 1);
+    int32_t *wrow = conn + (size_t)wv * (kWave / G) * (k | 1);   // a wave's row: its first group's
+    int32_t *sl = conn + (size_t)kTinyGroups * (k | 1) + wv * kWave;
+    int3 *res = (int3 *)(conn + (size_t)kTinyGroups * (k | 1) + kTinyBS) + wv * kWave;
+    int64_t *part = (int64_t *)(dyn + work);
+    unsigned long long *pdelta = (unsigned long long *)part;
+    uint8_t *tg = (uint8_t *)(part + k);
     const PairParts pq{A.pd16, A.pd32};
-    const uint32_t nokey = (uint32_t)k * kMaxBuckets;
-    for (int i = tid; i < kTinyWaves * k; i += kTinyBS) dyn[i] = 0;
-    __syncthreads();
     jet_next(C, k, T.pwgts, T.under, 1, S.nx);
     if (tid == 0) { S.done = C.done; S.mode = C.mode; }
     __syncthreads();
@@ -2086,11 +2033,36 @@ __device__ inline void jet_tiny_loop(const TinyArgs &T, int32_t *dyn, TinyShared
         const int32_t mode = S.mode;
         const int64_t maxwgt = C.maxwgt, opt = C.opt;
 
-        // selection (k_jet_select_*): one row per wave
+        // selection (k_jet_select_*)
+        for (int i = tid; i < kTinyGroups * (k | 1); i += kTinyBS) conn[i] = 0;
         for (int q = tid; q < k; q += kTinyBS) tg[q] = sel_target(A, mode, maxwgt, q) ? 1 : 0;
         __syncthreads();
         int32_t ncand = 0;
-        for (int32_t v = wv; v < n; v += kTinyWaves) {
+        uint64_t kbytes = 0;
+        for (int32_t i = tid; i < T.c0; i += kTinyBS) {
+            const int32_t v = T.ids[i];
+            const SelRow r = sel_row(A, mode, v);
+            const bool el = sel_eligible(mode, maxwgt, opt, r);
+            const eid_t b = el ? A.xadj[v] : 0;
+            const int32_t d = el ? (int32_t)(A.xadj[v + 1] - b) : 0;
+            int32_t u[kRowT], w[kRowT], q[kRowT], pc;
+            PartKey best;
+            load_short_row(A.adjncy, A.adjwgt, b, d, u, w);
+            A.wq.gather(u, q);
+            short_row_sums(q, w, r.p, mode != kModeRS, tg, pc, best);
+            ncand += sel_decide(A, C, mode, v, r, el, pc, best);
+        }
+        if (T.c1 > T.c0) {
+            const int32_t cnt = T.c1 - T.c0;
+            const int32_t rpw = max(4, min(kWave, (cnt + kTinyWaves - 1) / kTinyWaves));
+            const int32_t base = wv * rpw;
+            const int32_t *ids = T.ids + T.c0;
+            const int32_t nv = lane < rpw && base + lane < cnt ? ids[base + lane] : -1;
+            ncand += select_mid<4>(A, C, mode, maxwgt, opt, ids, cnt, base, kTinyWaves * rpw, rpw, nv, my, tg, sl, res,
+                                   kbytes);
+        }
+        for (int32_t i = T.c1 + wv; i < n; i += kTinyWaves) {
+            const int32_t v = T.ids[i];
             const SelRow r = sel_row(A, mode, v);
             const int32_t p = r.p;
             if (!sel_eligible(mode, maxwgt, opt, r)) {
@@ -2119,23 +2091,23 @@ __device__ inline void jet_tiny_loop(const TinyArgs &T, int32_t *dyn, TinyShared
                 A.wq.gather(u, q);
 #pragma unroll
                 for (int t = 0; t < kTinyChunk; t++)
-                    if (q[t] >= 0) atomicAdd(&my[q[t]], w[t]);
+                    if (q[t] >= 0) atomicAdd(&wrow[q[t]], w[t]);
             }
             wave_lds_sync();
-            const int32_t pc = my[p];
+            const int32_t pc = wrow[p];
             PartKey best{0, -1};
             if (one) {
 #pragma unroll
                 for (int t = 0; t < kTinyChunk; t++) {
                     if (q[t] >= 0 && q[t] != p && tg[q[t]]) {
-                        PartKey cand{my[q[t]], q[t]};
+                        PartKey cand{wrow[q[t]], q[t]};
                         if (BetterPart()(cand, best)) best = cand;
                     }
                 }
             } else {
                 for (int qq = lane; qq < k; qq += kWave) {
                     if (qq == p || !tg[qq]) continue;
-                    PartKey cand{my[qq], qq};
+                    PartKey cand{wrow[qq], qq};
                     if (BetterPart()(cand, best)) best = cand;
                 }
             }
@@ -2144,9 +2116,9 @@ __device__ inline void jet_tiny_loop(const TinyArgs &T, int32_t *dyn, TinyShared
             if (one) {
 #pragma unroll
                 for (int t = 0; t < kTinyChunk; t++)
-                    if (q[t] >= 0) my[q[t]] = 0;
+                    if (q[t] >= 0) wrow[q[t]] = 0;
             } else {
-                for (int qq = lane; qq < k; qq += kWave) my[qq] = 0;
+                for (int qq = lane; qq < k; qq += kWave) wrow[qq] = 0;
             }
             wave_lds_sync();
             if (lane == 0) ncand += sel_decide(A, C, mode, v, r, true, pc, best);
@@ -2156,7 +2128,58 @@ __device__ inline void jet_tiny_loop(const TinyArgs &T, int32_t *dyn, TinyShared
 
         if (mode == kModeLP) {
             // afterburner (k_afterburner*)
-            for (int32_t v = wv; v < n; v += kTinyWaves) {
+            for (int32_t i = tid; i < T.c0; i += kTinyBS) {
+                const int32_t v = T.ids[i], ig = A.pregain[v];
+                bool keep = false;
+                if (ig != kNoGain) {
+                    const int32_t p = T.where[v], bd = A.dest[v];
+                    const eid_t b = A.xadj[v];
+                    int32_t u[kRowT], w[kRowT];
+                    uint64_t x[kRowT];
+                    load_short_row(A.adjncy, A.adjwgt, b, (int32_t)(A.xadj[v + 1] - b), u, w);
+#pragma unroll
+                    for (int t = 0; t < kRowT; t++) x[t] = u[t] >= 0 ? A.ab[u[t]] : 0ull;
+                    int64_t change = 0;
+#pragma unroll
+                    for (int t = 0; t < kRowT; t++)
+                        if (u[t] >= 0) change += ab_change(v, ig, p, bd, u[t], w[t], x[t]);
+                    keep = (int64_t)ig + change >= 0;
+                }
+                T.sel[v] = keep ? 1 : 0;
+            }
+            for (int32_t i0 = T.c0 + grp; i0 < T.c1; i0 += R4 * kTinyGroups) {
+                int32_t v[R4], ig[R4], p[R4], bd[R4], u[R4][E], w[R4][E];
+                eid_t b[R4], e[R4];
+#pragma unroll
+                for (int r = 0; r < R4; r++) {
+                    v[r] = i0 + r * kTinyGroups < T.c1 ? T.ids[i0 + r * kTinyGroups] : -1;
+                    ig[r] = v[r] >= 0 ? A.pregain[v[r]] : kNoGain;
+                }
+#pragma unroll
+                for (int r = 0; r < R4; r++) {
+                    const bool live = ig[r] != kNoGain;
+                    p[r] = live ? T.where[v[r]] : 0;
+                    bd[r] = live ? A.dest[v[r]] : 0;
+                    b[r] = live ? A.xadj[v[r]] : 0;
+                    e[r] = live ? A.xadj[v[r] + 1] : 0;
+                }
+#pragma unroll
+                for (int r = 0; r < R4; r++) load_entries<E, G>(A.adjncy, A.adjwgt, b[r], e[r], gl, u[r], w[r]);
+#pragma unroll
+                for (int r = 0; r < R4; r++) {
+                    uint64_t x[E];
+#pragma unroll
+                    for (int t = 0; t < E; t++) x[t] = u[r][t] >= 0 ? A.ab[u[r][t]] : 0ull;
+                    int64_t change = 0;
+#pragma unroll
+                    for (int t = 0; t < E; t++)
+                        if (u[r][t] >= 0) change += ab_change(v[r], ig[r], p[r], bd[r], u[r][t], w[r][t], x[t]);
+                    change = group_sum<G>(change);
+                    if (gl == 0 && v[r] >= 0) T.sel[v[r]] = ig[r] != kNoGain && (int64_t)ig[r] + change >= 0 ? 1 : 0;
+                }
+            }
+            for (int32_t i = T.c1 + wv; i < n; i += kTinyWaves) {
+                const int32_t v = T.ids[i];
                 const int32_t ig = A.pregain[v];
                 if (ig == kNoGain) {
                     if (lane == 0) T.sel[v] = 0;
@@ -2194,100 +2217,9 @@ __device__ inline void jet_tiny_loop(const TinyArgs &T, int32_t *dyn, TinyShared
                 store_pair(A.pd16, A.pd32, v, w, d);
             }
         } else {
-            // RW / RS eviction (k_rb_*, k_rs_*)
-            for (int32_t v = tid; v < n; v += kTinyBS) T.val[v] = (uint32_t)v;
-            __syncthreads();
-            tiny_sort(A.key, T.val, T.k2, T.v2, n, T.sort_bits, S);
-            for (int32_t i = tid; i < n; i += kTinyBS) T.wsc[i] = A.key[i] < nokey ? A.vwgt[T.val[i]] : 0;
-            __syncthreads();
-            tiny_scan_i64(T.wsc, n, S);
-            for (int32_t i = tid; i < n; i += kTinyBS) {
-                uint32_t kk = A.key[i];
-                if (kk >= nokey) continue;
-                uint32_t p = kk / kMaxBuckets;
-                if (i == 0 || A.key[i - 1] / kMaxBuckets != p) T.pstart[p] = i;
-            }
-            __syncthreads();
-            for (int32_t i = tid; i < n; i += kTinyBS) {
-                uint32_t kk = A.key[i];
-                int32_t v = (int32_t)T.val[i];
-                if (kk >= nokey) {
-                    T.sel[i] = 0;
-                    continue;
-                }
-                int32_t p = (int32_t)(kk / kMaxBuckets);
-                int32_t s0 = T.pstart[p];
-                int64_t before = T.wsc[i] - A.vwgt[v] - (s0 > 0 ? T.wsc[s0 - 1] : 0);
-                bool evict = before < T.pwgts[p] - maxwgt;
-                T.sel[i] = evict ? 1 : 0;
-                if (mode != kModeRW || !evict) {
-                    int32_t w = T.where[v];
-                    A.dest[v] = w;
-                    store_pair(A.pd16, A.pd32, v, w, w);
-                }
-            }
-            __syncthreads();
-            if (mode == kModeRS) {
-                // the evicted list in sorted order, its weight prefix, the cookie cutter
-                constexpr int E = kTinyN / kTinyBS;
-                int32_t ne = 0;
-                for (int32_t base = 0; base < n; base += kTinyN) {   // chunks of kTinyN, in order
-                    const int32_t b0 = base + tid * E;
-                    int32_t f[E], cnt = 0;
-#pragma unroll
-                    for (int e = 0; e < E; e++) {
-                        f[e] = (b0 + e < n && T.sel[b0 + e]) ? 1 : 0;
-                        cnt += f[e];
-                    }
-                    uint32_t tot;
-                    uint32_t off = (uint32_t)ne + block_exclusive_scan<uint32_t>((uint32_t)cnt, S.ssh, &tot);
-#pragma unroll
-                    for (int e = 0; e < E; e++)
-                        if (f[e]) T.elist[off++] = b0 + e;
-                    ne += (int32_t)tot;
-                }
-                __syncthreads();
-                if (tid == 0) T.bs[0] = 0;
-                for (int32_t i = tid; i < ne; i += kTinyBS) T.bs[i + 1] = A.vwgt[T.val[T.elist[i]]];
-                __syncthreads();
-                tiny_scan_i64(T.bs + 1, ne, S);
-                if (tid == 0) {
-                    int32_t start = 0;
-                    for (int32_t p = 0; p < k; p++) {
-                        T.es[p] = start;
-                        int64_t cap = maxwgt > T.pwgts[p] ? maxwgt - T.pwgts[p] : 0;
-                        int32_t end = start;
-                        if (cap > 0 && start < ne) {
-                            int64_t find = T.bs[start] + cap;
-                            int32_t lo = start, hi = (int32_t)min((int64_t)ne, (int64_t)start + cap);
-                            while (lo + 1 < hi) {
-                                int32_t mid = (lo + hi) / 2;
-                                if (T.bs[mid] >= find) hi = mid; else lo = mid;
-                            }
-                            int64_t dh = T.bs[hi] - find, dl = T.bs[lo] - find;
-                            dh = dh < 0 ? -dh : dh;
-                            dl = dl < 0 ? -dl : dl;
-                            end = dh < dl ? hi : lo;
-                        }
-                        T.ee[p] = end;
-                        start = end;
-                    }
-                }
-                __syncthreads();
-                for (int32_t i = tid; i < ne; i += kTinyBS) {
-                    int32_t lo = 0, hi = k - 1;
-                    while (lo < hi) {
-                        int32_t mid = (lo + hi + 1) >> 1;
-                        if (T.es[mid] <= i) lo = mid; else hi = mid - 1;
-                    }
-                    int32_t v = (int32_t)T.val[T.elist[i]];
-                    int32_t w = T.where[v];
-                    if (i < T.ee[lo] && lo != w) {
-                        A.dest[v] = lo;
-                        store_pair(A.pd16, A.pd32, v, w, lo);
-                    }
-                }
-            }
+            // RW / RS eviction (the selection's LDS is free again)
+            const RbView rv{n, k, A.key, A.vwgt, T.where, A.dest, A.pd16, A.pd32, T.pwgts, &C};
+            rb_block<R>(rv, T.sort_bits, T.bs, *(RbLds<R> *)dyn, part);
         }
         __syncthreads();
 
@@ -2295,14 +2227,56 @@ __device__ inline void jet_tiny_loop(const TinyArgs &T, int32_t *dyn, TinyShared
         for (int q = tid; q < k; q += kTinyBS) pdelta[q] = 0;
         __syncthreads();
         int64_t d2 = 0;
-        for (int32_t v = wv; v < n; v += kTinyWaves) {
+        auto weigh = [&](int32_t v, int32_t pv, int32_t dv) {
+            const int32_t wvv = A.vwgt[v];
+            atomicAdd(&pdelta[pv], (unsigned long long)(-(int64_t)wvv));
+            atomicAdd(&pdelta[dv], (unsigned long long)(int64_t)wvv);
+        };
+        for (int32_t i = tid; i < T.c0; i += kTinyBS) {
+            const int32_t v = T.ids[i], pv = T.where[v], dv = A.dest[v];
+            if (pv == dv) continue;
+            weigh(v, pv, dv);
+            const eid_t b = A.xadj[v];
+            int32_t u[kRowT], w[kRowT], pu[kRowT], du[kRowT];
+            load_short_row(A.adjncy, A.adjwgt, b, (int32_t)(A.xadj[v + 1] - b), u, w);
+            pq.gather(u, pu, du);
+#pragma unroll
+            for (int t = 0; t < kRowT; t++)
+                if (u[t] >= 0) d2 += move_d2(pv, dv, pu[t], du[t], w[t]);
+        }
+        for (int32_t i0 = T.c0 + grp; i0 < T.c1; i0 += R4 * kTinyGroups) {
+            int32_t v[R4], pv[R4], dv[R4], u[R4][E], w[R4][E];
+            eid_t b[R4], e[R4];
+#pragma unroll
+            for (int r = 0; r < R4; r++) v[r] = i0 + r * kTinyGroups < T.c1 ? T.ids[i0 + r * kTinyGroups] : -1;
+#pragma unroll
+            for (int r = 0; r < R4; r++) {
+                pv[r] = v[r] >= 0 ? T.where[v[r]] : 0;
+                dv[r] = v[r] >= 0 ? A.dest[v[r]] : 0;
+            }
+#pragma unroll
+            for (int r = 0; r < R4; r++) {
+                const bool moved = pv[r] != dv[r];
+                b[r] = moved ? A.xadj[v[r]] : 0;
+                e[r] = moved ? A.xadj[v[r] + 1] : 0;
+                if (moved && gl == 0) weigh(v[r], pv[r], dv[r]);
+            }
+#pragma unroll
+            for (int r = 0; r < R4; r++) load_entries<E, G>(A.adjncy, A.adjwgt, b[r], e[r], gl, u[r], w[r]);
+#pragma unroll
+            for (int r = 0; r < R4; r++) {
+                int32_t pu[E], du[E];
+                pq.gather(u[r], pu, du);
+#pragma unroll
+                for (int t = 0; t < E; t++)
+                    if (u[r][t] >= 0) d2 += move_d2(pv[r], dv[r], pu[t], du[t], w[r][t]);
+            }
+        }
+        for (int32_t i = T.c1 + wv; i < n; i += kTinyWaves) {
+            const int32_t v = T.ids[i];
             const int32_t pv = T.where[v], dv = A.dest[v];
             if (pv == dv) continue;
-            if (lane == 0) {
-                const int32_t wvv = A.vwgt[v];
-                atomicAdd(&pdelta[pv], (unsigned long long)(-(int64_t)wvv));
-                atomicAdd(&pdelta[dv], (unsigned long long)(int64_t)wvv);
-            }
+            if (lane == 0) weigh(v, pv, dv);
             const eid_t b = A.xadj[v], e = A.xadj[v + 1];
             for (eid_t c0 = b; c0 < e; c0 += kTinyRow) {
                 int32_t u[kTinyChunk], w[kTinyChunk], pu[kTinyChunk], du[kTinyChunk];
@@ -2343,11 +2317,12 @@ __device__ inline void jet_tiny_loop(const TinyArgs &T, int32_t *dyn, TinyShared
     }
 }
 
+template <int R>
 __global__ void __launch_bounds__(kTinyBS) k_jet_tiny(TinyArgs T)
 {
-    extern __shared__ int32_t dyn[];
+    extern __shared__ __align__(16) char dyn[];
     __shared__ TinyShared S;
-    jet_tiny_loop(T, dyn, S);
+    jet_tiny_loop<R>(T, dyn, tiny_work_lds<R>(T.A.k), S);
 }
 
 // ---------------------------------------------------------------- small levels of many graphs
@@ -2376,10 +2351,12 @@ struct TinyRunDev {
 // block per run: lock cleared, best = where, part weights, the control block
 // (k_jet_init), the narrow part copy, the Jet loop, where = best, the cut
 // carried to the next level, the projection.
+template <int NR>
 __global__ void __launch_bounds__(kTinyBS) k_jet_tiny_batch(const TinyRunDev *__restrict__ runs,
-                                                           const TinyStep *__restrict__ steps)
+                                                           const TinyStep *__restrict__ steps, int32_t kmax)
 {
-    extern __shared__ int32_t dyn[];
+    extern __shared__ __align__(16) char dyn[];
+    const size_t work = tiny_work_lds<NR>(kmax);
     __shared__ TinyShared S;
     __shared__ int64_t cut;
     const TinyRunDev &R = runs[blockIdx.x];
@@ -2430,7 +2407,7 @@ __global__ void __launch_bounds__(kTinyBS) k_jet_tiny_batch(const TinyRunDev *__
             C.filt_num = st.finest ? 1 : 3;
         }
         __syncthreads();
-        jet_tiny_loop(T, dyn, S);
+        jet_tiny_loop<NR>(T, dyn, work, S);
         for (int32_t v = tid; v < n; v += kTinyBS) T.where[v] = T.best[v];
         if (tid == 0) {
             cut = C.best_cut;
@@ -2557,28 +2534,23 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
         T.A = SelArgs{k,    g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, pwgts, lock, under, ctl,
                       dest, pregain, key, nullptr, wq, ab, pd16, pd32};
         T.n = n;
-        T.sort_bits = bits_for((uint64_t)k * kMaxBuckets);
+        T.sort_bits = bits_for((uint64_t)k * kMaxBuckets - 1);
+        T.ids = g.bins.ids;
+        T.c0 = (int32_t)g.bins.off[1];
+        T.c1 = (int32_t)g.bins.off[2];
         T.where = where;
         T.under = under;
         T.best = best;
-        T.pstart = c.arena.ralloc<int32_t>((size_t)k);
-        T.elist = c.arena.ralloc<int32_t>((size_t)n);
-        T.es = c.arena.ralloc<int32_t>((size_t)k);
-        T.ee = c.arena.ralloc<int32_t>((size_t)k);
         T.sel = sel;
         T.lock = lock;
         T.w8 = w8;
         T.w16 = w16;
-        T.val = c.arena.ralloc<uint32_t>((size_t)n);
-        T.k2 = c.arena.ralloc<uint32_t>((size_t)n);
-        T.v2 = c.arena.ralloc<uint32_t>((size_t)n);
         T.pwgts = pwgts;
-        T.wsc = c.arena.ralloc<int64_t>((size_t)n);
         T.bs = c.arena.ralloc<int64_t>((size_t)n + 1);
-        const size_t lds = tiny_lds(k);
         {
             KScope ks(c, "k_jet_tiny", 0.0);
-            k_jet_tiny<<<1, kTinyBS, lds, c.stream>>>(T);
+            if (n <= kTinyBS) k_jet_tiny<1><<<1, kTinyBS, tiny_lds<1>(k), c.stream>>>(T);
+            else k_jet_tiny<4><<<1, kTinyBS, tiny_lds<4>(k), c.stream>>>(T);   // (Tuning::tiny_max <= 4096)
             HGP_LAUNCH_CHECK();
         }
         read_scalars(c, ctl, sizeof(JetCtl));
@@ -2770,11 +2742,7 @@ TinyScratch alloc_tiny_scratch(Ctx &c, int32_t n, int32_t k)
     s.dest = c.arena.lalloc<int32_t>(N);
     s.pregain = c.arena.lalloc<int32_t>(N);
     s.best = c.arena.lalloc<int32_t>(N);
-    s.elist = c.arena.lalloc<int32_t>(N);
     s.under = c.arena.lalloc<int32_t>(K);
-    s.es = c.arena.lalloc<int32_t>(K);
-    s.ee = c.arena.lalloc<int32_t>(K);
-    s.pstart = c.arena.lalloc<int32_t>(K);
     s.iters = c.arena.lalloc<int32_t>(HGP_MAX_LEVELS);
     s.lock = c.arena.lalloc<uint8_t>(N);
     s.sel = c.arena.lalloc<uint8_t>(N);
@@ -2786,11 +2754,7 @@ TinyScratch alloc_tiny_scratch(Ctx &c, int32_t n, int32_t k)
         s.pd32 = c.arena.lalloc<uint32_t>(N);
     }
     s.key = c.arena.lalloc<uint32_t>(N);
-    s.val = c.arena.lalloc<uint32_t>(N);
-    s.k2 = c.arena.lalloc<uint32_t>(N);
-    s.v2 = c.arena.lalloc<uint32_t>(N);
     s.ab = c.arena.lalloc<uint64_t>(N);
-    s.wsc = c.arena.lalloc<int64_t>(N);
     s.bs = c.arena.lalloc<int64_t>(N + 1);
     s.pwgts = c.arena.lalloc<int64_t>(K);
     s.cut = c.arena.lalloc<int64_t>(1);
@@ -2804,7 +2768,7 @@ void tiny_batch(Ctx &c, const std::vector<TinyRun> &runs)
     if (runs.empty()) return;
     std::vector<TinyRunDev> rd;
     std::vector<TinyStep> sd;
-    int32_t kmax = 1;
+    int32_t kmax = 1, nmax = 1;
     for (const TinyRun &r : runs) {
         if (r.k > kTinyMaxK || r.k < 2) throw Error{-4, "tiny_batch: k out of range"};
         kmax = std::max(kmax, r.k);
@@ -2829,24 +2793,20 @@ void tiny_batch(Ctx &c, const std::vector<TinyRun> &runs)
                           s.under,  (JetCtl *)s.ctl, s.dest, s.pregain, s.key, nullptr, NarrowParts{s.w8, s.w16},
                           s.ab, s.pd16, s.pd32};
             T.n = g.n;
-            T.sort_bits = bits_for((uint64_t)r.k * kMaxBuckets);
+            T.sort_bits = bits_for((uint64_t)r.k * kMaxBuckets - 1);
+            T.ids = g.bins.ids;
+            T.c0 = (int32_t)g.bins.off[1];
+            T.c1 = (int32_t)g.bins.off[2];
             T.where = where;
             T.under = s.under;
             T.best = s.best;
-            T.pstart = s.pstart;
-            T.elist = s.elist;
-            T.es = s.es;
-            T.ee = s.ee;
             T.sel = s.sel;
             T.lock = s.lock;
             T.w8 = s.w8;
             T.w16 = s.w16;
-            T.val = s.val;
-            T.k2 = s.k2;
-            T.v2 = s.v2;
             T.pwgts = s.pwgts;
-            T.wsc = s.wsc;
             T.bs = s.bs;
+            nmax = std::max(nmax, g.n);
             st.finest = l == 0;
             if (l > 0 && (l > r.lo || r.lo > 0)) {
                 st.cmap_fine = r.cmap[(size_t)l - 1];
@@ -2871,7 +2831,9 @@ void tiny_batch(Ctx &c, const std::vector<TinyRun> &runs)
     HGP_CHECK_HIP(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, c.stream));
     {
         KScope ks(c, "k_jet_tiny_batch", 0.0);
-        k_jet_tiny_batch<<<(unsigned)rd.size(), kTinyBS, tiny_lds(kmax), c.stream>>>(drun, dstep);
+        const unsigned nb = (unsigned)rd.size();
+        if (nmax <= 8 * kTinyBS) k_jet_tiny_batch<8><<<nb, kTinyBS, tiny_lds<8>(kmax), c.stream>>>(drun, dstep, kmax);
+        else k_jet_tiny_batch<16><<<nb, kTinyBS, tiny_lds<16>(kmax), c.stream>>>(drun, dstep, kmax);
         HGP_LAUNCH_CHECK();
     }
     HGP_CHECK_HIP(hipStreamSynchronize(c.stream));
