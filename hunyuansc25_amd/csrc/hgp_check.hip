@@ -9,13 +9,18 @@
 // pass proves the offsets monotone before the entry pass reads any row, so a
 // malformed xadj never sends a kernel outside adjncy.
 //
-// Entries are walked in tiles of kEPT x 64 consecutive entries, one tile per
-// wave: lane l takes entries l, l + 64, ... (each load instruction reads 64
-// consecutive entries).  Two lanes find the rows of the tile's ends by a
-// binary search over xadj; every lane then finds the row of its first entry
-// by a search between those two rows (a few cached lines) and follows the
-// rows forward, so hub rows cost no more than short ones and xadj is read
-// about once.
+// Entries are walked in tiles of kEPT x 64 consecutive entries; a wave walks
+// consecutive tiles, lane l taking entries l, l + 64, ... of each (each load
+// instruction reads 64 consecutive entries).  The wave finds the row of its
+// first entry by a 64-way search, then counts the row starts at each entry of
+// a tile in LDS and scans the counts, so every lane knows the rows of its
+// entries and the wave goes over xadj once, 64 rows a load.  Following the
+// rows one by one after a binary search per tile, chains of dependent reads,
+// bounded both walks: R-MAT with 2^22 vertices and 52M entries is checked in
+// 0.19 ms (1.0 ms so; 2.2 TB/s now), R-MAT with 2^20 vertices and 33M entries
+// evaluated in 0.24 ms (0.47 ms so; the part gathers, at 190 G/s at best, take
+// 0.18 ms of it).  16 entries a lane take registers the occupancy needs: 0.25
+// ms for the check.
 #include "hgp_check.hpp"
 #include "hgp_host.hpp"
 
@@ -28,46 +33,50 @@ namespace hgp {
 namespace {
 
 constexpr int kChkBS = 256;
-constexpr int kEPT = 16;                        // entries per lane and tile
+constexpr int kEPT = 16;                     // entries per lane and tile
 constexpr int64_t kWaveTile = (int64_t)kWave * kEPT;
 constexpr int64_t kTile = (int64_t)kChkBS * kEPT;
 constexpr unsigned kEntryGrid = 2048;           // grid of the entry walkers (grid-stride)
 
-// Row v with xadj[v] <= e < xadj[v + 1] (xadj monotone, xadj[0] = 0, e < xadj[n]).
+// Row v with xadj[v] <= e < xadj[v + 1] (xadj monotone, xadj[0] = 0, e <
+// xadj[n]); all lanes of a wave call it with the same e.
 __device__ inline int32_t row_of(const eid_t *__restrict__ xadj, int32_t n, int64_t e)
 {
-    int32_t lo = 0, hi = n;
-    while (hi - lo > 1) {
-        int32_t mid = lo + (hi - lo) / 2;
-        if (xadj[mid] <= e) lo = mid; else hi = mid;
+    int32_t lo = 0, len = n;   // the row is in [lo, lo + len)
+    while (len > 1) {
+        const int32_t step = (len - 1) / kWave + 1;
+        const int64_t o = (int64_t)lane_id() * step;
+        const bool below = o < len && (o == 0 || xadj[lo + o] <= e);
+        const int c = __popcll(__ballot(below)) - 1;
+        lo += c * step;
+        len = min(step, len - c * step);
     }
     return lo;
 }
 
-// Calls f(v, j) for this lane's entries j of the wave's tile [t0, t1)
-// (t0 + lane, t0 + lane + 64, ...; row v).  Every lane of the wave must call
-// it.  The row index stays in [0, n - 1], whatever xadj holds.
-template <class F>
-__device__ inline void walk_tile(const eid_t *__restrict__ xadj, int32_t n, int64_t t0, int64_t t1, F f)
+// Counts the rows that start at each of the len entries from t0 on into starts
+// (kWaveTile words of LDS of the wave's own).  The rows (r, n) are looked at,
+// r the row of the entry before t0 (or of t0 itself); returns the row of the
+// last entry.  Each row counts at most once, so r plus the starts up to an
+// entry, the entry's row, stays below n whatever xadj holds.
+__device__ inline int32_t row_starts(const eid_t *__restrict__ xadj, int32_t n, int64_t t0, int64_t len,
+                                     int32_t r, uint32_t *starts)
 {
     const int lane = lane_id();
-    int32_t r = 0;
-    if (lane == 0) r = row_of(xadj, n, t0);
-    if (lane == 1) r = row_of(xadj, n, t1 - 1);
-    const int32_t r0 = __shfl(r, 0, kWave), r1 = __shfl(r, 1, kWave);
-    int64_t j = t0 + lane;
-    if (j >= t1) return;
-    int32_t lo = r0, hi = r1 + 1;   // the row of j lies in [r0, r1] when xadj is monotone
-    while (hi - lo > 1) {
-        const int32_t mid = lo + (hi - lo) / 2;
-        if (xadj[mid] <= j) lo = mid; else hi = mid;
+#pragma unroll
+    for (int t = 0; t < kEPT; t++) starts[t * kWave + lane] = 0;
+    wave_lds_sync();
+    while (r < n - 1) {
+        const int left = min(n - 1 - r, kWave);
+        const eid_t s = lane < left ? xadj[r + 1 + lane] - t0 : len;
+        const uint64_t past = __ballot(s >= len);
+        const int c = past ? __ffsll((unsigned long long)past) - 1 : kWave;
+        if (lane < c && s >= 0) atomicAdd(&starts[s], 1u);
+        r += c;
+        if (c < kWave) break;
     }
-    int32_t v = lo;
-    eid_t nx = xadj[v + 1];
-    for (; j < t1; j += kWave) {
-        while (nx <= j && v < n - 1) nx = xadj[++v + 1];
-        f(v, j);
-    }
+    wave_lds_sync();
+    return r;
 }
 
 template <class T>
@@ -120,23 +129,41 @@ __global__ void __launch_bounds__(kChkBS) k_check_entries(int32_t n, int64_t m, 
                                                          const wgt_t *__restrict__ adjwgt, int symmetric,
                                                          CheckState *s)
 {
+    __shared__ uint32_t starts[kChkBS / kWave][kWaveTile];
     uint64_t wsum = 0, h0 = 0, h1 = 0;
-    const int64_t wave = (int64_t)blockIdx.x * (kChkBS / kWave) + threadIdx.x / kWave;
-    for (int64_t t0 = wave * kWaveTile; t0 < m; t0 += (int64_t)gridDim.x * kTile) {
+    const int w0 = threadIdx.x / kWave, lane = lane_id();
+    const int64_t wave = (int64_t)blockIdx.x * (kChkBS / kWave) + w0;
+    const int64_t tiles = (m + kWaveTile - 1) / kWaveTile;
+    const int64_t per = (tiles + (int64_t)gridDim.x * (kChkBS / kWave) - 1) / ((int64_t)gridDim.x * (kChkBS / kWave));
+    const int64_t end = min((wave + 1) * per * kWaveTile, m);
+    int32_t r = wave * per * kWaveTile < end ? row_of(xadj, n, wave * per * kWaveTile) : 0;
+    for (int64_t t0 = wave * per * kWaveTile; t0 < end; t0 += kWaveTile) {
         const int64_t t1 = min(t0 + kWaveTile, m);
-        walk_tile(xadj, n, t0, t1, [&](int32_t v, int64_t j) {
-            int32_t u = adjncy[j];
-            int32_t w = adjwgt ? adjwgt[j] : 1;
-            if (u < 0 || u >= n) atomicMin(&s->first[kChkNeighbour], (unsigned long long)v);
-            else if (u == v) atomicMin(&s->first[kChkSelfLoop], (unsigned long long)v);
-            if (w < 1) atomicMin(&s->first[kChkAdjwgt], (unsigned long long)v);
-            wsum += (uint64_t)(int64_t)w;
-            if (symmetric && u >= 0 && u < n && u != v) {
+        int32_t u[kEPT], w[kEPT];
+#pragma unroll
+        for (int t = 0; t < kEPT; t++) {
+            const int64_t j = t0 + t * kWave + lane;
+            u[t] = j < t1 ? __builtin_nontemporal_load(adjncy + j) : 0;
+            w[t] = j < t1 ? (adjwgt ? __builtin_nontemporal_load(adjwgt + j) : 1) : 0;
+        }
+        uint32_t row = r;
+        r = row_starts(xadj, n, t0, t1 - t0, r, starts[w0]);
+#pragma unroll
+        for (int t = 0; t < kEPT; t++) {
+            const uint32_t x = wave_inclusive_scan(starts[w0][t * kWave + lane]) + row;
+            row = wave_read(x, kWave - 1);
+            if (t0 + t * kWave + lane >= t1) continue;
+            const int32_t v = (int32_t)x;
+            if (u[t] < 0 || u[t] >= n) atomicMin(&s->first[kChkNeighbour], (unsigned long long)v);
+            else if (u[t] == v) atomicMin(&s->first[kChkSelfLoop], (unsigned long long)v);
+            if (w[t] < 1) atomicMin(&s->first[kChkAdjwgt], (unsigned long long)v);
+            wsum += (uint64_t)(int64_t)w[t];
+            if (symmetric && u[t] >= 0 && u[t] < n && u[t] != v) {
                 uint64_t a, b;
-                edge_hashes(min(u, v), max(u, v), w, a, b);
-                if (v < u) { h0 += a; h1 += b; } else { h0 -= a; h1 -= b; }
+                edge_hashes(min(u[t], v), max(u[t], v), w[t], a, b);
+                if (v < u[t]) { h0 += a; h1 += b; } else { h0 -= a; h1 -= b; }
             }
-        });
+        }
     }
     wsum = block_sum(wsum);
     h0 = block_sum(h0);
@@ -157,7 +184,9 @@ __global__ void k_eval_clear(int64_t *scr, int32_t k)
         scr[i] = 0;
 }
 
-// Part weights: LDS bins per block, one atomic per block and touched part;
+// Part weights: LDS bins per block, one atomic per block and touched part (so
+// few blocks: atomics on one line follow each other at 12 ns each; 256 parts
+// and 2^20 vertices take 16 us with 256 blocks, 34 us with 1024);
 // vertices whose part id is outside [0, k) are counted instead.
 __global__ void __launch_bounds__(kChkBS) k_eval_vertices(int32_t n, int32_t k, const wgt_t *__restrict__ vwgt,
                                                          const int32_t *__restrict__ part, int64_t *scr)
@@ -186,18 +215,39 @@ __global__ void __launch_bounds__(kChkBS) k_eval_entries(int32_t n, const eid_t 
                                                         const wgt_t *__restrict__ adjwgt,
                                                         const int32_t *__restrict__ part, int64_t *scr)
 {
+    __shared__ uint32_t starts[kChkBS / kWave][kWaveTile];
     const int64_t m = xadj[n];
     uint64_t cut = 0, bad = 0;
-    const int64_t wave = (int64_t)blockIdx.x * (kChkBS / kWave) + threadIdx.x / kWave;
-    for (int64_t t0 = wave * kWaveTile; t0 < m; t0 += (int64_t)gridDim.x * kTile) {
+    const int w0 = threadIdx.x / kWave, lane = lane_id();
+    const int64_t wave = (int64_t)blockIdx.x * (kChkBS / kWave) + w0;
+    const int64_t tiles = (m + kWaveTile - 1) / kWaveTile;
+    const int64_t per = (tiles + (int64_t)gridDim.x * (kChkBS / kWave) - 1) / ((int64_t)gridDim.x * (kChkBS / kWave));
+    const int64_t end = min((wave + 1) * per * kWaveTile, m);
+    int32_t r = wave * per * kWaveTile < end ? row_of(xadj, n, wave * per * kWaveTile) : 0;
+    for (int64_t t0 = wave * per * kWaveTile; t0 < end; t0 += kWaveTile) {
         const int64_t t1 = min(t0 + kWaveTile, m);
-        int32_t pv = -1, cv = -1;
-        walk_tile(xadj, n, t0, t1, [&](int32_t v, int64_t j) {
-            if (v != cv) { cv = v; pv = part[v]; }
-            int32_t u = adjncy[j];
-            if (u < 0 || u >= n) { bad++; return; }
-            if (part[u] != pv) cut += (uint64_t)(int64_t)(adjwgt ? adjwgt[j] : 1);
-        });
+        int32_t u[kEPT], w[kEPT];
+        bool in[kEPT];
+#pragma unroll
+        for (int t = 0; t < kEPT; t++) {
+            const int64_t j = t0 + t * kWave + lane;
+            u[t] = j < t1 ? __builtin_nontemporal_load(adjncy + j) : 0;
+            w[t] = j < t1 ? (adjwgt ? __builtin_nontemporal_load(adjwgt + j) : 1) : 0;
+        }
+#pragma unroll
+        for (int t = 0; t < kEPT; t++) {   // the neighbours' parts are on their way while the rows are found
+            in[t] = u[t] >= 0 && u[t] < n;
+            bad += in[t] ? 0 : 1;
+            u[t] = in[t] ? part[u[t]] : 0;
+        }
+        uint32_t row = r;
+        r = row_starts(xadj, n, t0, t1 - t0, r, starts[w0]);
+#pragma unroll
+        for (int t = 0; t < kEPT; t++) {
+            const uint32_t x = wave_inclusive_scan(starts[w0][t * kWave + lane]) + row;
+            row = wave_read(x, kWave - 1);
+            if (in[t] && u[t] != part[x]) cut += (uint64_t)(int64_t)w[t];
+        }
     }
     cut = block_sum(cut);
     bad = block_sum(bad);
@@ -252,7 +302,7 @@ void evaluate_launch(hipStream_t st, int32_t n, const eid_t *xadj, const vid_t *
     k_eval_clear<<<grid_for(kEvalHead + (int64_t)k, kChkBS), kChkBS, 0, st>>>(scr, k);
     HGP_LAUNCH_CHECK();
     if (n > 0) {
-        unsigned gv = (unsigned)std::min<int64_t>(((int64_t)n + kChkBS - 1) / kChkBS, 1024);
+        unsigned gv = (unsigned)std::min<int64_t>(((int64_t)n + kChkBS - 1) / kChkBS, 256);
         k_eval_vertices<<<gv, kChkBS, sizeof(unsigned long long) * (size_t)k, st>>>(n, k, vwgt, part, scr);
         HGP_LAUNCH_CHECK();
         k_eval_entries<<<kEntryGrid, kChkBS, 0, st>>>(n, xadj, adjncy, adjwgt, part, scr);

@@ -156,3 +156,30 @@ def test_evaluate_rejects(hgp, torch_mod):
     with pytest.raises(hgp.HgpError) as e:
         hgp.evaluate_device(6, *(t.data_ptr() for t in d), 0, out.data_ptr())
     assert e.value.code == -1
+
+
+@pytest.mark.parametrize("shape", ["edges", "empties", "hub", "one"])
+def test_rows_at_tile_edges(hgp, torch_mod, shape):
+    """Rows that start and end at the borders of the 64- and 512-entry pieces
+    the walkers take, runs of more than 64 empty rows, a row over several
+    pieces: the check names the right vertex, the evaluation the right cut."""
+    lens = {"edges": [512, 511, 1, 513, 511, 64, 63, 1, 65, 447, 512, 1024, 1],
+            "empties": [0] * 70 + [3] + [0] * 200 + [509] + [0] * 64 + [512, 1] + [0] * 130 + [7] + [0] * 65,
+            "hub": [5, 300000, 2, 0, 1], "one": [1, 1]}[shape]
+    n = len(lens)
+    x = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    row = np.repeat(np.arange(n), lens)
+    rng = np.random.default_rng(7)
+    a = ((row + 1 + rng.integers(0, n - 1, size=len(row))) % n).astype(np.int32)
+    aw = rng.integers(1, 9, size=len(row)).astype(np.int32)
+    vw = np.ones(n, np.int32)
+    where = rng.integers(0, 3, size=n).astype(np.int32)
+    d = _dev(torch_mod, x, a, vw, aw, where)
+    out = torch_mod.zeros(4, dtype=torch_mod.int64, device="cuda:0")
+    hgp.evaluate_device(n, *(_ptr(d[i]) for i in (0, 1, 3, 2, 4)), 3, out.data_ptr())
+    cut = int(aw[where[row] != where[a]].sum()) // 2
+    assert out.tolist() == [cut, int(np.bincount(where, minlength=3).max()), 0, 0]
+    for j in sorted({0, len(a) // 3, len(a) - 1, *(x[1:-1] - 1).clip(0).tolist(), *x[x < len(a)].tolist()})[:12]:
+        bad = aw.copy()
+        bad[j] = 0
+        _expect_check(hgp, torch_mod, x, a, vw, bad, False, f"edge weight < 1 in row {row[j]}")
