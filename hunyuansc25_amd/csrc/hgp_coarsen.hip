@@ -70,6 +70,87 @@ __device__ inline bool keeps_proposal(int32_t first, int32_t v, const int32_t *_
     return u >= 0 && avail[u] >= 0;
 }
 
+// The entries of one row in the order of BetterEdge: weight and hash in one
+// word (0: no edge), ties to the smaller neighbour (the edges share v, so
+// (lo, hi) ascends with the neighbour).
+struct RowBest {
+    uint64_t k = 0;
+    int32_t u = 0;
+};
+
+struct BetterRow {
+    __device__ bool operator()(const RowBest &a, const RowBest &b) const
+    {
+        return a.k > b.k || (a.k == b.k && a.k != 0 && a.u < b.u);
+    }
+};
+
+__device__ inline EdgeKey row_edge(const RowBest &b, int32_t v)
+{
+    if (b.k == 0) return EdgeKey{-1, 0, 0, 0u};
+    return EdgeKey{(int32_t)((b.k >> 32) - 1), min(b.u, v), max(b.u, v), (uint32_t)b.k};
+}
+
+// Improves best (the same in the G lanes of a group) with T entries per lane of
+// row v.  Whether a neighbour is free takes a gather, and the L2 answers 160 of
+// them a ns where 500 entries are streamed, but the order of the entries does
+// not need them: the group's best entry is looked up alone, and only when
+// `tries` of them were not free the lanes look up all their entries that would
+// improve best.  In a level's first round most neighbours are free (first
+// rounds of R-MAT with 2^22 vertices, rows of > 512 entries: 746 -> 179 us, of
+// 33..512 entries: 472 -> 254 us); later the long rows still gain from one try
+// (166 -> 107 us), the others do not (two tries: 259 -> 294 us), nor do rows
+// of one lane, whose few lookups go out together (23 against 27 us).
+template <int T, int G>
+__device__ inline void improve_best(RowBest &best, const int32_t (&u)[T], const int32_t (&w)[T], int32_t v, int32_t wv,
+                                    uint64_t s1, uint64_t tv, const int32_t *__restrict__ avail, int32_t maxvwgt, int tries)
+{
+    auto reduce = [](const RowBest &x) {
+        if constexpr (G == 1) return x;
+        else return group_best<G>(x, BetterRow());
+    };
+    uint64_t key[T];
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+        key[t] = 0;
+        if (u[t] >= 0 && u[t] != v && w[t] >= 0)
+            key[t] = (uint64_t)((uint32_t)w[t] + 1u) << 32 | edge_hash_row(s1, tv, v, u[t]);
+    }
+    bool open = true;   // the same in the group
+    for (int i = 0; i < tries; i++) {
+        RowBest m;
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+            const RowBest x{key[t], u[t]};
+            if (BetterRow()(x, m)) m = x;
+        }
+        m = reduce(m);
+        open = open && BetterRow()(m, best);
+        if (open) {
+            const int32_t a = avail[m.u];
+            if (a >= 0 && (int64_t)a + wv < maxvwgt) {
+                best = m;
+                open = false;
+            }
+        }
+        if (!__any(open)) return;
+#pragma unroll
+        for (int t = 0; t < T; t++)
+            if (open && u[t] == m.u) key[t] = 0;
+    }
+    RowBest m;
+    int32_t wu[T];
+#pragma unroll
+    for (int t = 0; t < T; t++) wu[t] = open && BetterRow()(RowBest{key[t], u[t]}, best) ? avail[u[t]] : -1;
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+        const RowBest x{wu[t] >= 0 && (int64_t)wu[t] + wv < maxvwgt ? key[t] : 0, u[t]};
+        if (BetterRow()(x, m)) m = x;
+    }
+    m = reduce(m);
+    if (BetterRow()(m, best)) best = m;
+}
+
 // Handshake proposal (replaces random_match_conflict, hunyuangraph_GPU_match.h:454-510,
 // and set_receive_send_topk_one, :800-861): every free vertex proposes to its
 // best free neighbour u with vwgt[u]+vwgt[v] < maxvwgt.  G lanes per row.
@@ -94,29 +175,20 @@ __global__ void __launch_bounds__(kRowBS) k_propose(const int32_t *__restrict__ 
         } else if (keeps_proposal(first, v, avail, prop)) {
             kbytes = 0;
         } else {
-            EdgeKey best{-1, 0, 0, 0u};
+            RowBest best;
             eid_t beg = xadj[v], end = xadj[v + 1];
             const uint64_t tv = mix64(s1 ^ (uint64_t)(uint32_t)v);
             // entries per lane and phase: a whole class-w row for a wave, a whole
             // class-m row for a 16-lane group, one entry otherwise
             constexpr int T = G == kWave ? (int)(kBinMid / kWave) : (G == 16 ? (int)(kBinHalf / 16) : 1);
             for (eid_t c0 = beg; c0 < end; c0 += (eid_t)T * G) {
-                int32_t u[T], w[T], wu[T];
+                int32_t u[T], w[T];
                 load_entries<T, G>(adjncy, adjwgt, c0, end, lane, u, w);
-                gather_slots<T>(avail, u, wu, -1);
-#pragma unroll
-                for (int t = 0; t < T; t++) {
-                    if (u[t] < 0 || u[t] == v || wu[t] < 0) continue;
-                    if ((int64_t)wu[t] + wv >= maxvwgt) continue;
-                    EdgeKey e{w[t], u[t] < v ? u[t] : v, u[t] < v ? v : u[t], 0u};
-                    e.h = edge_hash_row(s1, tv, v, u[t]);
-                    if (BetterEdge()(e, best)) best = e;
-                }
+                improve_best<T, G>(best, u, w, v, wv, s1, tv, avail, maxvwgt, first ? 2 : 0);
             }
-            best = group_best<G>(best, BetterEdge());
             if (lane == 0) {
-                prop[v] = best.w < 0 ? -1 : (best.lo == v ? best.hi : best.lo);
-                kbytes = 16 + 12 * (uint64_t)(end - beg);   // xadj; adjncy, adjwgt, avail[u]
+                prop[v] = best.k == 0 ? -1 : best.u;
+                kbytes = 16 + 8 * (uint64_t)(end - beg);   // xadj; adjncy, adjwgt
             }
         }
     }
@@ -148,7 +220,7 @@ __global__ void __launch_bounds__(kRowBS) k_propose_t(const int32_t *__restrict_
             const eid_t b = xadj[v];
             const int32_t d = (int32_t)(xadj[v + 1] - b);
             const uint64_t tv = mix64(s1 ^ (uint64_t)(uint32_t)v);
-            int32_t u[T], w[T], wu[T];
+            int32_t u[T], w[T];
 #pragma unroll
             for (int t = 0; t < T; t++) {
                 u[t] = -1;
@@ -158,18 +230,10 @@ __global__ void __launch_bounds__(kRowBS) k_propose_t(const int32_t *__restrict_
                     w[t] = adjwgt[b + t];
                 }
             }
-            gather_slots<T>(avail, u, wu, -1);
-            EdgeKey best{-1, 0, 0, 0u};
-#pragma unroll
-            for (int t = 0; t < T; t++) {
-                if (u[t] < 0 || u[t] == v || wu[t] < 0) continue;
-                if ((int64_t)wu[t] + wv >= maxvwgt) continue;
-                EdgeKey e{w[t], u[t] < v ? u[t] : v, u[t] < v ? v : u[t], 0u};
-                e.h = edge_hash_row(s1, tv, v, u[t]);
-                if (BetterEdge()(e, best)) best = e;
-            }
-            prop[v] = best.w < 0 ? -1 : (best.lo == v ? best.hi : best.lo);
-            kbytes = 16 + 12 * (uint64_t)d;
+            RowBest best;
+            improve_best<T, 1>(best, u, w, v, wv, s1, tv, avail, maxvwgt, 0);
+            prop[v] = best.k == 0 ? -1 : best.u;
+            kbytes = 16 + 8 * (uint64_t)d;
         }
     }
     kb_flush(kb, kbytes);
@@ -203,28 +267,20 @@ __global__ void __launch_bounds__(kSegBlk) k_propose_seg(RowSegs S, const eid_t 
             const EdgeKey sb = sbest[s];
             if (sb.w < 0 || avail[sb.lo == v ? sb.hi : sb.lo] >= 0) continue;
         }
-        EdgeKey best{-1, 0, 0, 0u};
+        RowBest rb;   // of the wave's entries
         eid_t j0 = S.j0[s], j1 = min(j0 + (eid_t)kSegLen, xadj[v + 1]);
         const uint64_t tv = mix64(s1 ^ (uint64_t)(uint32_t)v);
         constexpr int T = 8;   // entries per thread and phase
         for (eid_t c0 = j0; c0 < j1; c0 += (eid_t)T * kSegBlk) {
-            int32_t u[T], w[T], wu[T];
+            int32_t u[T], w[T];
             load_entries<T, kSegBlk>(adjncy, adjwgt, c0, j1, threadIdx.x, u, w);
-            gather_slots<T>(avail, u, wu, -1);
-#pragma unroll
-            for (int t = 0; t < T; t++) {
-                if (u[t] < 0 || u[t] == v || wu[t] < 0) continue;
-                if ((int64_t)wu[t] + wv >= maxvwgt) continue;
-                EdgeKey e{w[t], u[t] < v ? u[t] : v, u[t] < v ? v : u[t], 0u};
-                e.h = edge_hash_row(s1, tv, v, u[t]);
-                if (BetterEdge()(e, best)) best = e;
-            }
+            improve_best<T, kWave>(rb, u, w, v, wv, s1, tv, avail, maxvwgt, first ? 2 : 1);
         }
-        best = group_best<kSegBlk>(best, BetterEdge());
+        const EdgeKey best = group_best<kSegBlk>(row_edge(rb, v), BetterEdge());
         if (threadIdx.x == 0) {
             if (mi < 0) prop[v] = best.w < 0 ? -1 : (best.lo == v ? best.hi : best.lo);
             else sbest[s] = best;
-            kbytes += 8 + 12 * (uint64_t)(j1 - j0);   // xadj[v+1]; adjncy, adjwgt, avail[u]
+            kbytes += 8 + 8 * (uint64_t)(j1 - j0);   // xadj[v+1]; adjncy, adjwgt
         }
     }
     kb_flush(kb, kbytes);
