@@ -58,6 +58,7 @@ class Arena {
     void free_block();                   // return the block to HIP (nothing may be live)
     size_t capacity() const { return cap_; }
     size_t high_water() const { return peak_; }
+    size_t free_bytes() const { return hi_ - lo_; }
     char *base() const { return base_; }  // left allocations start here (left_mark() bytes in use)
 
     template <class T> T *lalloc(size_t n) { return (T *)left(sizeof(T) * (n ? n : 1)); }

@@ -42,13 +42,113 @@ struct NarrowParts {
     }
 };
 
+// Hot part ids.  The selection is bound by its neighbour gathers: the L2
+// answers 160 G random requests/s, whatever their size, and R-MAT rows hardly
+// share lines.  A block that keeps the narrow parts of kHotBytes worth of
+// vertices in LDS answers most of them itself: the 65536 heaviest rows of
+// R-MAT with 2^22 vertices receive 62% of its entries, a level with at most
+// that many vertices is held whole.  On larger levels the narrow copy is kept
+// in another order, hot vertices first, and the selection reads a copy of
+// adjncy that holds the positions:
+//   position(v) = rank among the hot vertices, or cap + rank among the others,
+// both in vertex order.  A cell holds the hot bits of 32 vertices and the
+// hot vertices before them.
+constexpr size_t kHotBytes = 65536;
+struct HotOrder {
+    const uint2 *cells = nullptr;   // null: position(v) = v
+    int32_t cap = 0;
+    __device__ int32_t position(int32_t v) const
+    {
+        if (!cells) return v;
+        const uint2 x = cells[v >> 5];
+        const uint32_t bit = 1u << (v & 31);
+        const int32_t r = (int32_t)x.y + __popc(x.x & (bit - 1));
+        return x.x & bit ? r : cap + v - r;
+    }
+};
+
+constexpr int kHotBuckets = 256;
+constexpr int kHotBS = 1024;
+
+// Degree buckets, eight per octave, monotone in d.
+__device__ inline int hot_bucket(int64_t d)
+{
+    if (d < 1) return 0;
+    const uint32_t f = __float_as_uint((float)d) >> 20;
+    return min((int)(f - (127u << 3)) + 1, kHotBuckets - 1);
+}
+
+__global__ void __launch_bounds__(kHotBS) k_hot_hist(int32_t n, const eid_t *__restrict__ xadj, int32_t *__restrict__ hist)
+{
+    __shared__ int32_t h[kHotBuckets];
+    for (int i = threadIdx.x; i < kHotBuckets; i += kHotBS) h[i] = 0;
+    __syncthreads();
+    for (int64_t v = (int64_t)blockIdx.x * kHotBS + threadIdx.x; v < n; v += (int64_t)gridDim.x * kHotBS)
+        atomicAdd(&h[hot_bucket(xadj[v + 1] - xadj[v])], 1);
+    __syncthreads();
+    for (int i = threadIdx.x; i < kHotBuckets; i += kHotBS)
+        if (h[i]) atomicAdd(&hist[i], h[i]);
+}
+
+// thr = the lowest bucket with at most cap vertices in it and above.
+__global__ void __launch_bounds__(kHotBuckets) k_hot_pick(const int32_t *__restrict__ hist, int32_t cap, int32_t *thr)
+{
+    __shared__ int32_t h[kHotBuckets];
+    h[threadIdx.x] = hist[threadIdx.x];
+    __syncthreads();
+    int64_t above = 0;
+    for (int b = threadIdx.x; b < kHotBuckets; b++) above += h[b];
+    const int t = __syncthreads_count(above > cap);
+    if (threadIdx.x == 0) *thr = t;
+}
+
+__global__ void __launch_bounds__(kBS) k_hot_bits(int32_t n, const eid_t *__restrict__ xadj,
+                                                  const int32_t *__restrict__ thr, uint2 *__restrict__ cells,
+                                                  int32_t *__restrict__ cnt)
+{
+    const int64_t v = (int64_t)blockIdx.x * kBS + threadIdx.x;
+    const uint64_t b = __ballot(v < n && hot_bucket(xadj[min(v, (int64_t)n - 1) + 1] - xadj[min(v, (int64_t)n - 1)]) >= *thr);
+    if (v < n && (v & 31) == 0) {
+        const uint32_t bits = (uint32_t)(b >> (threadIdx.x & 32));
+        cells[v >> 5].x = bits;
+        cnt[v >> 5] = __popc(bits);
+    }
+}
+
+__global__ void __launch_bounds__(kBS) k_hot_cells(int32_t ncell, const int32_t *__restrict__ before, uint2 *__restrict__ cells)
+{
+    const int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x;
+    if (i < ncell) cells[i].y = (uint32_t)before[i];
+}
+
+__global__ void __launch_bounds__(kBS) k_hot_codes(int64_t m, const vid_t *__restrict__ adjncy, HotOrder ho,
+                                                   vid_t *__restrict__ code)
+{
+    constexpr int T = 8;
+    const int64_t j0 = (int64_t)blockIdx.x * kBS * T + threadIdx.x;
+    int32_t u[T];
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+        const int64_t j = j0 + (int64_t)t * kBS;
+        u[t] = j < m ? __builtin_nontemporal_load(adjncy + j) : 0;
+    }
+#pragma unroll
+    for (int t = 0; t < T; t++) u[t] = ho.position(u[t]);
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+        const int64_t j = j0 + (int64_t)t * kBS;
+        if (j < m) __builtin_nontemporal_store(u[t], code + j);
+    }
+}
+
 __global__ void k_narrow(int32_t n, const int32_t *__restrict__ src, uint8_t *__restrict__ d8,
-                         uint16_t *__restrict__ d16)
+                         uint16_t *__restrict__ d16, HotOrder ho)
 {
     int32_t v = (int32_t)((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
     if (v >= n) return;
-    if (d8) d8[v] = (uint8_t)src[v];
-    else d16[v] = (uint16_t)src[v];
+    const int32_t x = ho.position(v);
+    if (d8) d8[x] = (uint8_t)src[v];
+    else d16[x] = (uint16_t)src[v];
 }
 
 // where and dest of a vertex packed into one word (8 bits each for k <= 256,
@@ -326,7 +426,38 @@ struct SelArgs {
     uint64_t *ab;             // LP: the afterburner's (pregain, where, dest) records
     uint16_t *pd16;           // RW/RS: (where, dest) words of the move accounting
     uint32_t *pd32;
+    int32_t hot = 0;          // positions below hot are held in LDS by the kernels that do so
+    int32_t held = 0;         // and this many of them exist
 };
+
+// The hot part ids in LDS (tab: kHotBytes); every thread of the block calls
+// load_hot.  Slots past the row hold -1, as in NarrowParts.
+__device__ inline void load_hot(const SelArgs &A, uint32_t *tab)
+{
+    const uint4 *src = (const uint4 *)(A.wq.p8 ? (const void *)A.wq.p8 : (const void *)A.wq.p16);
+    const int words = (int)(((size_t)A.held * (A.wq.p8 ? 1 : 2) + 15) / 16);
+    for (int i = threadIdx.x; i < words; i += blockDim.x) ((uint4 *)tab)[i] = src[i];
+    __syncthreads();
+}
+
+template <int T>
+__device__ inline void hot_gather(const SelArgs &A, const uint32_t *tab, const int32_t (&u)[T], int32_t (&q)[T])
+{
+    const uint32_t hot = (uint32_t)A.hot;
+    if (A.wq.p8) {
+#pragma unroll
+        for (int t = 0; t < T; t++) q[t] = u[t] >= (int32_t)hot ? (int32_t)A.wq.p8[u[t]] : -1;
+#pragma unroll
+        for (int t = 0; t < T; t++)
+            if ((uint32_t)u[t] < hot) q[t] = ((const uint8_t *)tab)[u[t]];
+    } else {
+#pragma unroll
+        for (int t = 0; t < T; t++) q[t] = u[t] >= (int32_t)hot ? (int32_t)A.wq.p16[u[t]] : -1;
+#pragma unroll
+        for (int t = 0; t < T; t++)
+            if ((uint32_t)u[t] < hot) q[t] = ((const uint16_t *)tab)[u[t]];
+    }
+}
 
 // The per-vertex inputs of a decision besides its connectivity: part, vertex
 // weight, lock (LP) and the weight of the own part (RW, RS).  Loaded once
@@ -640,11 +771,21 @@ __device__ inline int32_t select_mid(const SelArgs &A, const JetCtl &C, int32_t 
                 if (r0 + t * NQ >= ne) break;   // the same for the whole wave
                 const int32_t p = pt[t];
                 const bool lead = src[t] >= 0 && gl == 0;
-                if (mode == kModeRS) {
-                    int32_t own = 0;
+                // the own part's entries, most of a row's, are summed in
+                // registers (LDS atomics on one word follow each other); rows
+                // without other parts need nothing else
+                int32_t own = 0;
+                bool other = false;
 #pragma unroll
-                    for (int x = 0; x < E; x++) own += q[t][x] == p ? w[t][x] : 0;
-                    own = group_sum<G>(own);
+                for (int x = 0; x < E; x++) {
+                    if (q[t][x] == p) {
+                        own += w[t][x];
+                        q[t][x] = -1;
+                    }
+                    other |= q[t][x] >= 0;
+                }
+                own = group_sum<G>(own);
+                if (mode == kModeRS || !__any(other)) {
                     if (lead) res[src[t]] = make_int3(own, 0, -1);
                     continue;
                 }
@@ -652,11 +793,10 @@ __device__ inline int32_t select_mid(const SelArgs &A, const JetCtl &C, int32_t 
                 for (int x = 0; x < E; x++)
                     if (q[t][x] >= 0) atomicAdd(&my[q[t][x]], w[t][x]);
                 wave_lds_sync();
-                const int32_t pc = my[p];
                 PartKey best{0, -1};
 #pragma unroll
                 for (int x = 0; x < E; x++) {
-                    if (q[t][x] >= 0 && q[t][x] != p && tg[q[t][x]]) {
+                    if (q[t][x] >= 0 && tg[q[t][x]]) {
                         PartKey cand{my[q[t][x]], q[t][x]};
                         if (BetterPart()(cand, best)) best = cand;
                     }
@@ -666,7 +806,7 @@ __device__ inline int32_t select_mid(const SelArgs &A, const JetCtl &C, int32_t 
 #pragma unroll
                 for (int x = 0; x < E; x++)
                     if (q[t][x] >= 0) my[q[t][x]] = 0;
-                if (lead) res[src[t]] = make_int3(pc, best.c, best.q);
+                if (lead) res[src[t]] = make_int3(own, best.c, best.q);
                 wave_lds_sync();
             }
         }
@@ -719,23 +859,31 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_m(const int32_t *__restri
 // decide at once.  Waves loop on their own, without block barriers.
 constexpr int64_t kQuarterRow = kQuarterG * 8;
 
-template <bool Q>
-__global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restrict__ ids, int64_t cnt, int32_t rpw,
-                                                         SelArgs A)
+template <bool Q, bool Hot>
+__global__ void __launch_bounds__(Hot ? kHotBS : kRowBS) k_jet_select_w(const int32_t *__restrict__ ids, int64_t cnt,
+                                                                       int32_t rpw, SelArgs A)
 {
     extern __shared__ int32_t acc[];   // k ints per wave (4k with Q), then k part flags
+    constexpr int BS = Hot ? kHotBS : kRowBS;
     constexpr int S = (int)(kBinMid / kWave), NQ = Q ? kWave / kQuarterG : 1;
-    __shared__ int3 results[kRowBS];   // per row: connectivity to the own part, best other part
+    __shared__ int3 results[BS];   // per row: connectivity to the own part, best other part
+    __shared__ uint4 tab4[Hot ? kHotBytes / 16 : 1];
+    uint32_t *tab = (uint32_t *)tab4;
+    auto parts_of = [&](const auto &u, auto &q) {
+        if constexpr (Hot) hot_gather(A, tab, u, q);
+        else A.wq.gather(u, q);
+    };
     const JetCtl &C = *A.ctl;
     if (C.done) return;
     const int32_t mode = C.mode;
     const int64_t maxwgt = C.maxwgt, opt = C.opt;
     const int k = A.k, lane = lane_id();
-    const int wv = threadIdx.x / kWave, nw = kRowBS / kWave;
+    const int wv = threadIdx.x / kWave, nw = BS / kWave;
     const int quarter = lane / kQuarterG, gl = lane % kQuarterG;
     int32_t *my = acc + (size_t)wv * NQ * k;
     uint8_t *tg = (uint8_t *)(acc + (size_t)nw * NQ * k);
     for (int i = lane; i < NQ * k; i += kWave) my[i] = 0;
+    if constexpr (Hot) load_hot(A, tab);
     load_targets(A, mode, maxwgt, tg);
     int3 *res = results + wv * kWave;
     int32_t ncand = 0;
@@ -772,13 +920,20 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
                 const int32_t e = ql >= 0 ? b + d0 : b;
                 int32_t u[8], w[8], q[8];
                 load_entries<8, kQuarterG>(A.adjncy, A.adjwgt, b, e, gl, u, w);
-                A.wq.gather(u, q);
+                parts_of(u, q);
                 const bool lead = gl == 0 && ql >= 0;
-                if (mode == kModeRS) {
-                    int32_t own = 0;
+                int32_t own = 0;
+                bool other = false;
 #pragma unroll
-                    for (int t = 0; t < 8; t++) own += q[t] == p ? w[t] : 0;
-                    own = group_sum<kQuarterG>(own);
+                for (int t = 0; t < 8; t++) {
+                    if (q[t] == p) {
+                        own += w[t];
+                        q[t] = -1;
+                    }
+                    other |= q[t] >= 0;
+                }
+                own = group_sum<kQuarterG>(own);
+                if (mode == kModeRS || !__any(other)) {
                     if (lead) res[src] = make_int3(own, 0, -1);
                     continue;
                 }
@@ -787,11 +942,10 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
                 for (int t = 0; t < 8; t++)
                     if (q[t] >= 0) atomicAdd(&mq[q[t]], w[t]);
                 wave_lds_sync();
-                const int32_t pc = mq[p];
                 PartKey best{0, -1};
 #pragma unroll
                 for (int t = 0; t < 8; t++) {
-                    if (q[t] >= 0 && q[t] != p && tg[q[t]]) {
+                    if (q[t] >= 0 && tg[q[t]]) {
                         PartKey cand{mq[q[t]], q[t]};
                         if (BetterPart()(cand, best)) best = cand;
                     }
@@ -801,7 +955,7 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
 #pragma unroll
                 for (int t = 0; t < 8; t++)
                     if (q[t] >= 0) mq[q[t]] = 0;
-                if (lead) res[src] = make_int3(pc, best.c, best.q);
+                if (lead) res[src] = make_int3(own, best.c, best.q);
                 wave_lds_sync();
             }
         }
@@ -811,13 +965,20 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
             const int32_t p = wave_read(mr.p, l), b = wave_read(mb, l), e = b + wave_read(md, l);
             int32_t u[S], w[S], q[S];
             load_entries<S, kWave>(A.adjncy, A.adjwgt, b, e, lane, u, w);
-            A.wq.gather(u, q);
-            if (mode == kModeRS) {
-                // the strong rebalancer needs only the connectivity to the own part
-                int32_t own = 0;
+            parts_of(u, q);
+            int32_t own = 0;
+            bool other = false;
 #pragma unroll
-                for (int t = 0; t < S; t++) own += q[t] == p ? w[t] : 0;
-                own = wave_sum(own);
+            for (int t = 0; t < S; t++) {
+                if (q[t] == p) {
+                    own += w[t];
+                    q[t] = -1;
+                }
+                other |= q[t] >= 0;
+            }
+            own = wave_sum(own);
+            if (mode == kModeRS || !__any(other)) {
+                // the strong rebalancer needs only the connectivity to the own part
                 if (lane == 0) res[l] = make_int3(own, 0, -1);
                 continue;
             }
@@ -825,11 +986,10 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
             for (int t = 0; t < S; t++)
                 if (q[t] >= 0) atomicAdd(&my[q[t]], w[t]);
             wave_lds_sync();
-            int32_t pc = my[p];
             PartKey best{0, -1};
 #pragma unroll
             for (int t = 0; t < S; t++) {
-                if (q[t] >= 0 && q[t] != p && tg[q[t]]) {
+                if (q[t] >= 0 && tg[q[t]]) {
                     PartKey cand{my[q[t]], q[t]};
                     if (BetterPart()(cand, best)) best = cand;
                 }
@@ -839,7 +999,7 @@ __global__ void __launch_bounds__(kRowBS) k_jet_select_w(const int32_t *__restri
 #pragma unroll
             for (int t = 0; t < S; t++)
                 if (q[t] >= 0) my[q[t]] = 0;
-            if (lane == 0) res[l] = make_int3(pc, best.c, best.q);
+            if (lane == 0) res[l] = make_int3(own, best.c, best.q);
             wave_lds_sync();
         }
         wave_lds_sync();
@@ -886,36 +1046,35 @@ __global__ void __launch_bounds__(kSegBlk) k_jet_select_seg(RowSegs S, SelArgs A
         int32_t u[T], w[T], q[T];
         load_entries<T, kSegBlk>(A.adjncy, A.adjwgt, b, min(ee, b + kHalf), threadIdx.x, u, w);
         A.wq.gather(u, q);
-        if (mode == kModeRS) {
-            // only the connectivity to the own part: a block sum, no k-int row
-            int32_t own = 0;
+        // the own part's entries, often many, are summed in registers: LDS
+        // atomics on one word follow each other
+        int32_t own = 0;
+        auto add = [&] {
 #pragma unroll
-            for (int t = 0; t < T; t++) own += q[t] == p ? w[t] : 0;
-            if (two) {
-                load_entries<T, kSegBlk>(A.adjncy, A.adjwgt, b + kHalf, ee, threadIdx.x, u, w);
-                A.wq.gather(u, q);
-#pragma unroll
-                for (int t = 0; t < T; t++) own += q[t] == p ? w[t] : 0;
+            for (int t = 0; t < T; t++) {
+                if (q[t] == p) {
+                    own += w[t];
+                    q[t] = -1;
+                } else if (q[t] >= 0 && mode != kModeRS) {
+                    atomicAdd(&acc[q[t]], w[t]);
+                }
             }
-            own = group_sum<kSegBlk>(own);
-            if (threadIdx.x == 0) {
-                if (mi < 0) sel_decide(A, C, mode, v, rr, eligible, own, PartKey{0, -1});
-                else if (eligible && own) atomicAdd(&conn[(size_t)mi * k + p], own);
-            }
-            continue;
-        }
-        // a two-phase segment keeps only its second half in registers: walk the parts
-        bool walk_parts = two || e - b > (eid_t)k;
-#pragma unroll
-        for (int t = 0; t < T; t++)
-            if (q[t] >= 0) atomicAdd(&acc[q[t]], w[t]);
+        };
+        add();
         if (two) {
             load_entries<T, kSegBlk>(A.adjncy, A.adjwgt, b + kHalf, ee, threadIdx.x, u, w);
             A.wq.gather(u, q);
-#pragma unroll
-            for (int t = 0; t < T; t++)
-                if (q[t] >= 0) atomicAdd(&acc[q[t]], w[t]);
+            add();
         }
+        own = group_sum<kSegBlk>(own);
+        if (mi >= 0 && threadIdx.x == 0 && own) atomicAdd(&conn[(size_t)mi * k + p], own);
+        if (mode == kModeRS) {
+            // only the connectivity to the own part
+            if (mi < 0 && threadIdx.x == 0) sel_decide(A, C, mode, v, rr, eligible, own, PartKey{0, -1});
+            continue;
+        }
+        // a two-phase segment keeps only its second half in registers: walk the parts
+        const bool walk_parts = two || e - b > (eid_t)k;
         __syncthreads();
         if (mi >= 0) {
             // partial sums of a multi row: move them to conn and clear
@@ -941,7 +1100,6 @@ __global__ void __launch_bounds__(kSegBlk) k_jet_select_seg(RowSegs S, SelArgs A
             __syncthreads();
             continue;
         }
-        int32_t pc = eligible ? acc[p] : 0;
         PartKey best{0, -1};
         if (eligible) {
             if (walk_parts) {
@@ -953,7 +1111,7 @@ __global__ void __launch_bounds__(kSegBlk) k_jet_select_seg(RowSegs S, SelArgs A
             } else {
 #pragma unroll
                 for (int t = 0; t < T; t++) {
-                    if (q[t] < 0 || q[t] == p || !tg[q[t]]) continue;
+                    if (q[t] < 0 || !tg[q[t]]) continue;
                     PartKey cand{acc[q[t]], q[t]};
                     if (BetterPart()(cand, best)) best = cand;
                 }
@@ -970,7 +1128,84 @@ __global__ void __launch_bounds__(kSegBlk) k_jet_select_seg(RowSegs S, SelArgs A
             }
         }
         __syncthreads();
-        if (threadIdx.x == 0) ncand += sel_decide(A, C, mode, v, rr, eligible, pc, best);
+        if (threadIdx.x == 0) ncand += sel_decide(A, C, mode, v, rr, eligible, own, best);
+    }
+    sel_count(A, mode, ncand);
+    kb_flush(A.kb, kbytes);
+}
+
+// The same with the hot part ids in LDS: one block of 16 waves per CU shares
+// them and each wave takes a segment of its own with a k-int LDS row, so no
+// block barrier follows a segment.  R-MAT with 2^22 vertices, k = 256: the
+// first levels' 476 us a launch become 317 us (bound by the gathers that are
+// left, 122 G/s), the levels of up to 65536 vertices 400 us 240 us; the sums
+// of the own part, in registers instead of LDS atomics on one word, are half
+// of that.
+__global__ void __launch_bounds__(kHotBS) k_jet_select_seg_hot(RowSegs S, SelArgs A, int32_t *__restrict__ conn)
+{
+    extern __shared__ int32_t acc[];   // k ints per wave, then k part flags
+    constexpr int T = 8;
+    __shared__ uint4 tab4[kHotBytes / 16];
+    uint32_t *tab = (uint32_t *)tab4;
+    const JetCtl &C = *A.ctl;
+    if (C.done) return;
+    const int32_t mode = C.mode;
+    const int64_t maxwgt = C.maxwgt, opt = C.opt;
+    const int k = A.k, lane = lane_id(), wv = threadIdx.x / kWave, nw = kHotBS / kWave;
+    int32_t *my = acc + (size_t)wv * k;
+    uint8_t *tg = (uint8_t *)(acc + (size_t)nw * k);
+    for (int i = lane; i < k; i += kWave) my[i] = 0;
+    load_hot(A, tab);
+    load_targets(A, mode, maxwgt, tg);
+    int32_t ncand = 0;
+    uint64_t kbytes = 0;
+    for (int64_t s = (int64_t)wv * gridDim.x + blockIdx.x; s < S.nseg; s += (int64_t)gridDim.x * nw) {
+        const int32_t v = S.row[s], mi = S.mi[s];
+        const eid_t b = S.j0[s], e = min(b + (eid_t)kSegLen, A.xadj[v + 1]);
+        const SelRow rr = sel_row(A, mode, v);
+        const int32_t p = rr.p;
+        const bool eligible = sel_eligible(mode, maxwgt, opt, rr);
+        if (!eligible) {
+            if (lane == 0 && mi < 0) sel_decide(A, C, mode, v, rr, false, 0, PartKey{0, -1});
+            continue;
+        }
+        if (lane == 0) kbytes += 8 + 12 * (uint64_t)(e - b);
+        int32_t own = 0;
+        for (eid_t c0 = b; c0 < e; c0 += (eid_t)T * kWave) {
+            int32_t u[T], w[T], q[T];
+            load_entries<T, kWave>(A.adjncy, A.adjwgt, c0, e, lane, u, w);
+            hot_gather(A, tab, u, q);
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                if (q[t] == p) own += w[t];
+                else if (q[t] >= 0 && mode != kModeRS) atomicAdd(&my[q[t]], w[t]);
+            }
+        }
+        int32_t *row = mi >= 0 ? conn + (size_t)mi * k : nullptr;
+        own = wave_sum(own);
+        if (mi >= 0 && lane == 0 && own) atomicAdd(&row[p], own);
+        if (mode == kModeRS) {
+            // only the connectivity to the own part
+            if (mi < 0 && lane == 0) sel_decide(A, C, mode, v, rr, true, own, PartKey{0, -1});
+            continue;
+        }
+        wave_lds_sync();
+        PartKey best{0, -1};
+        for (int r = lane; r < k; r += kWave) {
+            const int32_t x = my[r];
+            my[r] = 0;
+            if (mi >= 0) {
+                if (x) atomicAdd(&row[r], x);
+            } else if (r != p && tg[r]) {
+                PartKey cand{x, r};
+                if (BetterPart()(cand, best)) best = cand;
+            }
+        }
+        wave_lds_sync();
+        if (mi < 0) {
+            best = group_best<kWave>(best, BetterPart());
+            if (lane == 0) ncand += sel_decide(A, C, mode, v, rr, true, own, best);
+        }
     }
     sel_count(A, mode, ncand);
     kb_flush(A.kb, kbytes);
@@ -1667,7 +1902,8 @@ __global__ void __launch_bounds__(kSegBlk) k_move_delta_seg(RowSegs S, int32_t k
 // copy costs no launch of its own (after the last iteration k_copy_best
 // makes it).
 __global__ void k_move_commit(int32_t n, const JetCtl *ctl, const int32_t *__restrict__ dest, int32_t *__restrict__ where,
-                              uint8_t *__restrict__ w8, uint16_t *__restrict__ w16, int32_t *__restrict__ best)
+                              uint8_t *__restrict__ w8, uint16_t *__restrict__ w16, int32_t *__restrict__ best,
+                              HotOrder ho)
 {
     if (ctl->done) return;
     int32_t v = (int32_t)((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
@@ -1675,8 +1911,9 @@ __global__ void k_move_commit(int32_t n, const JetCtl *ctl, const int32_t *__res
     if (ctl->copy_best) best[v] = where[v];
     int32_t d = dest[v];
     where[v] = d;
-    if (w8) w8[v] = (uint8_t)d;
-    else w16[v] = (uint16_t)d;
+    const int32_t x = ho.position(v);
+    if (w8) w8[x] = (uint8_t)d;
+    else w16[x] = (uint16_t)d;
 }
 
 // Keeps the iteration's partition when k_jet_next found it better (also when
@@ -1822,14 +2059,94 @@ inline size_t sel_w_lds(int32_t k, bool q)
     return sizeof(int32_t) * (kRowBS / kWave) * (q ? kWave / kQuarterG : 1) * (size_t)k;
 }
 
+// The hot part ids of a level: cap positions, of which held exist; code: the
+// positions in place of adjncy.
+struct HotParts {
+    HotOrder order;
+    int32_t cap = 0, held = 0;
+    const vid_t *code = nullptr;
+};
+
+// Entries of a class (or of both) from which the blocks with hot part ids are
+// worth filling their LDS (3 us, and fewer waves per CU).
+constexpr int64_t kHotEntries = (int64_t)1 << 20;
+constexpr size_t kLdsBytes = 160 << 10;
+constexpr unsigned kHotBlocks = 256;   // one per CU
+
+// Whether the level gets the hot order: the positions cost one pass over the
+// entries, so it has to be large, and the hot vertices have to receive at
+// least a third of the entries (counted from the degree classes, heaviest
+// first, each as if its rows had the class's mean length).
+bool want_hot_order(const Ctx &c, const DevGraph &g, int32_t k, int32_t cap)
+{
+    if (g.n <= cap || g.m < 4 * kHotEntries || 8 * g.bins.ent[kClsLong] < g.m) return false;
+    double left = cap, mass = 0;
+    for (int cls = kClsLong; cls >= 0 && left > 0; cls--) {
+        const double rows = (double)g.bins.count(cls), take = std::min(left, rows);
+        if (rows > 0) mass += (double)g.bins.ent[cls] * take / rows;
+        left -= take;
+    }
+    if (3 * mass < (double)g.m) return false;
+    // room for it beside everything the level allocates otherwise
+    return c.arena.free_bytes() > sizeof(vid_t) * (size_t)g.m + (size_t)128 * (size_t)g.n +
+                                      sizeof(int32_t) * (size_t)g.segs.nmulti * (size_t)k + ((size_t)64 << 20);
+}
+
+// Arrays on the right end of the arena.
+void hot_order(Ctx &c, const DevGraph &g, HotParts &h)
+{
+    const int32_t ncell = (g.n + 31) / 32;
+    uint2 *cells = c.arena.ralloc<uint2>((size_t)ncell);
+    vid_t *code = c.arena.ralloc<vid_t>((size_t)g.m);
+    const size_t mark = c.arena.right_mark();
+    int32_t *hist = c.arena.ralloc<int32_t>(kHotBuckets + 1);
+    int32_t *cnt = c.arena.ralloc<int32_t>((size_t)ncell), *before = c.arena.ralloc<int32_t>((size_t)ncell + 1);
+    fill<int32_t>(c, hist, kHotBuckets, 0);
+    k_hot_hist<<<kHotBlocks, kHotBS, 0, c.stream>>>(g.n, g.xadj, hist);
+    k_hot_pick<<<1, kHotBuckets, 0, c.stream>>>(hist, h.cap, hist + kHotBuckets);
+    k_hot_bits<<<grid_for(g.n, kBS), kBS, 0, c.stream>>>(g.n, g.xadj, hist + kHotBuckets, cells, cnt);
+    HGP_LAUNCH_CHECK();
+    offsets_from_counts(c, cnt, before, ncell);
+    k_hot_cells<<<grid_for(ncell, kBS), kBS, 0, c.stream>>>(ncell, before, cells);
+    h.order.cells = cells;
+    h.order.cap = h.cap;
+    KScope ks(c, "k_hot_codes", 8.0 * (double)g.m);
+    k_hot_codes<<<grid_for((g.m + 7) / 8, kBS), kBS, 0, c.stream>>>(g.m, g.adjncy, h.order, code);
+    HGP_LAUNCH_CHECK();
+    h.code = code;
+    h.held = h.cap;
+    c.arena.right_release(mark);
+}
+
+// A launch of k_jet_select_w over nw rows with `ent` entries.
+void launch_select_w(Ctx &c, const SelArgs &A, const HotParts &h, const int32_t *list, int64_t nw, int64_t ent)
+{
+    const int k = A.k;
+    const size_t tg = ((size_t)k + 3) & ~(size_t)3, fixed = kHotBytes + sizeof(int3) * kHotBS + 64;
+    const bool q = k <= kQuarterK;
+    if (A.hot && ent >= kHotEntries) {
+        const size_t one = 16 * sizeof(int32_t) * (size_t)k, four = 4 * one;
+        const int32_t rpw = (int32_t)std::max<int64_t>(4, std::min<int64_t>(kWave, nw / (kHotBlocks * 16 * 4)));
+        const unsigned blocks = (unsigned)std::min<int64_t>((nw + 16 * rpw - 1) / (16 * rpw), kHotBlocks);
+        if (q && fixed + four + tg <= kLdsBytes)
+            return k_jet_select_w<true, true><<<blocks, kHotBS, four + tg, c.stream>>>(list, nw, rpw, A);
+        if (fixed + one + tg <= kLdsBytes)
+            return k_jet_select_w<false, true><<<blocks, kHotBS, one + tg, c.stream>>>(list, nw, rpw, A);
+    }
+    const int32_t rpw = rows_per_wave(nw);
+    const unsigned blocks = wave_blocks(nw, rpw, 4096);
+    if (q) k_jet_select_w<true, false><<<blocks, kRowBS, sel_w_lds(k, true) + tg, c.stream>>>(list, nw, rpw, A);
+    else k_jet_select_w<false, false><<<blocks, kRowBS, sel_w_lds(k, false) + tg, c.stream>>>(list, nw, rpw, A);
+}
+
 void launch_select(Ctx &c, const DevGraph &g, int32_t k, const int32_t *where, const int64_t *pwgts,
                    const uint8_t *lock, const int32_t *under, JetCtl *ctl, int32_t *dest, int32_t *pregain,
                    uint32_t *key, int32_t *conn, NarrowParts wq, uint64_t *ab, uint16_t *pd16, uint32_t *pd32,
-                   const HubConn &hc)
+                   const HubConn &hc, const HotParts &h)
 {
     const RowBins &b = g.bins;
-    SelArgs A{k,   g.xadj, g.adjncy, g.adjwgt, g.vwgt, where, pwgts, lock, under, ctl,
-              dest, pregain, key, nullptr, wq, ab, pd16, pd32};
+    SelArgs A{k,   g.xadj, h.code ? h.code : g.adjncy, g.adjwgt, g.vwgt, where, pwgts, lock, under, ctl,
+              dest, pregain, key, nullptr, wq, ab, pd16, pd32, h.cap, h.held};
     const size_t tg_bytes = ((size_t)k + 3) & ~(size_t)3;   // part flags of the selection kernels
     // fixed bytes: ids, where, pwgts[p], vwgt, the decision (24 per row); eligible rows add xadj and
     // 12 B per entry (adjncy, adjwgt, where gather) in the kernel
@@ -1837,13 +2154,7 @@ void launch_select(Ctx &c, const DevGraph &g, int32_t k, const int32_t *where, c
         if (int64_t nw = b.short_rows()) {
             KScope ks(c, "k_jet_select_few", 24.0 * (double)nw, true);
             A.kb = ks.dev();
-            int32_t rpw = rows_per_wave(nw);
-            if (k <= kQuarterK)
-                k_jet_select_w<true><<<wave_blocks(nw, rpw, 4096), kRowBS, sel_w_lds(k, true) + tg_bytes, c.stream>>>(
-                    b.list(0), nw, rpw, A);
-            else
-                k_jet_select_w<false><<<wave_blocks(nw, rpw, 4096), kRowBS, sel_w_lds(k, false) + tg_bytes,
-                                        c.stream>>>(b.list(0), nw, rpw, A);
+            launch_select_w(c, A, h, b.list(0), nw, b.ent[0] + b.ent[1] + b.ent[2]);
             HGP_LAUNCH_CHECK();
         }
     }
@@ -1872,14 +2183,7 @@ void launch_select(Ctx &c, const DevGraph &g, int32_t k, const int32_t *where, c
     if (int64_t nw = b.few() ? 0 : (quarter ? 0 : b.count(1)) + b.count(2)) {
         KScope ks(c, "k_jet_select_w", 24.0 * (double)nw, true);
         A.kb = ks.dev();
-        int32_t rpw = rows_per_wave(nw);
-        const int32_t *list = quarter ? b.list(2) : b.list(1);
-        if (k <= kQuarterK)
-            k_jet_select_w<true><<<wave_blocks(nw, rpw, 4096), kRowBS, sel_w_lds(k, true) + tg_bytes, c.stream>>>(
-                list, nw, rpw, A);
-        else
-            k_jet_select_w<false><<<wave_blocks(nw, rpw, 4096), kRowBS, sel_w_lds(k, false) + tg_bytes, c.stream>>>(
-                list, nw, rpw, A);
+        launch_select_w(c, A, h, quarter ? b.list(2) : b.list(1), nw, (quarter ? 0 : b.ent[1]) + b.ent[2]);
         HGP_LAUNCH_CHECK();
     }
     if (hc.hidx) {
@@ -1895,8 +2199,13 @@ void launch_select(Ctx &c, const DevGraph &g, int32_t k, const int32_t *where, c
         {
             KScope ks(c, "k_jet_select_seg", 24.0 * (double)g.segs.nseg, true);
             A.kb = ks.dev();
-            k_jet_select_seg<<<seg_grid(g.segs), kSegBlk, sizeof(int32_t) * (size_t)k + tg_bytes, c.stream>>>(
-                g.segs, A, conn);
+            const size_t lds = 16 * sizeof(int32_t) * (size_t)k + tg_bytes;
+            if (A.hot && b.ent[kClsLong] >= kHotEntries && kHotBytes + 64 + lds <= kLdsBytes)
+                k_jet_select_seg_hot<<<(unsigned)std::min<int64_t>((g.segs.nseg + 15) / 16, kHotBlocks), kHotBS, lds,
+                                       c.stream>>>(g.segs, A, conn);
+            else
+                k_jet_select_seg<<<seg_grid(g.segs), kSegBlk, sizeof(int32_t) * (size_t)k + tg_bytes, c.stream>>>(
+                    g.segs, A, conn);
             HGP_LAUNCH_CHECK();
         }
         A.kb = nullptr;
@@ -2484,8 +2793,24 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
     // where and dest in one word (move accounting), pregain, where and dest
     // in 8 bytes (afterburner)
     const bool byte_parts = k <= 256;
-    uint8_t *w8 = byte_parts ? c.arena.ralloc<uint8_t>((size_t)n) : nullptr;
-    uint16_t *w16 = byte_parts ? nullptr : c.arena.ralloc<uint16_t>((size_t)n);
+    const bool tiny = n <= tuning().tiny_max && k <= kTinyK;
+    HotParts hot;
+    const int32_t hot_cap = (int32_t)(kHotBytes / (byte_parts ? 1 : 2));
+    if (!tiny && !tuning().hub_track) {
+        // (with few long rows the neighbours of a row are mostly near each other
+        // and hit the L1: banded graphs, rows of 33..512 entries: 13.5 us a
+        // launch without, 16.3 us with the ids in LDS)
+        if (n <= hot_cap && 8 * g.bins.ent[kClsLong] >= g.m) {
+            hot.cap = hot_cap;
+            hot.held = n;
+        } else if (want_hot_order(c, g, k, hot_cap)) {
+            hot.cap = hot_cap;
+            hot_order(c, g, hot);
+        }
+    }
+    const size_t npos = (size_t)n + (hot.code ? (size_t)hot_cap : 0);
+    uint8_t *w8 = byte_parts ? c.arena.ralloc<uint8_t>(npos) : nullptr;
+    uint16_t *w16 = byte_parts ? nullptr : c.arena.ralloc<uint16_t>(npos);
     uint16_t *pd16 = byte_parts ? c.arena.ralloc<uint16_t>((size_t)n) : nullptr;
     uint32_t *pd32 = byte_parts ? nullptr : c.arena.ralloc<uint32_t>((size_t)n);
     uint64_t *ab = c.arena.ralloc<uint64_t>((size_t)n);
@@ -2501,7 +2826,7 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
     HGP_CHECK_HIP(hipMemcpyAsync(best, where, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToDevice, c.stream));
     part_weights(c, n, g.vwgt, where, k, pwgts);
     k_jet_init<<<1, kBS, 0, c.stream>>>(ctl, k, pwgts, d_cut, maxwgt, opt, p.patience, finest ? 1 : 3);
-    k_narrow<<<grid_for(n, kBS), kBS, 0, c.stream>>>(n, where, w8, w16);   // refreshed by each commit
+    k_narrow<<<grid_for(n, kBS), kBS, 0, c.stream>>>(n, where, w8, w16, hot.order);   // refreshed by each commit
     HGP_LAUNCH_CHECK();
     // connectivity rows of the long rows, when asked for, while k-int rows
     // are short beside them (k <= kTrackMaxK) and the level runs the
@@ -2512,7 +2837,6 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
     HubConn hc;
     hc.k = k;
     const int64_t nhub = g.bins.count(kClsLong);
-    const bool tiny = n <= tuning().tiny_max && k <= kTinyK;
     if (nhub > 0 && k <= kTrackMaxK && !tiny && tuning().hub_track) {
         int32_t *hidx = c.arena.ralloc<int32_t>((size_t)n);
         hc.tconn = c.arena.ralloc<int32_t>((size_t)nhub * (size_t)k);
@@ -2682,13 +3006,13 @@ RefineStats refine_level(Ctx &c, const DevGraph &g, int32_t k, int64_t tvwgt, bo
                 HGP_CHECK_HIP(hipStreamSynchronize(c.stream));
             }
         }
-        k_move_commit<<<gv, kBS, 0, c.stream>>>(n, ctl, dest, where, w8, w16, best);
+        k_move_commit<<<gv, kBS, 0, c.stream>>>(n, ctl, dest, where, w8, w16, best, hot.order);
         HGP_LAUNCH_CHECK();
         k_jet_next<<<1, kNextBS, 0, c.stream>>>(ctl, k, pwgts, ms, under, 0, mirror);
         HGP_LAUNCH_CHECK();
     };
     auto issue_select = [&] {
-        launch_select(c, g, k, where, pwgts, lock, under, ctl, dest, pregain, key, conn, wq, ab, pd16, pd32, hc);
+        launch_select(c, g, k, where, pwgts, lock, under, ctl, dest, pregain, key, conn, wq, ab, pd16, pd32, hc, hot);
     };
     // Levels of at most Tuning::graph_max_vertices vertices record each
     // launch sequence once as a HIP graph and replay it (not while kernels are
