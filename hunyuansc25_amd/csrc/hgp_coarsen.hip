@@ -734,8 +734,8 @@ __device__ inline void group_bitonic(uint32_t &key, int32_t &val)
     for (int k = 2; k <= G; k <<= 1) {
 #pragma unroll
         for (int j = k >> 1; j > 0; j >>= 1) {
-            uint32_t ok = __shfl_xor(key, j, G);
-            int32_t ov = __shfl_xor(val, j, G);
+            uint32_t ok = lane_xor(key, j);
+            int32_t ov = (int32_t)lane_xor((uint32_t)val, j);
             bool asc = (lane & k) == 0;
             bool lower = (lane & j) == 0;
             bool take = (lower == asc) ? ok < key : ok > key;
@@ -750,6 +750,7 @@ __device__ inline void group_bitonic(uint32_t &key, int32_t &val)
 template <int G>
 __device__ inline int32_t group_inclusive_scan(int32_t v)
 {
+    if constexpr (G == kWave) return wave_inclusive_scan(v);
     const int lane = glane<G>();
 #pragma unroll
     for (int o = 1; o < G; o <<= 1) {
@@ -774,10 +775,11 @@ __device__ inline void seg_reg_row(int32_t c, int lane, const int32_t *__restric
     int32_t w = 0;
     if (lane < len) {
         eid_t j = row.at(lane);
+        const int32_t wj = adjwgt[j];   // (beside adjncy, not after cmap)
         int32_t cc = cmap[adjncy[j]];
         if (cc != c) {
             key = (uint32_t)cc;
-            w = adjwgt[j];
+            w = wj;
         }
     }
     group_bitonic<G>(key, w);
@@ -818,8 +820,8 @@ __global__ void __launch_bounds__(kRowBS) k_seg_reg(const int32_t *__restrict__ 
 }
 
 // Bitonic network over R*64 entries held R per lane (entry e = r*64 + lane):
-// partners closer than 64 are exchanged with xor-shuffles, farther ones are
-// register swaps inside the lane.
+// partners closer than 64 are exchanged on the VALU, farther ones are register
+// swaps inside the lane.
 template <int R, int KR>
 __device__ inline void wave_bitonic(uint32_t (&key)[KR], int32_t (&val)[KR])
 {
@@ -849,8 +851,8 @@ __device__ inline void wave_bitonic(uint32_t (&key)[KR], int32_t (&val)[KR])
             } else {
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    uint32_t ok = __shfl_xor(key[r], j, kWave);
-                    int32_t ov = __shfl_xor(val[r], j, kWave);
+                    uint32_t ok = lane_xor(key[r], j);
+                    int32_t ov = (int32_t)lane_xor((uint32_t)val[r], j);
                     bool asc = ((r * kWave + lane) & k) == 0;
                     bool lower = (lane & j) == 0;
                     bool take = (lower == asc) ? ok < key[r] : ok > key[r];

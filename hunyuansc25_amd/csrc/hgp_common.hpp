@@ -94,7 +94,7 @@ void destroy_context(std::unique_ptr<Ctx> c);      // releases a private context
 // and sets them through hgp_set_tuning.
 struct Tuning {
     int32_t tiny_max = 512;      // levels of <= this many vertices (k <= 256) run the Jet loop in one block
-    int64_t few_rows = 8192;     // levels with <= this many rows of <= 512 entries run them in one launch
+    int64_t few_rows = 16384;    // levels with <= this many rows of <= 512 entries run them in one launch
     int64_t fill_waves = 8192;   // waves the wave-per-row kernels spread a level's rows over
     int32_t seg_grid = 32768;    // grid cap of the segment kernels
     int32_t batch_lanes = 8;     // lanes of hgp_partition_batch when the caller passes <= 0
@@ -295,6 +295,28 @@ __device__ inline void half_values(T v, T &lo, T &hi)
     }
     __builtin_memcpy(&lo, a, sizeof(T));
     __builtin_memcpy(&hi, b, sizeof(T));
+}
+
+// v of lane (own lane xor j), j a power of two below 64 that is a constant
+// after unrolling; the lanes of each aligned group of 2j must be active.
+__device__ inline uint32_t lane_xor(uint32_t v, int j)
+{
+    switch (j) {
+    case 1: return dpp_move<0xB1>(v);                      // quad_perm [1,0,3,2]
+    case 2: return dpp_move<0x4E>(v);                      // quad_perm [2,3,0,1]
+    case 4: return dpp_move<0x1B>(dpp_move<0x141>(v));     // row_half_mirror (xor 7), quad_perm [3,2,1,0]
+    case 8: return dpp_move<0x128>(v);                     // row_ror:8
+    case 16: {
+        uint32_t even, odd;   // the even and the odd row of each pair
+        half_values<16>(v, even, odd);
+        return threadIdx.x & 16 ? even : odd;
+    }
+    default: {
+        uint32_t lo, hi;
+        half_values<32>(v, lo, hi);
+        return threadIdx.x & 32 ? lo : hi;
+    }
+    }
 }
 
 // op over the G lanes of each group (G a power of two up to 64, aligned),
