@@ -2068,8 +2068,10 @@ struct HotParts {
 };
 
 // Entries of a class (or of both) from which the blocks with hot part ids are
-// worth filling their LDS (3 us, and fewer waves per CU).
-constexpr int64_t kHotEntries = (int64_t)1 << 20;
+// worth filling their LDS (3 us, and fewer waves per CU): with 1..4M entries,
+// R-MAT with 2^17 vertices and k = 1000, they take 22 us a launch where the
+// kernels without them take 15.
+constexpr int64_t kHotEntries = (int64_t)1 << 22;
 constexpr size_t kLdsBytes = 160 << 10;
 constexpr unsigned kHotBlocks = 256;   // one per CU
 
@@ -2079,7 +2081,7 @@ constexpr unsigned kHotBlocks = 256;   // one per CU
 // first, each as if its rows had the class's mean length).
 bool want_hot_order(const Ctx &c, const DevGraph &g, int32_t k, int32_t cap)
 {
-    if (g.n <= cap || g.m < 4 * kHotEntries || 8 * g.bins.ent[kClsLong] < g.m) return false;
+    if (g.n <= cap || g.m < 2 * kHotEntries || 8 * g.bins.ent[kClsLong] < g.m) return false;
     double left = cap, mass = 0;
     for (int cls = kClsLong; cls >= 0 && left > 0; cls--) {
         const double rows = (double)g.bins.count(cls), take = std::min(left, rows);

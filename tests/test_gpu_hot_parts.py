@@ -1,5 +1,5 @@
 """Refinement of large levels against the oracle, bit for bit, where the
-selection keeps part ids in LDS: levels held whole (up to 65536 byte ids, 32768
+selection keeps part ids in LDS (classes of at least 4M entries): levels held whole (up to 65536 byte ids, 32768
 of 16 bits), larger ones in the order with the heaviest vertices first, k
 whose LDS rows leave room for four rows a wave, for one, and for none.
 (reference: hunyuangraph_GPU_krefine.h:1995-2135, 2515-2556, 3184-3241)"""
@@ -9,9 +9,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("scale,nedges,k", [(15, 1 << 21, 40), (15, 1 << 21, 256), (15, 1 << 21, 257),
-                                            (15, 1 << 21, 1000), (15, 1 << 21, 1500), (16, 1 << 21, 40),
-                                            (17, 1 << 22, 40), (16, 1 << 22, 300)])
+@pytest.mark.parametrize("scale,nedges,k", [(15, 1 << 21, 40), (15, 1 << 23, 1000), (15, 1 << 23, 1500),
+                                            (16, 1 << 24, 40), (17, 1 << 24, 256), (17, 1 << 24, 257)])
 def test_selection(hgp, orc, scale, nedges, k):
     x, a, vw, aw = hgp.gen_rmat(scale, nedges, seed=scale + k)
     n = len(x) - 1
