@@ -866,99 +866,138 @@ __device__ inline void wave_bitonic(uint32_t (&key)[KR], int32_t (&val)[KR])
     }
 }
 
-// Stable LSD radix sort of a block's P = (BS/64)*R*64 entries (registers
-// 0..R-1 of RMAX in use) by the low 8*passes bits of the key (8-bit digits),
-// entry w*C + r*64 + lane (C = R*64) held in register r of lane `lane` of
-// wave w.  Each pass after the first ranks a wave's entries by digit
-// (entries of equal digit keep their order: register-major, then lane) from
-// 8 ballots per register and a per-wave count of each digit (wc, 256 ints
-// per wave); the first pass, whose input order is arbitrary anyway, takes
-// its ranks from LDS atomics on the same counts.  The counts become scatter
-// bases by a scan over (digit, wave), and the entries scatter into sk/sw; the entries are read back into
-// registers for the next pass.  The last pass leaves the sorted entries in
-// sk/sw, P of them.  Keys beyond the low bits (the sentinel) must sort last
-// on those bits alone.
+// Radix sort, least significant digit first, of a block's entries by the low
+// `bits` bits of the key; entry w*C + r*64 + lane (C = R*64) is held in register
+// r of lane `lane` of wave w (registers 0..R-1 of RMAX in use).  Entries with
+// the sentinel are dropped; the others are left in sk/sw, and their number is
+// returned.
+//
+// The first digit is as wide as sk has words for counters (14 bits for 16384
+// entries, 12 for 4096): the input order is arbitrary, so LDS atomics on one
+// count per digit value are ranks.  Each later pass, of up to 9 bits, has to
+// keep the order: a wave ranks its entries register by register with a ballot
+// per bit and a count per digit value and wave (wc, 512 per wave), the counts
+// become scatter bases by a scan over (digit, wave), and the entries go through
+// sk/sw.  A bit costs a later pass four VALU instructions per register and the
+// first pass nothing: with 8-bit digits throughout, three passes for ids of 17
+// bits and more, the two kernels took 7.8 and 5.9 ms per partition of R-MAT
+// with 2^22 vertices, now 7.0 and 5.5.
+constexpr int kDigit = 9, kDigits = 1 << kDigit;
+
 template <int RMAX, int BS>
-__device__ inline void block_radix(uint32_t (&key)[RMAX], int32_t (&val)[RMAX], int R, uint32_t *sk, int32_t *sw,
-                                   int32_t *wc, int32_t *dsum, int passes)
+__device__ inline int32_t block_radix(uint32_t (&key)[RMAX], int32_t (&val)[RMAX], int R, uint32_t *sk, int32_t *sw,
+                                      uint16_t *wc, int32_t *dsum, int bits)
 {
-    constexpr int NW = BS / kWave;
+    constexpr int NW = BS / kWave, PMAX = BS * RMAX, B1 = __builtin_ctz(PMAX);
+    static_assert(BS >= kDigits && (PMAX & (PMAX - 1)) == 0, "a thread per digit value");
     const int C = R * kWave;
     const int w = threadIdx.x / kWave, lane = lane_id();
     const uint64_t lt = lanemask_lt();
-    int32_t *my = wc + w * 256;
-    for (int pass = 0; pass < passes; pass++) {
-        const int shift = 8 * pass;
-        for (int i = lane; i < 256; i += kWave) my[i] = 0;
-        wave_lds_sync();
-        int32_t rk[RMAX];
-        if (pass == 0) {
-            // the first pass may order equal digits any way (the input order
-            // is arbitrary anyway): ranks from LDS atomics
+    int done = min(bits, B1);
+    int32_t rk[RMAX], nvalid;
+    {
+        const int nd = 1 << done;
+        const uint32_t mask = (uint32_t)nd - 1;
+        for (int i = threadIdx.x; i < nd; i += BS) sk[i] = 0;
+        __syncthreads();
 #pragma unroll
-            for (int r = 0; r < RMAX; r++) {
-                if (r >= R) break;
-                rk[r] = atomicAdd(&my[(key[r] >> shift) & 255u], 1);
-            }
-            wave_lds_sync();
-        } else {
-#pragma unroll
-            for (int r = 0; r < RMAX; r++) {
-                if (r >= R) break;   // R is the same for the whole block
-                const uint32_t d = (key[r] >> shift) & 255u;
-                uint64_t peers = ~0ull;   // lanes whose register r holds the same digit
-#pragma unroll
-                for (int b = 0; b < 8; b++) {
-                    const bool bit = (d >> b) & 1u;
-                    const uint64_t bb = __ballot(bit);
-                    peers &= bit ? bb : ~bb;
-                }
-                const int32_t base = my[d];
-                rk[r] = base + __popcll(peers & lt);
-                wave_lds_sync();   // every lane has its base
-                if ((peers & lt) == 0) my[d] = base + __popcll(peers);
-                wave_lds_sync();
-            }
+        for (int r = 0; r < RMAX; r++) {
+            if (r >= R) break;   // R is the same for the whole block
+            rk[r] = key[r] != kSent ? (int32_t)atomicAdd(&sk[key[r] & mask], 1u) : 0;
         }
         __syncthreads();
-        // base of (digit d, wave x): entries of smaller digits, then of digit d in waves < x
-        const int d = threadIdx.x & 255;
-        int32_t run = 0;
-        if (threadIdx.x < 256) {
+        // counts to bases, RMAX digit values per thread at most
+        const int per = max(nd / BS, 1), d0 = (int)threadIdx.x * per;
+        int32_t c[RMAX], sum = 0;
 #pragma unroll
-            for (int x = 0; x < NW; x++) {
-                const int32_t c = wc[x * 256 + d];
-                wc[x * 256 + d] = run;
-                run += c;
-            }
+        for (int i = 0; i < RMAX; i++) {
+            c[i] = i < per && d0 < nd ? (int32_t)sk[d0 + i] : 0;
+            sum += c[i];
         }
-        const int32_t incl = wave_inclusive_scan(run);
-        if (threadIdx.x < 256 && lane == kWave - 1) dsum[w] = incl;
-        __syncthreads();
-        if (threadIdx.x < 256) {
-            int32_t pre = incl - run;
-            for (int x = 0; x < w; x++) pre += dsum[x];
+        int32_t run = block_exclusive_scan(sum, dsum, &nvalid);
 #pragma unroll
-            for (int x = 0; x < NW; x++) wc[x * 256 + d] += pre;
+        for (int i = 0; i < RMAX; i++) {
+            if (i < per && d0 < nd) sk[d0 + i] = (uint32_t)run;
+            run += c[i];
         }
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < RMAX; r++) {
             if (r >= R) break;
-            const int32_t at = wc[w * 256 + ((key[r] >> shift) & 255u)] + rk[r];
-            sk[at] = key[r];
-            sw[at] = val[r];
+            if (key[r] != kSent) rk[r] += (int32_t)sk[key[r] & mask];
         }
-        __syncthreads();
-        if (pass + 1 < passes) {
+        __syncthreads();   // the bases have been read: sk/sw take the entries
 #pragma unroll
-            for (int r = 0; r < RMAX; r++) {
-                if (r >= R) break;
-                key[r] = sk[w * C + r * kWave + lane];
-                val[r] = sw[w * C + r * kWave + lane];
+        for (int r = 0; r < RMAX; r++) {
+            if (r >= R) break;
+            if (key[r] != kSent) {
+                sk[rk[r]] = key[r];
+                sw[rk[r]] = val[r];
             }
         }
+        __syncthreads();
     }
+    uint16_t *my = wc + w * kDigits;
+    for (; done < bits; done += kDigit) {
+        const int nb = min(bits - done, kDigit);
+        const uint32_t mask = (1u << nb) - 1;
+        for (int i = lane; i < kDigits; i += kWave) my[i] = 0;
+#pragma unroll
+        for (int r = 0; r < RMAX; r++) {
+            if (r >= R) break;
+            const int i = w * C + r * kWave + lane;
+            key[r] = i < nvalid ? sk[i] : kSent;
+            val[r] = i < nvalid ? sw[i] : 0;
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int r = 0; r < RMAX; r++) {
+            if (r >= R) break;
+            const uint32_t d = (key[r] >> done) & mask;
+            uint64_t peers = __ballot(key[r] != kSent);   // lanes whose register r holds the same digit
+#pragma unroll
+            for (int x = 0; x < kDigit; x++) {
+                if (x >= nb) break;
+                const bool bit = (d >> x) & 1u;
+                const uint64_t bb = __ballot(bit);
+                peers &= bit ? bb : ~bb;
+            }
+            const int32_t base = my[d];
+            rk[r] = base + __popcll(peers & lt);
+            wave_lds_sync();   // every lane has its base
+            if (key[r] != kSent && (peers & lt) == 0) my[d] = (uint16_t)(base + __popcll(peers));
+            wave_lds_sync();
+        }
+        __syncthreads();
+        // base of (digit d, wave x): entries of smaller digits, then of digit d in waves < x
+        const int d = threadIdx.x;
+        int32_t run = 0;
+        if (d < kDigits) {
+#pragma unroll
+            for (int x = 0; x < NW; x++) {
+                const int32_t c = wc[x * kDigits + d];
+                wc[x * kDigits + d] = (uint16_t)run;
+                run += c;
+            }
+        }
+        const int32_t pre = block_exclusive_scan(run, dsum, (int32_t *)nullptr);
+        if (d < kDigits) {
+#pragma unroll
+            for (int x = 0; x < NW; x++) wc[x * kDigits + d] = (uint16_t)(wc[x * kDigits + d] + pre);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < RMAX; r++) {
+            if (r >= R) break;
+            if (key[r] != kSent) {
+                const int32_t at = my[(key[r] >> done) & mask] + rk[r];
+                sk[at] = key[r];
+                sw[at] = val[r];
+            }
+        }
+        __syncthreads();
+    }
+    return nvalid;
 }
 
 // Rows of 65..kSegWaveMax entries: one wave per row, sorted in registers
@@ -1040,25 +1079,25 @@ __global__ void __launch_bounds__(kRowBS) k_seg_wave(const int32_t *__restrict__
 }
 
 // Rows of up to BS*RMAX entries: one block of BS threads per row, radix sort
-// through LDS (padded to BS*RMAX, half or a quarter of it; `passes` 8-bit
-// digits cover every coarse id), then tails (last entry of each run of equal ids) are ranked by
+// through LDS (padded to BS*RMAX, half or a quarter of it; coarse ids have
+// `bits` bits), then tails (last entry of each run of equal ids) are ranked by
 // a block scan and their inclusive weight prefixes differenced.
 template <int BS, int RMAX>
-__global__ void __launch_bounds__(BS) k_seg_lds(const int32_t *__restrict__ ids, int64_t cnt,
+__global__ void __launch_bounds__(BS, BS == 512 ? 6 : 4) k_seg_lds(const int32_t *__restrict__ ids, int64_t cnt,
                                                     const int32_t *__restrict__ rep,
                                                     const int32_t *__restrict__ match,
                                                     const eid_t *__restrict__ xadj, const vid_t *__restrict__ adjncy,
                                                     const wgt_t *__restrict__ adjwgt,
                                                     const int32_t *__restrict__ cmap, const int64_t *__restrict__ toff,
                                                     int32_t *__restrict__ tadj, int32_t *__restrict__ twgt,
-                                                    int32_t *__restrict__ ccnt, int passes, unsigned long long *kb)
+                                                    int32_t *__restrict__ ccnt, int bits, unsigned long long *kb)
 {
     constexpr int PMAX = BS * RMAX;
     __shared__ uint32_t sk[PMAX];
     uint64_t kbytes = 0;
     __shared__ int32_t sw[PMAX];
-    __shared__ int32_t wc[BS / kWave * 256];
-    __shared__ int32_t dsum[4];
+    __shared__ uint16_t wc[BS / kWave * kDigits];
+    __shared__ int32_t dsum[BS / kWave];
     __shared__ int64_t sh[BS / kWave + 1];
     const int tid = threadIdx.x;
     for (int64_t gi = blockIdx.x; gi < cnt; gi += gridDim.x) {
@@ -1066,6 +1105,7 @@ __global__ void __launch_bounds__(BS) k_seg_lds(const int32_t *__restrict__ ids,
         int32_t v = rep[c], u = match[v];
         CatRow row(xadj, v, u);
         int len = (int)(row.dv + (u != v ? xadj[u + 1] - row.bu : 0));
+        int32_t nvalid;
         const int P = len <= PMAX / 4 ? PMAX / 4 : (len <= PMAX / 2 ? PMAX / 2 : PMAX);
         {
             // entries straight into registers (entry w*C + r*64 + lane), sorted by the block
@@ -1090,18 +1130,18 @@ __global__ void __launch_bounds__(BS) k_seg_lds(const int32_t *__restrict__ ids,
                 key[r] = cc != c ? (uint32_t)cc : kSent;
                 val[r] = cc != c ? val[r] : 0;
             }
-            block_radix<RMAX, BS>(key, val, R, sk, sw, wc, dsum, passes);
+            nvalid = block_radix<RMAX, BS>(key, val, R, sk, sw, wc, dsum, bits);
         }
         // Thread tid owns entries [tid*E, tid*E + E), E = P / BS (one each when P < BS).
         const int E = P >= BS ? P / BS : 1;
         const int first = tid * E;
         uint32_t kk[RMAX];
         int32_t ww[RMAX];
-        uint32_t after = first + E < P ? sk[first + E] : kSent;
+        uint32_t after = first + E < nvalid ? sk[first + E] : kSent;
 #pragma unroll
         for (int e = 0; e < RMAX; e++) {
             int i = first + e;
-            bool own = e < E && i < P;
+            bool own = e < E && i < nvalid;
             kk[e] = own ? sk[i] : kSent;
             ww[e] = own ? sw[i] : 0;
         }
@@ -1790,18 +1830,18 @@ DevGraph contract(Ctx &c, const DevGraph &g, const int32_t *match, const int32_t
         if (cb.count(3)) {
             KScope ks(c, "k_seg_lds", bytes(3), true);
             unsigned blocks = (unsigned)std::min<int64_t>(cb.count(3), 8192);
-            const int passes = std::max(1, (bits_for((uint64_t)cn) + 7) / 8);   // coarse ids < 2^(8*passes) - 1
+            const int bits = std::max(1, bits_for((uint64_t)cn));
             k_seg_lds<kSegBS, kSegE><<<blocks, kSegBS, 0, c.stream>>>(cb.list(3), cb.count(3), rep, match, g.xadj,
                                                                       g.adjncy, g.adjwgt, cmap, toff, tadj, twgt,
-                                                                      ccnt, passes, ks.dev());
+                                                                      ccnt, bits, ks.dev());
             HGP_LAUNCH_CHECK();
         }
         if (cb.count(4)) {
             KScope ks(c, "k_seg_lds_big", bytes(4), true);
             unsigned blocks = (unsigned)std::min<int64_t>(cb.count(4), 4096);
-            const int passes = std::max(1, (bits_for((uint64_t)cn) + 7) / 8);
+            const int bits = std::max(1, bits_for((uint64_t)cn));
             k_seg_lds<kSegBigBS, kSegBig / kSegBigBS><<<blocks, kSegBigBS, 0, c.stream>>>(
-                cb.list(4), cb.count(4), rep, match, g.xadj, g.adjncy, g.adjwgt, cmap, toff, tadj, twgt, ccnt, passes,
+                cb.list(4), cb.count(4), rep, match, g.xadj, g.adjncy, g.adjwgt, cmap, toff, tadj, twgt, ccnt, bits,
                 ks.dev());
             HGP_LAUNCH_CHECK();
         }
