@@ -714,9 +714,10 @@ int hgp_partition_batch(int32_t count, const int32_t *n, const int64_t *const *x
         // refines alone: worth it for the larger levels once the group keeps
         // the other CUs busy meanwhile.  Graphs/s fusing levels of up to 1024 /
         // 4096 / 8192 vertices: 48 graphs 484 / 444 / 376, 128 graphs 525 / 553
-        // / 490, 256 graphs 567 / 610 / 603, 768 graphs 566 / 612 / 668.
+        // / 490, 256 graphs 567 / 610 / 603, 768 graphs 566 / 612 / 668.  A limit
+        // that the caller has set to another value is taken as it is.
         int32_t fuse_n = std::min(tuning().batch_fuse_max, kTinyMaxN);
-        if (count < 512) fuse_n = std::min(fuse_n, count < 96 ? 1024 : 4096);
+        if (fuse_n == Tuning().batch_fuse_max && count < 512) fuse_n = std::min(fuse_n, count < 96 ? 1024 : 4096);
         if (fuse_n > 0 && !o.level_stats && o.refiner == 0) {
             // Groups of graphs (largest first, up to ~8 GB of hierarchies):
             // phase A coarsens and initially partitions each graph on the

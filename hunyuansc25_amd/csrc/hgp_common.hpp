@@ -103,8 +103,8 @@ struct Tuning {
     int32_t graph_max_vertices = 0;   // levels of <= this many vertices replay their Jet launch
                                       // sequences as HIP graphs (0: never)
     int32_t batch_fuse_max = 8192;    // hgp_partition_batch refines the levels of <= this many vertices
-                                      // of all graphs in one launch (0: per graph; at most 16384; small
-                                      // batches fuse smaller levels only)
+                                      // of all graphs in one launch (0: per graph; at most 16384; at the
+                                      // default, small batches fuse smaller levels only)
 };
 Tuning &tuning();
 

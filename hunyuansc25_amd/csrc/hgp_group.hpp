@@ -1,8 +1,8 @@
 // hgp_group.hpp -- lane groups of G threads working on one CSR row.
 //
 // Row-parallel kernels take their vertices from degree classes (RowBins):
-// rows of <= 8 entries get 8-lane groups, rows of <= 512 entries one wave,
-// longer rows one block per segment.  Group reductions are DPP moves and lane
+// rows of <= 8 entries get a lane each or 8-lane groups, rows of <= 512
+// entries 16 lanes up to a wave, longer rows one block per segment.  Group reductions are DPP moves and lane
 // swaps inside a wave for G <= 64 and go through LDS across the block's waves
 // for a whole block (G > 64).  Every reduction here uses a strict total order (or an integer
 // sum), so results do not depend on which lane saw which entry.
@@ -13,8 +13,8 @@
 namespace hgp {
 
 constexpr int kRowBS = 256;             // block size of row-parallel kernels
-// Degree classes of the rows of a level: 0 = <= 8 entries (8 lanes per row),
-// 1 = <= 32 (32 lanes), 2 = <= 512 (one wave), 3 = longer (segments of
+// Degree classes of the rows of a level: 0 = <= 8 entries,
+// 1 = <= 32, 2 = <= 512 (one wave), 3 = longer (segments of
 // kSegLen entries, a block of kSegBlk threads each).
 constexpr int64_t kBinSmall = 8;
 constexpr int64_t kBinHalf = 32;

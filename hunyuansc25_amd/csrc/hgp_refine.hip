@@ -1,10 +1,11 @@
 // hgp_refine.hip -- Jet k-way refinement of one level (k_refine,
 // hunyuangraph_GPU_krefine.h:4434-4882), projection, edge cut, part weights.
 //
-// Connectivity is recomputed from the CSR each iteration: kG lanes per
-// vertex accumulate edge weights per part in a dense LDS row of k ints, then
-// reduce the arg-max with xor shuffles.  Every decision reads the state at
-// the start of the iteration, and the candidate orders of the rebalancers are
+// Connectivity is recomputed from the CSR each iteration: rows of up to 8
+// entries by a lane each in registers, longer ones by a lane group, a wave or a
+// block that accumulates edge weights per part in a dense LDS row of k ints and
+// reduces the arg-max.  Every decision reads the state at the start of the
+// iteration, and the candidate orders of the rebalancers are
 // (part, gain bucket, vertex id) via a stable radix sort, so the result does
 // not depend on scheduling.
 #include "hgp_graph.hpp"

@@ -184,7 +184,7 @@ typedef struct hgp_tuning {
     int32_t tiny_max_vertices;  /* levels of <= this many vertices (k <= 256) run the
                                    whole refinement loop in one block (0..4096, default 512) */
     int32_t few_rows;           /* levels with <= this many rows of <= 512 entries run
-                                   those rows in one launch (default 8192) */
+                                   those rows in one launch (default 16384) */
     int32_t fill_waves;         /* waves the wave-per-row kernels spread a level over (default 8192) */
     int32_t seg_grid;           /* grid cap of the long-row segment kernels (default 32768) */
     int32_t batch_lanes;        /* lanes of hgp_partition_batch when it is passed <= 0 (1..64, default 8) */
@@ -197,7 +197,9 @@ typedef struct hgp_tuning {
     int32_t batch_fuse_max_vertices; /* hgp_partition_batch refines the levels of <= this many
                                    vertices (the coarse end of each hierarchy, k <= 256) of
                                    every graph of a group in one launch, a block per graph
-                                   (0: each graph on its own; 0..16384, default 8192) */
+                                   (0: each graph on its own; 0..16384, default 8192;
+                                   at the default, batches of fewer than 96 / 512 graphs
+                                   stop at 1024 / 4096) */
 } hgp_tuning;
 int hgp_get_tuning(hgp_tuning *t);
 int hgp_set_tuning(const hgp_tuning *t);
