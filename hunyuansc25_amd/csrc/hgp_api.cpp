@@ -1230,7 +1230,7 @@ int hgp_initpart(int32_t n, const int64_t *xadj, const int32_t *adjncy, const in
         if (n == 0) return;
         std::lock_guard<std::mutex> lk(g_api_mu);
         Ctx &c = context(o.device);
-        size_t extra = (size_t)std::min(p.trials, n) * (size_t)n * 16;
+        size_t extra = (size_t)std::min(p.trials, n) * (size_t)n * 16 + dense_trial_bytes(n);
         with_arena(c, estimate_arena(n, xadj[n], k, true) + extra, [&] {
             DevGraph g = upload(c, n, xadj, adjncy, vwgt, adjwgt);
             int32_t *dw = c.arena.lalloc<int32_t>((size_t)n);

@@ -60,6 +60,8 @@ DevGraph contract(Ctx &c, const DevGraph &g, const int32_t *match, const int32_t
 
 // Recursive bisection of g into k parts; where (device, n) out.
 void initial_partition(Ctx &c, const DevGraph &g, int32_t k, const Params &p, int32_t *where);
+// Arena bytes of the trials' matrices, taken where they are free (0: lists only).
+size_t dense_trial_bytes(int32_t n);
 
 // ---------------------------------------------------------------- refinement
 

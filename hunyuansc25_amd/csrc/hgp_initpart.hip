@@ -556,8 +556,9 @@ __global__ void __launch_bounds__(kWave) k_ip_trials_heap(const int32_t *__restr
 //    VALU;
 //  * 256 threads for node graphs of kWideTrial vertices and more, one wave
 //    below, where a step has no work for more.
-// Used where the dense trials below are not: node graphs of more than kDenseN
-// vertices, or rows that do not ascend.
+// Used where the dense trials below are not: coarsest graphs of more than
+// kDenseN vertices, rows that do not ascend, an arena without room for the
+// matrices.
 constexpr int32_t kWideTrial = 128;
 constexpr uint8_t kStSide = 1, kStMoved = 2, kStAlone = 4;   // state byte: side, queued or moved, no edges
 
@@ -1533,6 +1534,13 @@ bool fm_uses_heap(int32_t fm_kind, int32_t n)
 
 }  // namespace
 
+// The matrices and, on top, what the scans after them take.
+size_t dense_trial_bytes(int32_t n)
+{
+    if (n > kDenseN) return 0;
+    return sizeof(int32_t) * (size_t)(n * (dense_stride(n) + 3) + n * (dense_words(n) + 1)) + (64 << 10);
+}
+
 void initial_partition(Ctx &c, const DevGraph &g, int32_t k, const Params &p, int32_t *where)
 {
     int32_t n = g.n;
@@ -1598,14 +1606,6 @@ void initial_partition(Ctx &c, const DevGraph &g, int32_t k, const Params &p, in
     int32_t *total = c.arena.ralloc<int32_t>(1);
     int64_t maxtrials = (int64_t)std::min(p.trials, n);
     uint8_t *trial_where = c.arena.ralloc<uint8_t>((size_t)(maxtrials * n));
-    // dense trials: the graph as matrices, rebuilt per depth node by node
-    const bool dense = !heap && g.ascending && n <= kDenseN;
-    int32_t *W = nullptr;
-    uint32_t *B = nullptr;
-    if (dense) {
-        W = c.arena.ralloc<int32_t>((size_t)(n * (dense_stride(n) + 3)));
-        B = c.arena.ralloc<uint32_t>((size_t)(n * (dense_words(n) + 1)));
-    }
     char *gscratch = nullptr;
     if (n > lds_cap) {
         // sum over nodes of T * round256(trial_bytes(nn)): trial_bytes is affine
@@ -1634,6 +1634,19 @@ void initial_partition(Ctx &c, const DevGraph &g, int32_t k, const Params &p, in
     int32_t *f0 = c.arena.ralloc<int32_t>((size_t)n);
     int32_t *pos = c.arena.ralloc<int32_t>((size_t)n);
     int64_t *ndeg = c.arena.ralloc<int64_t>((size_t)n);
+    // dense trials: the graph as matrices, rebuilt per depth node by node.  They
+    // take 69 MB at 4096 vertices, more than the whole estimate of a small graph
+    // whose coarsening stops early (pairs, mostly isolated vertices), and the
+    // lists a few MB for the same moves: dense only where the arena as it is has
+    // room for them, so that no call grows its arena or its claim on a budget
+    // for them.
+    const bool dense = !heap && g.ascending && n <= kDenseN && c.arena.free_bytes() >= dense_trial_bytes(n);
+    int32_t *W = nullptr;
+    uint32_t *B = nullptr;
+    if (dense) {
+        W = c.arena.ralloc<int32_t>((size_t)(n * (dense_stride(n) + 3)));
+        B = c.arena.ralloc<uint32_t>((size_t)(n * (dense_words(n) + 1)));
+    }
 
     unsigned gv = grid_for(n, 256);
     k_ip_init<<<grid_groups(n, kWave), kRowBS, 0, c.stream>>>(n, g.vwgt, g.xadj, g.adjwgt, node_of[0], label[0],

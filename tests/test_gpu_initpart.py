@@ -43,3 +43,29 @@ def test_trials_of_rows_out_of_order(hgp, orc, n):
     w = hgp.initpart(x, a, vw, aw, 5, seed=2, trials=8)
     o = orc.dga_initpart(x, a, vw, aw, 5, seed=2, trials=8)
     np.testing.assert_array_equal(w, o)
+
+
+def test_dense_trials_run(hgp):
+    """The stage entry point has room for the matrices of up to 4096 vertices."""
+    for n, dense in ((2, True), (4096, True), (4097, False)):
+        x, a, vw, aw = _graph(n, n, clusters=False)
+        hgp.ktimer_enable(True)
+        hgp.initpart(x, a, vw, aw, 2, seed=5, trials=3)
+        ran = hgp.ktimer_report()
+        hgp.ktimer_enable(False)
+        assert ("k_ip_dense" in ran) == dense, n
+
+
+def test_matrices_yield_to_the_memory_there_is(hgp, orc):
+    """The dense trials' matrices (66 MB here) are taken only where the arena
+    has the room: a graph whose coarsening stops after one step, at 4050
+    vertices, is served within a budget that its lists need a few MB of."""
+    n = 8100
+    pairs, links = [(v, v + 1) for v in range(0, n, 2)], [(v + 1, v + 2) for v in range(0, 3600, 4)]
+    x, a, aw = csr_from_edges(n, pairs + links, [5] * len(pairs) + [1] * len(links))
+    vw = np.ones(n, np.int32)
+    ref, _ = orc.dga_partition(x, a, 2, vw, aw, seed=3)
+    with hgp.Server(slots=1, budget_bytes=71_000_000) as s:
+        part, st, _ = s.wait(s.submit(x, a, 2, vw, aw, seed=3))
+    assert st["coarsest_n"] == 4050
+    np.testing.assert_array_equal(part, ref)
