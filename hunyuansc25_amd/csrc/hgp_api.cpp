@@ -715,9 +715,10 @@ int hgp_partition_batch(int32_t count, const int32_t *n, const int64_t *const *x
         // the other CUs busy meanwhile.  Graphs/s fusing levels of up to 1024 /
         // 4096 / 8192 vertices: 48 graphs 484 / 444 / 376, 128 graphs 525 / 553
         // / 490, 256 graphs 567 / 610 / 603, 768 graphs 566 / 612 / 668.  A limit
-        // that the caller has set to another value is taken as it is.
-        int32_t fuse_n = std::min(tuning().batch_fuse_max, kTinyMaxN);
-        if (fuse_n == Tuning().batch_fuse_max && count < 512) fuse_n = std::min(fuse_n, count < 96 ? 1024 : 4096);
+        // that the caller has set is taken as it is.
+        int32_t fuse_n = tuning().batch_fuse_max;
+        if (fuse_n < 0) fuse_n = count < 96 ? 1024 : count < 512 ? 4096 : 8192;
+        fuse_n = std::min(fuse_n, kTinyMaxN);
         if (fuse_n > 0 && !o.level_stats && o.refiner == 0) {
             // Groups of graphs (largest first, up to ~8 GB of hierarchies):
             // phase A coarsens and initially partitions each graph on the
@@ -984,7 +985,7 @@ int hgp_set_tuning(const hgp_tuning *t)
         if (!t) throw Error{-1, "tuning is NULL"};
         if (t->tiny_max_vertices < 0 || t->tiny_max_vertices > 4096 || t->few_rows < 0 || t->fill_waves < 1 ||
             t->seg_grid < 1 || t->batch_lanes < 1 || t->batch_lanes > 64 || t->hub_track < 0 || t->hub_track > 1 ||
-            t->graph_max_vertices < 0 || t->batch_fuse_max_vertices < 0 || t->batch_fuse_max_vertices > kTinyMaxN)
+            t->graph_max_vertices < 0 || t->batch_fuse_max_vertices < -1 || t->batch_fuse_max_vertices > kTinyMaxN)
             throw Error{-1, "tuning value out of range"};
         std::lock_guard<std::mutex> lk(g_api_mu);
         Tuning &x = tuning();

@@ -102,9 +102,9 @@ struct Tuning {
                                  // iterations (k <= 512) instead of rebuilding them in each selection
     int32_t graph_max_vertices = 0;   // levels of <= this many vertices replay their Jet launch
                                       // sequences as HIP graphs (0: never)
-    int32_t batch_fuse_max = 8192;    // hgp_partition_batch refines the levels of <= this many vertices
-                                      // of all graphs in one launch (0: per graph; at most 16384; at the
-                                      // default, small batches fuse smaller levels only)
+    int32_t batch_fuse_max = -1;      // hgp_partition_batch refines the levels of <= this many vertices
+                                      // of all graphs in one launch (0: per graph; at most 16384; -1: by
+                                      // the batch's size)
 };
 Tuning &tuning();
 

@@ -197,9 +197,9 @@ typedef struct hgp_tuning {
     int32_t batch_fuse_max_vertices; /* hgp_partition_batch refines the levels of <= this many
                                    vertices (the coarse end of each hierarchy, k <= 256) of
                                    every graph of a group in one launch, a block per graph
-                                   (0: each graph on its own; 0..16384, default 8192;
-                                   at the default, batches of fewer than 96 / 512 graphs
-                                   stop at 1024 / 4096) */
+                                   (0: each graph on its own; 1..16384; -1, the default:
+                                   1024 in batches of fewer than 96 graphs, 4096 of fewer
+                                   than 512, 8192 beyond) */
 } hgp_tuning;
 int hgp_get_tuning(hgp_tuning *t);
 int hgp_set_tuning(const hgp_tuning *t);

@@ -150,3 +150,21 @@ def test_tuning_round_trip_and_range(hgp):
         assert hgp.get_tuning()["batch_lanes"] == 3       # a refused setting changes nothing
     finally:
         hgp.set_tuning(**t0)
+
+
+def test_fuse_limit_left_to_itself(hgp):
+    """No limit is -1, which no setting of the caller's stands for, and
+    survives a change of other knobs."""
+    t0 = hgp.get_tuning()
+    assert t0["batch_fuse_max_vertices"] == -1
+    try:
+        hgp.set_tuning(batch_lanes=5)
+        assert hgp.get_tuning()["batch_fuse_max_vertices"] == -1
+        for fuse in (0, 8192, 16384, -1):
+            hgp.set_tuning(batch_fuse_max_vertices=fuse)
+            assert hgp.get_tuning()["batch_fuse_max_vertices"] == fuse
+        with pytest.raises(hgp.HgpError) as e:
+            hgp.set_tuning(batch_fuse_max_vertices=-2)
+        assert e.value.code == -1
+    finally:
+        hgp.set_tuning(**t0)

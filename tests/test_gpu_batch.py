@@ -75,3 +75,26 @@ def test_batch_fused_small_levels_match_alone(hgp):
                 assert stats[i]["cut"] > 0 and stats[i]["max_pwgt"] > 0
     finally:
         hgp.set_tuning(**t0)
+
+
+def test_fuse_limit_that_the_caller_sets(hgp):
+    """The limit left to itself (-1) fuses levels of up to 1024 vertices in a
+    batch of two graphs; 8192 set by the caller is 8192: every level of a
+    3600-vertex grid is refined in the fused launch."""
+    gs, ks = [hgp.gen_grid2d(60, 60)] * 2, [8, 8]
+    t0 = hgp.get_tuning()
+    assert t0["batch_fuse_max_vertices"] == -1
+    ran = {}
+    try:
+        for fuse in (-1, 8192):
+            hgp.set_tuning(batch_fuse_max_vertices=fuse)
+            hgp.ktimer_enable(True)
+            hgp.partition_batch(gs, ks, lanes=1, seed=4)
+            ran[fuse] = hgp.ktimer_report()
+            hgp.ktimer_enable(False)
+    finally:
+        hgp.set_tuning(**t0)
+    for r in ran.values():
+        assert r["k_jet_tiny_batch"][0] == 1
+    assert any(name.startswith("k_jet_select") for name in ran[-1])
+    assert not any(name.startswith("k_jet_select") for name in ran[8192])
