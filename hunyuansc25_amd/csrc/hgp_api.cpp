@@ -490,10 +490,10 @@ void fused_phase_a(Ctx &c, const hgp_options &o, const HostJob &j, int32_t fuse_
     HGP_CHECK_HIP(hipSetDevice(c.device));
     if (j.n == 0) return;
     if (j.k == 1 || j.k > kTinyMaxK) {
-        exec_job(c, o, j, job_bytes(j));
+        exec_job(c, o, j, job_bytes(j) + kMatrixRoom);
         return;
     }
-    with_arena(c, job_bytes(j), [&] {
+    with_arena(c, job_bytes(j) + kMatrixRoom, [&] {
         auto t0 = std::chrono::steady_clock::now();
         const size_t m0 = c.arena.left_mark();
         f.lv.assign(1, upload(c, j.n, j.xadj, j.adjncy, j.vwgt, j.adjwgt));
@@ -668,7 +668,7 @@ int hgp_partition(int32_t n, const int64_t *xadj, const int32_t *adjncy, const i
         std::lock_guard<std::mutex> lk(g_api_mu);
         HostJob j{n, xadj, adjncy, vwgt, adjwgt, k, part, stats};
         check_job(o, j);
-        if (n > 0) exec_job(context(o.device), o, j, job_bytes(j));
+        if (n > 0) exec_job(context(o.device), o, j, job_bytes(j) + kMatrixRoom);
     });
 }
 
@@ -801,7 +801,7 @@ int hgp_partition_batch(int32_t count, const int32_t *n, const int64_t *const *x
                     HostJob j{n[i], xadj[i], adjncy[i], vwgt ? vwgt[i] : nullptr, adjwgt ? adjwgt[i] : nullptr, k[i],
                               part[i], stats ? stats + i : nullptr};
                     check_job(o, j);
-                    exec_job(*c, o, j, job_bytes(j));
+                    exec_job(*c, o, j, job_bytes(j) + kMatrixRoom);
                 });
                 st[i] = rc;
                 if (rc != HGP_OK) msg[i] = last_error_text();
@@ -837,7 +837,7 @@ int hgp_partition_device(int32_t n, const int64_t *d_xadj, const int32_t *d_adjn
         HGP_CHECK_HIP(hipMemcpy(&m, d_xadj + n, sizeof(int64_t), hipMemcpyDeviceToHost));
         if (m < 0) throw Error{-1, "xadj[n] < 0"};
         if (m > INT32_MAX) throw Error{-4, "more than 2^31-1 directed entries"};
-        with_arena(c, estimate_arena(n, m, k, false), [&] {
+        with_arena(c, estimate_arena(n, m, k, false) + kMatrixRoom, [&] {
             // the CSR invariants of check_graph (hunyuangraph_GPU_match.h:1718-1800),
             // checked on the device before any kernel gathers through it
             check_graph_device(c, n, d_xadj, d_adjncy, d_vwgt, d_adjwgt, o.validate != 0);

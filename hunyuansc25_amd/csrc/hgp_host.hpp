@@ -86,6 +86,12 @@ void check_options(const hgp_options &o, int32_t k);
 // starts with.
 size_t resident_job_bytes(int32_t n, int64_t m, int32_t k);
 
+// Beside the bytes of job_bytes and resident_job_bytes, for the matrices of the
+// dense bisection trials: 69 MB for a coarsest graph of 4096 vertices, where a
+// small graph's estimate (64 MB, and what its size adds) leaves them 62.  A run
+// without it takes the trials on lists when it has to.
+constexpr size_t kMatrixRoom = (size_t)12 << 20;
+
 // Throws Error{-1/-4} for invalid options or CSR; touches no device.
 void check_job(const hgp_options &o, const HostJob &j);
 // Device arena bytes the job is run with first.

@@ -182,6 +182,8 @@ struct hgp_server {
             queue.pop_front();
             Job *job = jobs.get(t);
             size_t need = job->bytes;
+            if (reserved() - held((size_t)w) + std::max(held((size_t)w), need + hgp::kMatrixRoom) <= budget)
+                need += hgp::kMatrixRoom;
             busy[w] = 1;
             claim[w] = std::max(ctx[w]->arena.capacity(), need);
             peak = std::max(peak, reserved());

@@ -57,15 +57,22 @@ def test_dense_trials_run(hgp):
 
 
 def test_matrices_yield_to_the_memory_there_is(hgp, orc):
-    """The dense trials' matrices (66 MB here) are taken only where the arena
+    """The dense trials' matrices (68 MB here) are taken only where the arena
     has the room: a graph whose coarsening stops after one step, at 4050
-    vertices, is served within a budget that its lists need a few MB of."""
+    vertices, is served within a budget that its lists need a few MB of, and
+    with its matrices, at the first go, where the budget has the room."""
     n = 8100
     pairs, links = [(v, v + 1) for v in range(0, n, 2)], [(v + 1, v + 2) for v in range(0, 3600, 4)]
     x, a, aw = csr_from_edges(n, pairs + links, [5] * len(pairs) + [1] * len(links))
     vw = np.ones(n, np.int32)
     ref, _ = orc.dga_partition(x, a, 2, vw, aw, seed=3)
-    with hgp.Server(slots=1, budget_bytes=71_000_000) as s:
-        part, st, _ = s.wait(s.submit(x, a, 2, vw, aw, seed=3))
-    assert st["coarsest_n"] == 4050
-    np.testing.assert_array_equal(part, ref)
+    for budget, dense in ((71_000_000, False), (1 << 30, True)):
+        hgp.ktimer_enable(True)
+        with hgp.Server(slots=1, budget_bytes=budget) as s:
+            part, st, _ = s.wait(s.submit(x, a, 2, vw, aw, seed=3))
+        ran = hgp.ktimer_report()
+        hgp.ktimer_enable(False)
+        assert st["coarsest_n"] == 4050
+        np.testing.assert_array_equal(part, ref)
+        assert ran.get("k_ip_dense", (0,))[0] == int(dense)
+        assert ran["k_ip_trials"][0] == 1 and st["arena_bytes"] < 90_000_000
