@@ -2,6 +2,7 @@
 // uncoarsen/refine) and the C ABI.
 #include "hunyuangraph.h"
 
+#include "hgp_batchplan.hpp"
 #include "hgp_check.hpp"
 #include "hgp_graph.hpp"
 #include "hgp_prims.hpp"
@@ -710,30 +711,19 @@ int hgp_partition_batch(int32_t count, const int32_t *n, const int64_t *const *x
             work(ctx[0]);
             for (auto &t : th) t.join();
         };
-        // The fused launch lasts as long as its slowest graph, which one CU
-        // refines alone: worth it for the larger levels once the group keeps
-        // the other CUs busy meanwhile.  Graphs/s fusing levels of up to 1024 /
-        // 4096 / 8192 vertices: 48 graphs 484 / 444 / 376, 128 graphs 525 / 553
-        // / 490, 256 graphs 567 / 610 / 603, 768 graphs 566 / 612 / 668.  A limit
-        // that the caller has set is taken as it is.
-        int32_t fuse_n = tuning().batch_fuse_max;
-        if (fuse_n < 0) fuse_n = count < 96 ? 1024 : count < 512 ? 4096 : 8192;
-        fuse_n = std::min(fuse_n, kTinyMaxN);
-        if (fuse_n > 0 && !o.level_stats && o.refiner == 0) {
+        if (tuning().batch_fuse_max != 0 && !o.level_stats && o.refiner == 0) {
             // Groups of graphs (largest first, up to ~8 GB of hierarchies):
             // phase A coarsens and initially partitions each graph on the
             // lanes and keeps its hierarchy; one launch refines the small
             // levels of every graph of the group (a block per graph);
             // phase C refines the rest on the lanes.
-            const size_t budget = (size_t)8 << 30;
-            for (int32_t g0 = 0; g0 < count;) {
-                int32_t g1 = g0;
-                size_t gb = 0;
-                while (g1 < count && (g1 == g0 || gb < budget)) {
-                    const int32_t i = order[(size_t)g1];
-                    gb += xadj[i] && n[i] >= 0 ? (size_t)(24 * (xadj[i][n[i]] + 2 * (int64_t)n[i])) + (1 << 20) : 0;
-                    g1++;
-                }
+            std::vector<size_t> bytes((size_t)count, 0);
+            for (int32_t t = 0; t < count; t++) {
+                const int32_t i = order[(size_t)t];
+                if (xadj[i] && n[i] >= 0) bytes[(size_t)t] = (size_t)(24 * (xadj[i][n[i]] + 2 * (int64_t)n[i])) + (1 << 20);
+            }
+            for (const BatchGroup &grp : plan_batch(bytes, (size_t)8 << 30, tuning().batch_fuse_max)) {
+                const int32_t g0 = grp.g0, g1 = grp.g1, fuse_n = std::min(grp.fuse, kTinyMaxN);
                 std::vector<FusedGraph> fg((size_t)(g1 - g0));
                 over_lanes(g1 - g0, [&](Ctx *c, int32_t t) {
                     const int32_t i = order[(size_t)(g0 + t)];
@@ -783,7 +773,6 @@ int hgp_partition_batch(int32_t count, const int32_t *n, const int64_t *const *x
                 });
                 for (FusedGraph &f : fg)
                     if (f.buf) (void)hipFree(f.buf);
-                g0 = g1;
             }
             if (status) std::copy(st.begin(), st.end(), status);
             for (int32_t i = 0; i < count; i++)

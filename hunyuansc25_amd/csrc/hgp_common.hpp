@@ -104,7 +104,7 @@ struct Tuning {
                                       // sequences as HIP graphs (0: never)
     int32_t batch_fuse_max = -1;      // hgp_partition_batch refines the levels of <= this many vertices
                                       // of all graphs in one launch (0: per graph; at most 16384; -1: by
-                                      // the batch's size)
+                                      // the group's size)
 };
 Tuning &tuning();
 

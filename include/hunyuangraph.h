@@ -198,7 +198,7 @@ typedef struct hgp_tuning {
                                    vertices (the coarse end of each hierarchy, k <= 256) of
                                    every graph of a group in one launch, a block per graph
                                    (0: each graph on its own; 1..16384; -1, the default:
-                                   1024 in batches of fewer than 96 graphs, 4096 of fewer
+                                   1024 in groups of fewer than 96 graphs, 4096 of fewer
                                    than 512, 8192 beyond) */
 } hgp_tuning;
 int hgp_get_tuning(hgp_tuning *t);
