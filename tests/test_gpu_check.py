@@ -160,9 +160,10 @@ def test_evaluate_rejects(hgp, torch_mod):
 
 @pytest.mark.parametrize("shape", ["edges", "empties", "hub", "one"])
 def test_rows_at_tile_edges(hgp, torch_mod, shape):
-    """Rows that start and end at the borders of the 64- and 512-entry pieces
-    the walkers take, runs of more than 64 empty rows, a row over several
-    pieces: the check names the right vertex, the evaluation the right cut."""
+    """Rows that start and end at the borders of the 64-entry pieces and near
+    those of the 1024-entry tiles the walkers take, runs of more than 64 empty
+    rows, a row over several tiles: the check names the right vertex, the
+    evaluation the right cut."""
     lens = {"edges": [512, 511, 1, 513, 511, 64, 63, 1, 65, 447, 512, 1024, 1],
             "empties": [0] * 70 + [3] + [0] * 200 + [509] + [0] * 64 + [512, 1] + [0] * 130 + [7] + [0] * 65,
             "hub": [5, 300000, 2, 0, 1], "one": [1, 1]}[shape]
@@ -183,3 +184,40 @@ def test_rows_at_tile_edges(hgp, torch_mod, shape):
         bad = aw.copy()
         bad[j] = 0
         _expect_check(hgp, torch_mod, x, a, vw, bad, False, f"edge weight < 1 in row {row[j]}")
+
+
+@pytest.mark.parametrize("m_min", [8_400_000, 17_500_000])
+def test_rows_carried_from_tile_to_tile(hgp, torch_mod, m_min):
+    """From 8192 x 1024 entries on a wave walks several tiles of 1024 entries
+    and carries its row from one to the next: rows that start and end at, just
+    before and just after tile borders, over several tiles, and runs of more
+    than 64 empty rows before, at and after a border."""
+    rng = np.random.default_rng(m_min)
+    piece = [1024, 1023, 1, 1025, 1023, 0, 1024] + [0] * 70 + [1024, 3000, 72] + [0] * 130 + [1, 1023] + [0] * 64
+    piece += [1, 1022, 1, 5000, 120, 1024] + [0] * 300
+    lens, m = [], 0
+    while m < m_min:
+        p = piece + [int(v) for v in rng.integers(0, 40, 300)] + [0] * int(rng.integers(60, 140))
+        p.append(1024 - sum(p) % 1024)   # the next piece starts at a border
+        lens += p
+        m += sum(p)
+    n = len(lens)
+    x = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    row = np.repeat(np.arange(n, dtype=np.int32), lens)
+    a = ((row + 1 + rng.integers(0, n - 1, size=m, dtype=np.int32)) % n).astype(np.int32)
+    aw = rng.integers(1, 9, size=m, dtype=np.int32)
+    vw, where = np.ones(n, np.int32), rng.integers(0, 300, size=n).astype(np.int32)
+    d = _dev(torch_mod, x, a, vw, aw, where)
+    out = torch_mod.zeros(4, dtype=torch_mod.int64, device="cuda:0")
+    hgp.evaluate_device(n, *(_ptr(d[i]) for i in (0, 1, 3, 2, 4)), 300, out.data_ptr())
+    cut = int(aw[where[row] != where[a]].sum(dtype=np.int64)) // 2
+    assert out.tolist() == [cut, int(np.bincount(where, minlength=300).max()), 0, 0]
+    hgp.check_graph_device(n, *(_ptr(t) for t in d[:4]))
+    at = rng.integers(0, m // 1024, 6) * 1024   # tile borders, the row each side of them and rows' ends near them
+    for j in sorted({0, m - 1, *(int(t) + o for t in at for o in (-1, 0, 1) if 0 <= int(t) + o < m),
+                     *(int(v) for v in x[rng.integers(1, n, 8)] - 1 if v >= 0)}):
+        d[3][j] = 0
+        with pytest.raises(hgp.HgpError) as e:
+            hgp.check_graph_device(n, *(_ptr(t) for t in d[:4]))
+        assert f"edge weight < 1 in row {row[j]}" in str(e.value), (j, str(e.value))
+        d[3][j] = int(aw[j])
