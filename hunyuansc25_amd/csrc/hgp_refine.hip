@@ -901,7 +901,7 @@ __global__ void __launch_bounds__(Hot ? kHotBS : kRowBS) k_jet_select_w(const in
             const eid_t b = A.xadj[mv];
             mb = (int32_t)b;
             md = (int32_t)(A.xadj[mv + 1] - b);
-            kbytes += 16 + 12 * (uint64_t)md;
+            kbytes += 16 + (Hot ? 8 : 12) * (uint64_t)md;
         }
         uint64_t todo = __ballot(mel);
         if constexpr (Q) {
@@ -1170,7 +1170,7 @@ __global__ void __launch_bounds__(kHotBS) k_jet_select_seg_hot(RowSegs S, SelArg
             if (lane == 0 && mi < 0) sel_decide(A, C, mode, v, rr, false, 0, PartKey{0, -1});
             continue;
         }
-        if (lane == 0) kbytes += 8 + 12 * (uint64_t)(e - b);
+        if (lane == 0) kbytes += 8 + 8 * (uint64_t)(e - b);
         int32_t own = 0;
         for (eid_t c0 = b; c0 < e; c0 += (eid_t)T * kWave) {
             int32_t u[T], w[T], q[T];
@@ -2121,20 +2121,35 @@ void hot_order(Ctx &c, const DevGraph &g, HotParts &h)
     c.arena.right_release(mark);
 }
 
-// A launch of k_jet_select_w over nw rows with `ent` entries.
-void launch_select_w(Ctx &c, const SelArgs &A, const HotParts &h, const int32_t *list, int64_t nw, int64_t ent)
+// Whether k_jet_select_w over `ent` entries holds the hot part ids in LDS, and
+// with room for how many rows a wave: four (k <= 334), one (k <= 1322).  One row
+// a wave with them beats four without: R-MAT with 2^18 vertices, k = 340 / 400 /
+// 512, 36.0 / 36.6 / 34.8 ms a partition against 37.1 / 37.4 / 35.8.
+enum HotRows : int32_t { kHotNone = 0, kHotOne = 1, kHotFour = 4 };
+
+inline size_t hot_w_lds(int32_t k, int32_t rows) { return sizeof(int32_t) * (kHotBS / kWave) * (size_t)rows * (size_t)k; }
+
+HotRows hot_rows(const SelArgs &A, int64_t ent)
+{
+    const size_t fixed = kHotBytes + sizeof(int3) * kHotBS + 64 + (((size_t)A.k + 3) & ~(size_t)3);
+    if (!A.hot || ent < kHotEntries) return kHotNone;
+    if (A.k <= kQuarterK && fixed + hot_w_lds(A.k, 4) <= kLdsBytes) return kHotFour;
+    return fixed + hot_w_lds(A.k, 1) <= kLdsBytes ? kHotOne : kHotNone;
+}
+
+// A launch of k_jet_select_w over nw rows.
+void launch_select_w(Ctx &c, const SelArgs &A, HotRows hot, const int32_t *list, int64_t nw)
 {
     const int k = A.k;
-    const size_t tg = ((size_t)k + 3) & ~(size_t)3, fixed = kHotBytes + sizeof(int3) * kHotBS + 64;
+    const size_t tg = ((size_t)k + 3) & ~(size_t)3;
     const bool q = k <= kQuarterK;
-    if (A.hot && ent >= kHotEntries) {
-        const size_t one = 16 * sizeof(int32_t) * (size_t)k, four = 4 * one;
+    if (hot != kHotNone) {
         const int32_t rpw = (int32_t)std::max<int64_t>(4, std::min<int64_t>(kWave, nw / (kHotBlocks * 16 * 4)));
         const unsigned blocks = (unsigned)std::min<int64_t>((nw + 16 * rpw - 1) / (16 * rpw), kHotBlocks);
-        if (q && fixed + four + tg <= kLdsBytes)
-            return k_jet_select_w<true, true><<<blocks, kHotBS, four + tg, c.stream>>>(list, nw, rpw, A);
-        if (fixed + one + tg <= kLdsBytes)
-            return k_jet_select_w<false, true><<<blocks, kHotBS, one + tg, c.stream>>>(list, nw, rpw, A);
+        const size_t lds = hot_w_lds(k, hot) + tg;
+        if (hot == kHotFour) k_jet_select_w<true, true><<<blocks, kHotBS, lds, c.stream>>>(list, nw, rpw, A);
+        else k_jet_select_w<false, true><<<blocks, kHotBS, lds, c.stream>>>(list, nw, rpw, A);
+        return;
     }
     const int32_t rpw = rows_per_wave(nw);
     const unsigned blocks = wave_blocks(nw, rpw, 4096);
@@ -2152,12 +2167,13 @@ void launch_select(Ctx &c, const DevGraph &g, int32_t k, const int32_t *where, c
               dest, pregain, key, nullptr, wq, ab, pd16, pd32, h.cap, h.held};
     const size_t tg_bytes = ((size_t)k + 3) & ~(size_t)3;   // part flags of the selection kernels
     // fixed bytes: ids, where, pwgts[p], vwgt, the decision (24 per row); eligible rows add xadj and
-    // 12 B per entry (adjncy, adjwgt, where gather) in the kernel
+    // 12 B per entry (adjncy, adjwgt, where gather) in the kernel, 8 B where the hot part ids are in LDS
     if (b.few()) {
         if (int64_t nw = b.short_rows()) {
-            KScope ks(c, "k_jet_select_few", 24.0 * (double)nw, true);
+            const HotRows hot = hot_rows(A, b.ent[0] + b.ent[1] + b.ent[2]);
+            KScope ks(c, hot ? "k_jet_select_few_hot" : "k_jet_select_few", 24.0 * (double)nw, true);
             A.kb = ks.dev();
-            launch_select_w(c, A, h, b.list(0), nw, b.ent[0] + b.ent[1] + b.ent[2]);
+            launch_select_w(c, A, hot, b.list(0), nw);
             HGP_LAUNCH_CHECK();
         }
     }
@@ -2184,9 +2200,10 @@ void launch_select(Ctx &c, const DevGraph &g, int32_t k, const int32_t *where, c
         HGP_LAUNCH_CHECK();
     }
     if (int64_t nw = b.few() ? 0 : (quarter ? 0 : b.count(1)) + b.count(2)) {
-        KScope ks(c, "k_jet_select_w", 24.0 * (double)nw, true);
+        const HotRows hot = hot_rows(A, (quarter ? 0 : b.ent[1]) + b.ent[2]);
+        KScope ks(c, hot ? "k_jet_select_w_hot" : "k_jet_select_w", 24.0 * (double)nw, true);
         A.kb = ks.dev();
-        launch_select_w(c, A, h, quarter ? b.list(2) : b.list(1), nw, (quarter ? 0 : b.ent[1]) + b.ent[2]);
+        launch_select_w(c, A, hot, quarter ? b.list(2) : b.list(1), nw);
         HGP_LAUNCH_CHECK();
     }
     if (hc.hidx) {
@@ -2200,10 +2217,11 @@ void launch_select(Ctx &c, const DevGraph &g, int32_t k, const int32_t *where, c
         HGP_LAUNCH_CHECK();
     } else if (g.segs.nseg) {
         {
-            KScope ks(c, "k_jet_select_seg", 24.0 * (double)g.segs.nseg, true);
+            const size_t lds = hot_w_lds(k, 1) + tg_bytes;
+            const bool hot = A.hot && b.ent[kClsLong] >= kHotEntries && kHotBytes + 64 + lds <= kLdsBytes;
+            KScope ks(c, hot ? "k_jet_select_seg_hot" : "k_jet_select_seg", 24.0 * (double)g.segs.nseg, true);
             A.kb = ks.dev();
-            const size_t lds = 16 * sizeof(int32_t) * (size_t)k + tg_bytes;
-            if (A.hot && b.ent[kClsLong] >= kHotEntries && kHotBytes + 64 + lds <= kLdsBytes)
+            if (hot)
                 k_jet_select_seg_hot<<<(unsigned)std::min<int64_t>((g.segs.nseg + 15) / 16, kHotBlocks), kHotBS, lds,
                                        c.stream>>>(g.segs, A, conn);
             else
