@@ -16,11 +16,15 @@
 // a tile in LDS and scans the counts, so every lane knows the rows of its
 // entries and the wave goes over xadj once, 64 rows a load.  Following the
 // rows one by one after a binary search per tile, chains of dependent reads,
-// bounded both walks: R-MAT with 2^22 vertices and 52M entries is checked in
-// 0.19 ms (1.0 ms so; 2.2 TB/s now), R-MAT with 2^20 vertices and 33M entries
-// evaluated in 0.24 ms (0.47 ms so; the part gathers, at 190 G/s at best, take
-// 0.18 ms of it).  16 entries a lane take registers the occupancy needs: 0.25
-// ms for the check.
+// bounded both walks.  Calls, so and now: check of R-MAT with 2^22 vertices and
+// 134M entries 1017 and 297 us (3.8 TB/s), evaluation of R-MAT with 2^20
+// vertices and 33.5M entries 452 and 256 us (the part gathers, at 190 G/s at
+// best, take 180 us of it).  16 entries a lane cost occupancy (150 and 92
+// VGPRs, 3 and 5 waves a SIMD; 8 entries: 77 and 58, 6 and 8 waves), 8 cost
+// twice the tiles: they take 275 us for that check and 249 for that evaluation,
+// but 60 us instead of 56 for the check of a banded graph of 2.1M entries (36
+// instead of 32 evaluated) and 137 instead of 123 for the symmetric one of a
+// 3-D RGG of 12M.
 #include "hgp_check.hpp"
 #include "hgp_host.hpp"
 

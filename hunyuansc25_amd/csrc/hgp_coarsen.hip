@@ -701,7 +701,7 @@ __global__ void k_rep(int32_t n, const eid_t *__restrict__ xadj, const wgt_t *__
 // by cmap.  Each row is sorted by coarse id, entries equal to c are dropped
 // and equal ids are merged by summing weights; the merged row is written at
 // toff[c] (the concatenation's offset) of tadj/twgt and its length to ccnt[c].
-// Rows of <= 64 entries sort in registers (bitonic over xor-shuffles), rows of
+// Rows of <= 64 entries sort in registers (bitonic over VALU exchanges), rows of
 // <= kSegBig entries in LDS (radix, one block per row), longer rows through
 // the device radix sort.
 

@@ -6,8 +6,8 @@
 // in one "forest": every vertex of the coarsest graph sits in the contiguous
 // range of the tree node that owns it, rows hold forest positions, and edges
 // never cross nodes.  One launch runs every trial of every node of the depth
-// (one wave per GGGP + FM trial), so k-1 bisections take ceil(log2 k) launches
-// and no host round-trips.  Tree node ids are heap ids (root 1, children 2i
+// (a block per GGGP + FM trial; a wave for small node graphs and for the FM on
+// queues), so k-1 bisections take ceil(log2 k) launches and no host round-trips.  Tree node ids are heap ids (root 1, children 2i
 // and 2i+1), which also key the trial random streams.
 #include "hgp_graph.hpp"
 #include "hgp_prims.hpp"
@@ -30,7 +30,7 @@ constexpr int kHeapBytesPerVertex = 34;
 constexpr int kHeapLdsBudget = 60 * 1024;
 // fm_kind -1 keeps the scan: on the dense coarsest graphs this pipeline
 // produces (R-MAT 2^22: 995 vertices, average degree ~300) the queues took
-// 188 ms against 7 ms, a move's row being ~300 serial queue updates
+// 187 ms against 2 ms, a move's row being ~300 serial queue updates
 constexpr int32_t kAutoHeapMinVertices = INT32_MAX;
 
 __host__ __device__ inline int64_t trial_bytes(int64_t n, bool heap, bool in_lds)
@@ -853,8 +853,10 @@ __device__ inline int64_t scan_trial(const TrialRows &G, char *base, int32_t n, 
             int64_t dd = ideal0 - pw0;
             dd = dd < 0 ? -dd : dd;
             const int64_t into = (from ? pw0 : pw1) + wv, outof = (from ? pw1 : pw0) - wv;
-            // selects instead of short-circuit branches: those were compiled into
-            // code that kept the old mincutorder where the second test alone held
+            // selects instead of short-circuit branches: as `if ((a && b) || (c && d))`
+            // around the three assignments this is compiled (ROCm 7.2, all operands
+            // in scalar registers) into a jump for c && d that lands behind the move
+            // of mincutorder and before those of mincut and mindiff
             const bool keep = ((newcut < mincut) & (into <= onemax) & (outof <= onemax)) |
                               ((newcut == mincut) & (dd < mindiff));
             if (!keep && nswaps - mincutorder > limit) break;
@@ -1272,8 +1274,7 @@ __device__ inline int64_t dense_trial(const DenseNode &D, char *lds, const Node 
             int64_t dd = ideal0 - pw0;
             dd = dd < 0 ? -dd : dd;
             const int64_t into = (from ? pw0 : pw1) + wv, outof = (from ? pw1 : pw0) - wv;
-            // selects instead of short-circuit branches: those were compiled into
-            // code that kept the old mincutorder where the second test alone held
+            // (selects for the reason given in scan_trial)
             const bool keep = ((newcut < mincut) & (into <= onemax) & (outof <= onemax)) |
                               ((newcut == mincut) & (dd < mindiff));
             if (!keep && nswaps - mincutorder > limit) break;

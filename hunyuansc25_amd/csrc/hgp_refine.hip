@@ -2079,7 +2079,10 @@ constexpr unsigned kHotBlocks = 256;   // one per CU
 // Whether the level gets the hot order: the positions cost one pass over the
 // entries, so it has to be large, and the hot vertices have to receive at
 // least a third of the entries (counted from the degree classes, heaviest
-// first, each as if its rows had the class's mean length).
+// first, each as if its rows had the class's mean length).  These shares were
+// set on R-MAT alone, where they tell the levels that gain from those that do
+// not; no other graph kind here has an eighth of its entries in long rows.  A
+// level in an arena without the room runs the kernels that gather every id.
 bool want_hot_order(const Ctx &c, const DevGraph &g, int32_t k, int32_t cap)
 {
     if (g.n <= cap || g.m < 2 * kHotEntries || 8 * g.bins.ent[kClsLong] < g.m) return false;
@@ -2284,9 +2287,12 @@ void project(Ctx &c, int32_t n, const int32_t *cmap, const int32_t *where_c, int
 // in one block of kTinyBS threads: the same phases as the kernels above
 // (selection, afterburner, LP filter, RW/RS eviction with its sort and cookie
 // cutter, move accounting, commit, bookkeeping) separated by block barriers
-// instead of launches, and no host round trip per iteration.  The block's 16 waves walk rows one after another, so the path
-// pays off only while a level's rows are few: measured on grids, 3-D RGGs
-// and banded graphs, 512 vertices beat both 256 and 1024.
+// instead of launches, and no host round trip per iteration.  One CU works on
+// the level, so the path pays off only while its rows are few and short.  Levels
+// of up to 256 / 512 / 1024 / 2048 vertices: grid 64 x 64, k = 8, 5.81 / 5.63 /
+// 5.54 / 5.44 ms a call, grid 256 x 256 12.06 / 11.95 / 11.88 / 11.89, but banded
+// with 200003 vertices, k = 37, 11.55 / 11.62 / 12.00 / 16.85 and R-MAT with 2^19,
+// k = 256, 34.14 / 34.17 / 35.26 / 36.06.
 constexpr int kTinyBS = 1024;
 constexpr int kTinyWaves = kTinyBS / kWave;
 constexpr int32_t kTinyK = 256;

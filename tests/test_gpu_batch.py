@@ -57,8 +57,8 @@ def test_batch_reports_bad_graph(hgp):
 
 def test_batch_fused_small_levels_match_alone(hgp):
     """The batch's fused launch over the small levels (one block per graph,
-    levels of up to 16384 vertices: the block's scans and compactions then
-    run in several chunks) gives every graph its partition alone."""
+    levels of up to 16384 vertices, the one-block loop at 8 and 16 rows a
+    wave) gives every graph its partition alone."""
     x, a, vw, aw = random_graph(3000, 0.004, seed=8, wmax=7, vmax=5)
     gs = [hgp.gen_rgg3d(12000, hgp.rgg_radius(12000, 12), seed=2), hgp.gen_grid2d(110, 110),
           hgp.gen_banded(9000, 32, 0.1, seed=3), (x, a, vw, aw), hgp.gen_rmat(13, 1 << 16, seed=4)]
