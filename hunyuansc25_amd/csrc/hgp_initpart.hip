@@ -20,11 +20,16 @@ namespace hgp {
 
 namespace {
 
-// LDS of a trial.  Scan FM: (ed, wd) pairs, row offsets (i32), queue (u16)
-// and a state byte, 15 bytes a vertex; node graphs of up to kScanLdsN
-// vertices run in LDS (two trials per CU at that size), larger ones in global
-// scratch with a 32-bit queue.  Heap FM: where, moved (u8), ed, id, queue,
-// position index (i32) and two heaps of (key, vertex), n + 1 slots each.
+// Arrays of a trial.  Scan FM in LDS: (ed, wd) pairs, row offsets (i32), queue
+// (u16) and a state byte, 15 bytes a vertex; node graphs of up to kScanLdsN
+// vertices run there (two trials per CU at that size).  Larger ones run in
+// global scratch with a 32-bit queue and the node's own row offsets, 13 a
+// vertex, 14 apart: a thousand trials walk their arrays side by side, and 13
+// apart they lose 3 % at 20000 vertices, 23 % at 30000 (1060 against 864 ms a
+// call; 17, with row offsets of their own, 860, but 3 B more a vertex and trial
+// is 92 MB more of the 440 such a call allocates).  Heap FM: where, moved (u8),
+// ed, id, queue, position index (i32) and two heaps of (key, vertex), n + 1
+// slots each.
 constexpr int32_t kScanLdsN = 4864;
 constexpr int kHeapBytesPerVertex = 34;
 constexpr int kHeapLdsBudget = 60 * 1024;
@@ -37,7 +42,7 @@ __host__ __device__ inline int64_t trial_bytes(int64_t n, bool heap, bool in_lds
 {
     if (heap) return ((2 * n + 3) & ~3ll) + 12 * n + 4 * n + 16 * (n + 1);
     const int64_t n4 = (n + 3) & ~3ll;   // the arg-max reads four vertices at a time
-    return (8 + 4 + (in_lds ? 2 : 4) + 1) * n4 + 16;
+    return (in_lds ? 15 : 14) * n4 + 16;
 }
 
 struct Node {
@@ -581,20 +586,28 @@ struct TrialRows {
 };
 
 // The trial's arrays: (ed, wd) per vertex, row offsets from the node's first
-// entry, queue / swap list, state bytes.
+// entry (in LDS only), queue / swap list, state bytes.
 template <class Q>
 struct ScanMem {
+    static constexpr bool kOffsets = sizeof(Q) == 2;   // (a 16-bit queue: in LDS)
     int2 *ew;
     int32_t *off;
     Q *queue;
     uint8_t *st;
-    __device__ ScanMem(char *base, int32_t n)
+    const eid_t *fx;   // the node's rows in the forest
+    __device__ ScanMem(char *base, int32_t n, const eid_t *node_rows) : fx(node_rows)
     {
         const int64_t n4 = (n + 3) & ~3;
         ew = (int2 *)base;
         off = (int32_t *)(base + 8 * n4);
-        queue = (Q *)(off + n4 + 4);
+        queue = (Q *)(kOffsets ? off + n4 + 4 : off);
         st = (uint8_t *)(queue + n4);
+    }
+    // first entry of row v, from the node's first one
+    __device__ int32_t row(int32_t v) const
+    {
+        if constexpr (kOffsets) return off[v];
+        else return (int32_t)(fx[v] - fx[0]);
     }
     // marks v queued; whether it was not before (one of several lanes that
     // mark the same vertex sees it fresh); old: the state byte before
@@ -670,8 +683,8 @@ __device__ inline int64_t trial_grow(const TrialRows &G, const ScanMem<Q> &M, in
             }
         } else {
             v = wave_read((int32_t)M.queue[first], 0);
-            rb = wave_read(M.off[v], 0);
-            re = wave_read(M.off[v + 1], 0);
+            rb = wave_read(M.row(v), 0);
+            re = wave_read(M.row(v + 1), 0);
             wv = G.vw[v];
             G.load(rb + lane, re, kWave, x, w);
         }
@@ -679,8 +692,8 @@ __device__ inline int64_t trial_grow(const TrialRows &G, const ScanMem<Q> &M, in
         if (first < last) {
             ahead = first;
             av = wave_read((int32_t)M.queue[first], 0);
-            ab = wave_read(M.off[av], 0);
-            ae = wave_read(M.off[av + 1], 0);
+            ab = wave_read(M.row(av), 0);
+            ae = wave_read(M.row(av + 1), 0);
             aw = G.vw[av];
             G.load(ab + lane, ae, kWave, ax, at);
         }
@@ -761,9 +774,9 @@ __device__ inline int64_t scan_trial(const TrialRows &G, char *base, int32_t n, 
     constexpr int NW = NT / kWave;
     constexpr int P = NT == kWave ? 4 : 2;   // row entries per thread in flight
     const int tid = threadIdx.x, lane = lane_id();
-    const ScanMem<Q> M(base, n);
-    const eid_t fb = fx[G.s0];
-    for (int32_t i = tid; i <= n; i += NT) M.off[i] = (int32_t)(fx[G.s0 + i] - fb);
+    const ScanMem<Q> M(base, n, fx + G.s0);
+    if constexpr (ScanMem<Q>::kOffsets)
+        for (int32_t i = tid; i <= n; i += NT) M.off[i] = (int32_t)(M.fx[i] - M.fx[0]);
     for (int32_t i = tid; i < ((n + 3) & ~3); i += NT) {
         M.st[i] = kStSide;
         M.ew[i] = make_int2(0, i < n ? fwd[G.s0 + i] : 0);   // the padding stays out of the arg-max: ed 0, not alone
@@ -784,7 +797,7 @@ __device__ inline int64_t scan_trial(const TrialRows &G, char *base, int32_t n, 
     int64_t cutacc = 0;
     for (int32_t v = tid; v < n; v += NT) {
         const int2 e = M.ew[v];
-        M.st[v] = (uint8_t)((M.st[v] & kStSide) | (M.off[v] == M.off[v + 1] ? kStAlone : 0));
+        M.st[v] = (uint8_t)((M.st[v] & kStSide) | (M.row(v) == M.row(v + 1) ? kStAlone : 0));
         cutacc += e.x;
     }
     cutacc = wave_sum(cutacc);
@@ -845,7 +858,7 @@ __device__ inline int64_t scan_trial(const TrialRows &G, char *base, int32_t n, 
             bv = wave_read(bv, 0);
             const int32_t bg = wave_read(g, 0);
             if (bg == INT32_MIN) break;
-            const int32_t rb = wave_read(M.off[bv], 0), re = wave_read(M.off[bv + 1], 0);
+            const int32_t rb = wave_read(M.row(bv), 0), re = wave_read(M.row(bv + 1), 0);
             const int32_t wv = wave_read(G.vw[bv], 0);
             int32_t x[P], w[P];   // the row, on its way while the move is judged
             G.load(rb + tid, re, NT, x, w);
@@ -878,7 +891,7 @@ __device__ inline int64_t scan_trial(const TrialRows &G, char *base, int32_t n, 
         for (nswaps--; nswaps > mincutorder; nswaps--) {
             const int32_t v = wave_read((int32_t)swaps[nswaps], 0);
             const int from = wave_read((int32_t)M.st[v], 0) & kStSide;
-            const int32_t rb = wave_read(M.off[v], 0), re = wave_read(M.off[v + 1], 0);
+            const int32_t rb = wave_read(M.row(v), 0), re = wave_read(M.row(v + 1), 0);
             const int32_t wv = wave_read(G.vw[v], 0);
             int32_t x[P], w[P];
             G.load(rb + tid, re, NT, x, w);
@@ -918,11 +931,11 @@ __global__ void __launch_bounds__(NT) k_ip_trials(const int32_t *__restrict__ ac
     int64_t cut;
     if (n <= lds_cap) {   // a 16-bit queue: lds_cap < 2^16
         cut = scan_trial<NT, uint16_t>(G, lds, n, nd, nid, t, fx, fwd, seed, fm_passes, S);
-        st = ScanMem<uint16_t>(lds, n).st;
+        st = ScanMem<uint16_t>(lds, n, fx + nd.start).st;
     } else {
         char *base = gscratch + nd.soff + (int64_t)t * ((trial_bytes(n, false, false) + 255) & ~255ll);
         cut = scan_trial<NT, int32_t>(G, base, n, nd, nid, t, fx, fwd, seed, fm_passes, S);
-        st = ScanMem<int32_t>(base, n).st;
+        st = ScanMem<int32_t>(base, n, fx + nd.start).st;
     }
     uint8_t *out = trial_where + nd.woff + (int64_t)t * n;
     for (int32_t i = threadIdx.x; i < n; i += NT) out[i] = st[i] & kStSide;

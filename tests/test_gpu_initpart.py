@@ -76,3 +76,17 @@ def test_matrices_yield_to_the_memory_there_is(hgp, orc):
         np.testing.assert_array_equal(part, ref)
         assert ran.get("k_ip_dense", (0,))[0] == int(dense)
         assert ran["k_ip_trials"][0] == 1 and st["arena_bytes"] < 90_000_000
+
+
+def test_list_trials_within_a_budget(hgp):
+    """A thousand trials on the lists of a coarsest graph of 15600 vertices take
+    226 MB of scratch, 14 B a vertex and trial: served within 262 MB."""
+    n = 31200
+    pairs, links = [(v, v + 1) for v in range(0, n, 2)], [(v + 1, v + 2) for v in range(0, 14000, 4)]
+    x, a, aw = csr_from_edges(n, pairs + links, [5] * len(pairs) + [1] * len(links))
+    vw = np.ones(n, np.int32)
+    ref, _ = hgp.partition(x, a, 2, vw, aw, seed=3)
+    with hgp.Server(slots=1, budget_bytes=262_000_000) as s:
+        part, st, _ = s.wait(s.submit(x, a, 2, vw, aw, seed=3))
+    assert st["coarsest_n"] == 15600
+    np.testing.assert_array_equal(part, ref)
